@@ -27,6 +27,8 @@
 // cross-wave reduction.  K is walked in 256-wide chunks spread over the 8
 // waves (a wave prefetches its next chunk's weight rows while it multiplies
 // the current one).
+#include <algorithm>
+
 #include "nvdsa_common.h"
 #include "nvdsa_kernels.h"
 
@@ -198,6 +200,483 @@ __global__ __launch_bounds__(kProjThreads) void indexer_project_kernel(IndexerAr
       static_cast<uint32_t>(o0) | (static_cast<uint32_t>(o1) << 16);
 }
 
+// ---------------------------------------------------------------------------
+// The q projection of many tokens (a prompt, a large batch): a tiled GEMM with
+// the rotation in its epilogue.  The 64-token groups above re-read wq_b for
+// every group and multiply out of registers that each MFMA waits to be
+// loaded; from a few hundred tokens on the product itself is the work.
+//
+// A workgroup owns TOK tokens x OUT weight rows.  Both tiles go through LDS in
+// K steps of 64 (128-byte rows of eight 16-byte chunks, chunk c of row r kept
+// at c ^ (r & 7): the operand reads of eight consecutive rows touch all
+// banks), two buffers: the next step's loads are issued before this step's
+// MFMAs and stored after them, one barrier per step.  Wave tiles are
+// TOK/WT x OUT/WO of 32x32x16 MFMAs, the weight rows as the A operand, so a
+// lane holds runs of four consecutive outputs of one token (the rotation's
+// pairs).  The rotated 16-bit tile is turned through LDS and stored in whole
+// 16-byte chunks of a token's row.
+constexpr int kGemmK = 64;
+constexpr int kGemmChunks = kGemmK / 8;
+
+template <int TOK, int OUT, int WT, int WO>
+struct GemmShape {
+  static constexpr int kThreads = 64 * WT * WO;
+  static constexpr int kTokW = TOK / WT, kOutW = OUT / WO;     // wave tile
+  static constexpr int kTT = kTokW / 32, kOT = kOutW / 32;     // its 32x32 tiles
+  static constexpr int kXLoads = TOK * kGemmChunks / kThreads;  // 16-byte chunks per thread and K step
+  static constexpr int kWLoads = OUT * kGemmChunks / kThreads;
+  static constexpr int kBuf = (TOK + OUT) * kGemmK;             // elements of one buffer
+  static constexpr int kOutStride = OUT + 8;                    // epilogue row, elements
+  static constexpr int kLds = 2 * kBuf > TOK * kOutStride ? 2 * kBuf : TOK * kOutStride;
+  static_assert(TOK * kGemmChunks % kThreads == 0 && OUT * kGemmChunks % kThreads == 0 && kTokW % 32 == 0 &&
+                kOutW % 32 == 0, "GEMM tiling");
+};
+
+template <typename T, int TOK, int OUT, int WT, int WO>
+__global__ __launch_bounds__(64 * WT * WO) void indexer_project_gemm_kernel(IndexerArgs a, int tok_tiles,
+                                                                            int out_tiles) {
+  using S = GemmShape<TOK, OUT, WT, WO>;
+  __shared__ __align__(16) uint16_t lds[S::kLds];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int l32 = lane & 31;
+  const int grp = lane >> 5;
+  const int wt = wave / WO, wo = wave % WO;
+
+  // Workgroup -> tile, XCD by XCD (the dispatcher deals ids to the 8 XCDs in
+  // turn): each XCD takes a contiguous run of tiles, ordered in bands of
+  // kBand token tiles, so the tiles an XCD runs together share both operands
+  // in its L2.
+  constexpr int kBand = 4;
+  const int ntiles = tok_tiles * out_tiles;
+  int p = blockIdx.x;
+  {
+    const int base = ntiles >> 3, extra = ntiles & 7, x = p & 7;
+    p = x * base + min(x, extra) + (p >> 3);
+  }
+  const int band = p / (kBand * out_tiles);
+  const int band_rows = min(kBand, tok_tiles - band * kBand);
+  const int q = p - band * kBand * out_tiles;
+  const int tok0 = (band * kBand + q % band_rows) * TOK;
+  const int out0 = q / band_rows * OUT;
+
+  const int K = static_cast<int>(a.rank);
+  const int ntok = static_cast<int>(a.tokens);
+  // Thread's chunk of each load round: row tid / 8 (+ rounds), chunk tid % 8.
+  const int lrow = tid >> 3, lch = tid & 7;
+  constexpr int kRound = S::kThreads / kGemmChunks;
+  const u32x4_t* xsrc[S::kXLoads];
+  const u32x4_t* wsrc[S::kWLoads];
+#pragma unroll
+  for (int j = 0; j < S::kXLoads; ++j) {  // tokens past the last reread it (their results are not stored)
+    const int t = min(tok0 + lrow + j * kRound, ntok - 1);
+    xsrc[j] = reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.q_c) + static_cast<int64_t>(t) * K) + lch;
+  }
+#pragma unroll
+  for (int j = 0; j < S::kWLoads; ++j)
+    wsrc[j] = reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.wq_b) +
+                                               static_cast<int64_t>(out0 + lrow + j * kRound) * K) + lch;
+  const int lpos = lrow * kGemmK + ((lch ^ (lrow & 7)) * 8);  // (kRound is a multiple of 8: the same swizzle every round)
+  static_assert(kRound % 8 == 0, "swizzle");
+
+  u32x4_t xv[S::kXLoads], wv[S::kWLoads];
+  auto load = [&](int step) {
+#pragma unroll
+    for (int j = 0; j < S::kXLoads; ++j) xv[j] = xsrc[j][step * kGemmChunks];
+#pragma unroll
+    for (int j = 0; j < S::kWLoads; ++j) wv[j] = wsrc[j][step * kGemmChunks];
+  };
+  auto store = [&](uint16_t* buf) {
+#pragma unroll
+    for (int j = 0; j < S::kXLoads; ++j) *reinterpret_cast<u32x4_t*>(&buf[lpos + j * kRound * kGemmK]) = xv[j];
+#pragma unroll
+    for (int j = 0; j < S::kWLoads; ++j)
+      *reinterpret_cast<u32x4_t*>(&buf[TOK * kGemmK + lpos + j * kRound * kGemmK]) = wv[j];
+  };
+
+  f32x16_t acc[S::kOT][S::kTT];
+#pragma unroll
+  for (int i = 0; i < S::kOT; ++i)
+#pragma unroll
+    for (int j = 0; j < S::kTT; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  const int steps = K / kGemmK;
+  load(0);
+  store(lds);
+  load(min(1, steps - 1));
+  lds_barrier();
+  const int xrow = (wt * S::kTokW + l32) * kGemmK;
+  const int wrow = TOK * kGemmK + (wo * S::kOutW + l32) * kGemmK;
+  typename T::vec8 wf[2][S::kOT], xf[2][S::kTT];
+  auto read = [&](const uint16_t* buf, int kk, int set) {
+    const int ch = ((2 * kk + grp) ^ (l32 & 7)) * 8;
+#pragma unroll
+    for (int i = 0; i < S::kOT; ++i)
+      wf[set][i] = *reinterpret_cast<const typename T::vec8*>(&buf[wrow + i * 32 * kGemmK + ch]);
+#pragma unroll
+    for (int j = 0; j < S::kTT; ++j)
+      xf[set][j] = *reinterpret_cast<const typename T::vec8*>(&buf[xrow + j * 32 * kGemmK + ch]);
+  };
+  read(lds, 0, 0);
+  for (int s = 0; s < steps; ++s) {
+    const uint16_t* cur = lds + (s & 1) * S::kBuf;
+    uint16_t* next = lds + ((s + 1) & 1) * S::kBuf;
+#pragma unroll
+    for (int kk = 0; kk < kGemmK / 16; ++kk) {
+      if (kk + 1 < kGemmK / 16) read(cur, kk + 1, (kk + 1) & 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < S::kOT; ++i)
+#pragma unroll
+        for (int j = 0; j < S::kTT; ++j) acc[i][j] = T::mfma32(wf[kk & 1][i], xf[kk & 1][j], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kk == 1) {
+        store(next);
+        load(min(s + 2, steps - 1));  // (the last steps reload the last tile: no branch in the loop)
+      }
+    }
+    lds_barrier();  // the next buffer is stored; this one is free (loads in flight stay in flight)
+    read(next, 0, 0);
+  }
+
+  // The products rounded to 16 bits, through LDS: element e of a 32x32 tile is
+  // output row 8 (e >> 2) + 4 grp + (e & 3) of token l32.
+#pragma unroll
+  for (int j = 0; j < S::kTT; ++j)
+#pragma unroll
+    for (int i = 0; i < S::kOT; ++i)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        *reinterpret_cast<uint2*>(&lds[(wt * S::kTokW + j * 32 + l32) * S::kOutStride + wo * S::kOutW + i * 32 +
+                                       8 * g4 + 4 * grp]) =
+            make_uint2(T::pack2(acc[i][j][4 * g4], acc[i][j][4 * g4 + 1]),
+                       T::pack2(acc[i][j][4 * g4 + 2], acc[i][j][4 * g4 + 3]));
+  __syncthreads();
+  // Then rotated and stored by 16-byte chunks (eight outputs of one token,
+  // within one head).  A rolled loop: unrolled over the accumulators the
+  // rotation is tens of KB of straight-line code, and fetching it cost more
+  // than running it (a 256 x 256 tile's epilogue 30 us, 16 us of it after the
+  // cheaper conversion; now a few).
+  constexpr int kRowChunks = OUT / 8;
+  const int head_dim = static_cast<int>(a.head_dim), rope = static_cast<int>(a.rope_dim);
+  const int64_t row_elems = a.heads * a.head_dim;
+  for (int c = tid; c < TOK * kRowChunks; c += S::kThreads) {
+    const int r = c / kRowChunks, ch = c % kRowChunks;
+    const int64_t t = tok0 + r;
+    if (t >= ntok) break;  // (r does not decrease along the loop)
+    u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[r * S::kOutStride + ch * 8]);
+    const int d = (out0 + ch * 8) % head_dim;
+    if (d < rope) {
+      const uint32_t* cp = reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.cos) + t * a.cos_stride + d);
+      const uint32_t* sp = reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.sin) + t * a.cos_stride + d);
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        if (d + 2 * h < rope) {
+          const uint32_t x2 = v[h], c2 = cp[h], s2 = sp[h];
+          float y0, y1;
+          rope_pair(T::to_float(static_cast<uint16_t>(x2)), T::to_float(static_cast<uint16_t>(x2 >> 16)),
+                    T::to_float(static_cast<uint16_t>(c2)), T::to_float(static_cast<uint16_t>(c2 >> 16)),
+                    T::to_float(static_cast<uint16_t>(s2)), T::to_float(static_cast<uint16_t>(s2 >> 16)), y0, y1);
+          v[h] = T::pack2(y0, y1);
+        }
+      }
+    }
+    *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(a.q_out) + t * row_elems + out0 + ch * 8) = v;
+  }
+}
+
+template <typename T, int TOK, int OUT, int WT, int WO>
+void launch_gemm_shape(const IndexerArgs& a, hipStream_t stream) {
+  const int tt = static_cast<int>(ceil_div(a.tokens, TOK)), ot = static_cast<int>(a.heads * a.head_dim / OUT);
+  launch_kernel(kKernIdxProject, indexer_project_gemm_kernel<T, TOK, OUT, WT, WO>, dim3(static_cast<uint32_t>(tt * ot)),
+                dim3(GemmShape<TOK, OUT, WT, WO>::kThreads), stream, a, tt, ot);
+}
+
+// ---------------------------------------------------------------------------
+// The products of hidden_states that go with many tokens: the index key
+// k = hidden . wk^T (128 wide, 16-bit) and the head weights hidden . w_proj^T
+// (w_proj in fp32, or 16-bit).  Both read hidden_states, the only large
+// operand, so one kernel reads it once: a workgroup owns 128 tokens x every
+// column x one slice of hidden_size (split so that about one workgroup per CU
+// runs), through LDS as above.  The key columns run on 32x32x16 MFMAs, the
+// head weights on 16x16x4 fp32 MFMAs: the 16-bit activations widened exactly,
+// so a product and its sum round as in an fp32 GEMM (the matrix cores' fp32
+// rate, 1/16 of the 16-bit one, is what bounds the kernel: 1.6 GFLOP at 4096
+// tokens, 10 us of the chip; measured 33 us, 40 us with one K step in flight:
+// the loads' latency).  It replaces two library GEMMs (27 + 24 us), the fp32
+// copy of hidden_states (22 us), a layer norm, the rotation and six small
+// copies and casts.  Slices leave fp32 partial sums; the finish
+// kernel adds them in slice order, rounds, and does the layer norm, the
+// rotation and the scale: one wave per token.
+constexpr int kKwTok = 128;
+constexpr int kKwThreads = 512;
+constexpr int kKwDim = 128;                   // index key width
+constexpr int kKwMaxSlices = 48;
+constexpr int kKwWRow = kGemmK + 4;            // fp32 LDS row of the head projection (floats)
+
+// HT: 16-head tiles.  K: the key columns too.
+template <typename T, int HT, bool K>
+__global__ __launch_bounds__(kKwThreads) void indexer_kw_kernel(IndexerKwArgs a, int slices) {
+  constexpr int kHeads = 16 * HT;
+  constexpr int kCols = (K ? kKwDim : 0) + kHeads;
+  constexpr int kX = kKwTok * kGemmK, kWk = K ? kKwDim * kGemmK : 0;  // elements of one buffer
+  __shared__ __align__(16) uint16_t xs[2][kX];
+  __shared__ __align__(16) uint16_t wks[2][K ? kWk : 8];
+  __shared__ __align__(16) float wps[2][kHeads * kKwWRow];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int slice = blockIdx.x % slices;
+  const int tok0 = static_cast<int>(blockIdx.x / slices) * kKwTok;
+  const int ntok = static_cast<int>(a.tokens);
+  const int hid = static_cast<int>(a.hid);
+  const int steps = hid / kGemmK;
+  const int per = static_cast<int>(ceil_div(steps, slices));
+  const int s_begin = slice * per, s_end = min(steps, s_begin + per);
+
+  const int lrow = tid >> 3, lch = tid & 7;     // 64 rows of eight chunks per round
+  constexpr int kXl = kKwTok / 64, kWl = K ? kKwDim / 64 : 0;
+  constexpr int kPl = (kHeads * kGemmK / 8 + kKwThreads - 1) / kKwThreads;  // runs of eight head-projection values
+  const u32x4_t* xsrc[kXl];
+  const u32x4_t* wsrc[kWl > 0 ? kWl : 1];
+#pragma unroll
+  for (int j = 0; j < kXl; ++j)
+    xsrc[j] = reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.hidden) +
+                                               static_cast<int64_t>(min(tok0 + lrow + 64 * j, ntok - 1)) * hid) + lch;
+#pragma unroll
+  for (int j = 0; j < kWl; ++j)
+    wsrc[j] = reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.wk) +
+                                               static_cast<int64_t>(lrow + 64 * j) * hid) + lch;
+  const int lpos = lrow * kGemmK + ((lch ^ (lrow & 7)) * 8);
+  // Two sets of staged loads: two K steps are in flight while one is multiplied.
+  u32x4_t xv[2][kXl], wv[2][kWl > 0 ? kWl : 1], pv[2][kPl][2];
+  auto load = [&](int set, int s) {
+#pragma unroll
+    for (int j = 0; j < kXl; ++j) xv[set][j] = xsrc[j][s * kGemmChunks];
+#pragma unroll
+    for (int j = 0; j < kWl; ++j) wv[set][j] = wsrc[j][s * kGemmChunks];
+#pragma unroll
+    for (int j = 0; j < kPl; ++j) {
+      const int r = min(lrow + 64 * j, kHeads - 1);
+      const int64_t at = static_cast<int64_t>(r) * hid + s * kGemmK + lch * 8;
+      if (a.w_fp32) {  // uniform
+        const u32x4_t* p = reinterpret_cast<const u32x4_t*>(static_cast<const float*>(a.w_proj) + at);
+        pv[set][j][0] = p[0];
+        pv[set][j][1] = p[1];
+      } else {
+        pv[set][j][0] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.w_proj) + at);
+      }
+    }
+  };
+  auto store = [&](int set, int buf) {
+#pragma unroll
+    for (int j = 0; j < kXl; ++j) *reinterpret_cast<u32x4_t*>(&xs[buf][lpos + 64 * j * kGemmK]) = xv[set][j];
+#pragma unroll
+    for (int j = 0; j < kWl; ++j) *reinterpret_cast<u32x4_t*>(&wks[buf][lpos + 64 * j * kGemmK]) = wv[set][j];
+#pragma unroll
+    for (int j = 0; j < kPl; ++j) {
+      const int r = lrow + 64 * j;
+      if (r >= kHeads) continue;
+      u32x4_t lo = pv[set][j][0], hi = pv[set][j][1];
+      if (!a.w_fp32) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t w = pv[set][j][0][e];
+          const uint32_t f0 = __float_as_uint(T::to_float(static_cast<uint16_t>(w)));
+          const uint32_t f1 = __float_as_uint(T::to_float(static_cast<uint16_t>(w >> 16)));
+          if (e < 2) {
+            lo[2 * e] = f0;
+            lo[2 * e + 1] = f1;
+          } else {
+            hi[2 * e - 4] = f0;
+            hi[2 * e - 3] = f1;
+          }
+        }
+      }
+      float* d = &wps[buf][r * kKwWRow + lch * 8];
+      *reinterpret_cast<u32x4_t*>(d) = lo;
+      *reinterpret_cast<u32x4_t*>(d + 4) = hi;
+    }
+  };
+
+  // Key columns: waves 4 (32 tokens) x 2 (64 columns).  Head weights: wave w
+  // takes tokens 16 w .. +15.
+  const int l32 = lane & 31, grp = lane >> 5, l16 = lane & 15, g = lane >> 4;
+  const int wt = wave >> 1, wo = wave & 1;
+  f32x16_t kacc[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) kacc[i][e] = 0.f;
+  f32x4_t hacc[HT];
+#pragma unroll
+  for (int i = 0; i < HT; ++i) hacc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (s_begin < s_end) {
+    const int last = s_end - 1;
+    load(0, s_begin);
+    store(0, 0);
+    load(1, min(s_begin + 1, last));
+    load(0, min(s_begin + 2, last));
+    lds_barrier();
+    auto step = [&](int s, auto parity) {
+      constexpr int cur = decltype(parity)::value;  // this step's buffer; the next one's tile is in set cur ^ 1
+      if constexpr (K) {
+#pragma unroll
+        for (int kk = 0; kk < kGemmK / 16; ++kk) {
+          const int ch = ((2 * kk + grp) ^ (l32 & 7)) * 8;
+          const auto xf = *reinterpret_cast<const typename T::vec8*>(&xs[cur][(wt * 32 + l32) * kGemmK + ch]);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const auto wf =
+                *reinterpret_cast<const typename T::vec8*>(&wks[cur][(wo * 64 + i * 32 + l32) * kGemmK + ch]);
+            kacc[i] = T::mfma32(wf, xf, kacc[i]);
+          }
+        }
+      }
+      // 32 K per block: lane group g holds K 8 g .. 8 g + 7 of it, and step m
+      // multiplies the four K values 8 g + m.
+#pragma unroll
+      for (int kb = 0; kb < kGemmK / 32; ++kb) {
+        const u32x4_t x8 = *reinterpret_cast<const u32x4_t*>(
+            &xs[cur][(wave * 16 + l16) * kGemmK + (((4 * kb + g) ^ (l16 & 7)) * 8)]);
+        float xf[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          xf[2 * e] = T::to_float(static_cast<uint16_t>(x8[e]));
+          xf[2 * e + 1] = T::to_float(static_cast<uint16_t>(x8[e] >> 16));
+        }
+#pragma unroll
+        for (int i = 0; i < HT; ++i) {
+          const float* wp = &wps[cur][(16 * i + l16) * kKwWRow + 32 * kb + 8 * g];
+          const f32x4_t w0 = *reinterpret_cast<const f32x4_t*>(wp);
+          const f32x4_t w1 = *reinterpret_cast<const f32x4_t*>(wp + 4);
+#pragma unroll
+          for (int m = 0; m < 8; ++m)
+            hacc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(m < 4 ? w0[m & 3] : w1[m & 3], xf[m], hacc[i], 0, 0, 0);
+        }
+      }
+      store(cur ^ 1, cur ^ 1);
+      load(cur ^ 1, min(s + 3, last));
+      lds_barrier();
+    };
+    for (int s = s_begin; s < s_end; s += 2) {
+      step(s, std::integral_constant<int, 0>{});
+      if (s + 1 < s_end) step(s + 1, std::integral_constant<int, 1>{});
+    }
+  }
+  // Partial sums [slice][token][column]: the key columns, then the heads.
+  float* out = a.partial + static_cast<int64_t>(slice) * ntok * kCols;
+  if constexpr (K) {
+    const int t = tok0 + wt * 32 + l32;
+    if (t < ntok) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4)
+          *reinterpret_cast<float4*>(out + static_cast<int64_t>(t) * kCols + wo * 64 + i * 32 + 8 * g4 + 4 * grp) =
+              make_float4(kacc[i][4 * g4], kacc[i][4 * g4 + 1], kacc[i][4 * g4 + 2], kacc[i][4 * g4 + 3]);
+    }
+  }
+  const int t = tok0 + wave * 16 + l16;  // head 16 i + 4 g + e of token l16
+  if (t < ntok) {
+#pragma unroll
+    for (int i = 0; i < HT; ++i)
+      *reinterpret_cast<float4*>(out + static_cast<int64_t>(t) * kCols + (K ? kKwDim : 0) + 16 * i + 4 * g) =
+          make_float4(hacc[i][0], hacc[i][1], hacc[i][2], hacc[i][3]);
+  }
+}
+
+// One wave per token: lane l holds key dims 2 l, 2 l + 1 (the rotation's
+// pairs) and, for l < heads, head l's weight.
+template <typename T, bool K>
+__global__ __launch_bounds__(256) void indexer_kw_finish_kernel(IndexerKwArgs a, int slices) {
+  const int lane = threadIdx.x & 63;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (t >= a.tokens) return;
+  const int heads = static_cast<int>(a.heads);
+  const int cols = (K ? kKwDim : 0) + heads;
+  const float* p = a.partial + t * cols;
+  const int64_t stride = a.tokens * cols;
+  float k0 = 0.f, k1 = 0.f, w = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < slices; ++s) {
+    if constexpr (K) {
+      const float2 v = *reinterpret_cast<const float2*>(p + s * stride + 2 * lane);
+      k0 += v.x;
+      k1 += v.y;
+    }
+    if (lane < heads) w += p[s * stride + (K ? kKwDim : 0) + lane];
+  }
+  if (lane < heads) {
+    uint16_t* out = static_cast<uint16_t*>(a.w_out) + t * heads + lane;
+    if (a.w_fp32) {
+      *out = T::from_float(w * a.score_scale);
+    } else {  // rounded after the projection and again after the scale
+      uint16_t o = T::from_float(w);
+      if (a.score_scale != 1.f) o = T::from_float(T::to_float(o) * a.score_scale);
+      *out = o;
+    }
+  }
+  if constexpr (K) {
+    // The projection is rounded to 16 bits, then the layer norm in fp32
+    // (eps 1e-6), rounded, then the rotation.
+    const float x0 = T::to_float(T::from_float(k0)), x1 = T::to_float(T::from_float(k1));
+    const float mean = wave_all_op(x0 + x1, AddOp{}) * (1.f / kKwDim);
+    const float d0 = x0 - mean, d1 = x1 - mean;
+    const float var = wave_all_op(d0 * d0 + d1 * d1, AddOp{}) * (1.f / kKwDim);
+    const float rstd = 1.f / sqrtf(var + 1e-6f);
+    const uint32_t gw = static_cast<const uint32_t*>(a.norm_weight)[lane];
+    float y0 = d0 * rstd * T::to_float(static_cast<uint16_t>(gw));
+    float y1 = d1 * rstd * T::to_float(static_cast<uint16_t>(gw >> 16));
+    if (a.norm_bias != nullptr) {
+      const uint32_t gb = static_cast<const uint32_t*>(a.norm_bias)[lane];
+      y0 += T::to_float(static_cast<uint16_t>(gb));
+      y1 += T::to_float(static_cast<uint16_t>(gb >> 16));
+    }
+    uint32_t o = T::pack2(y0, y1);
+    if (2 * lane < a.rope_dim) {
+      const uint32_t c2 = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.cos) + t * a.cos_stride + 2 * lane);
+      const uint32_t s2 = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.sin) + t * a.cos_stride + 2 * lane);
+      float r0, r1;
+      rope_pair(T::to_float(static_cast<uint16_t>(o)), T::to_float(static_cast<uint16_t>(o >> 16)),
+                T::to_float(static_cast<uint16_t>(c2)), T::to_float(static_cast<uint16_t>(c2 >> 16)),
+                T::to_float(static_cast<uint16_t>(s2)), T::to_float(static_cast<uint16_t>(s2 >> 16)), r0, r1);
+      o = T::pack2(r0, r1);
+    }
+    static_cast<uint32_t*>(a.k_out)[t * (kKwDim / 2) + lane] = o;
+  }
+}
+
+// K slices of a launch: about one workgroup per CU.
+int kw_slices(int64_t tokens, int64_t hid) {
+  const int64_t s = std::min<int64_t>({256 / std::max<int64_t>(1, ceil_div(tokens, kKwTok)), kKwMaxSlices, hid / kGemmK});
+  return static_cast<int>(std::max<int64_t>(1, s));
+}
+
+template <typename T, int HT, bool K>
+hipError_t launch_kw_shape(const IndexerKwArgs& a, hipStream_t stream) {
+  const int slices = kw_slices(a.tokens, a.hid);
+  launch_kernel(kKernIdxKw, indexer_kw_kernel<T, HT, K>, dim3(static_cast<uint32_t>(ceil_div(a.tokens, kKwTok) * slices)),
+                dim3(kKwThreads), stream, a, slices);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  launch_kernel(kKernIdxKwFinish, indexer_kw_finish_kernel<T, K>, dim3(static_cast<uint32_t>(ceil_div(a.tokens, 4))),
+                dim3(256), stream, a, slices);
+  return hipGetLastError();
+}
+
+template <typename T, bool K>
+hipError_t launch_kw(const IndexerKwArgs& a, hipStream_t stream) {
+  switch (a.heads) {
+    case 16: return launch_kw_shape<T, 1, K>(a, stream);
+    case 32: return launch_kw_shape<T, 2, K>(a, stream);
+    default: return launch_kw_shape<T, 4, K>(a, stream);
+  }
+}
+
 // In-place RoPE of the first rope_dim dims of every [token, head] row: one
 // (even, odd) pair per thread (the reference op
 // dsa_indexer_query_rope_inplace, dsa_indexer_project_kernel.cpp:60-90).
@@ -223,6 +702,28 @@ __global__ __launch_bounds__(256) void indexer_rope_kernel(RopeArgs a) {
 template <typename T>
 hipError_t launch_project(const IndexerArgs& a, hipStream_t stream) {
   const int q_tiles = static_cast<int>(a.heads * a.head_dim / kRowTile);
+  if (a.w_proj == nullptr && a.tokens > kTokPerGroup) {
+    // More than one 64-token group: the tiled GEMM (n_head and head_dim are
+    // multiples of 16, so its output tiles divide the rows of wq_b).  Its
+    // tile by the time each would take, measured at 4096 outputs of K 2048: a
+    // launch's 64 x 64 tiles fill the chip's 256 CUs at 14 us and then cost
+    // 27.5 ns each, 128 x 128 ones 32 us and 93 ns, 256 x 256 ones 76 us per
+    // round of 256.  64-token groups / 64 / 128 / 256 tiles: 65 tokens 15.8 /
+    // 14.2 / 32 / 60 us, 512: 89 / 22 / 34 / 66, 1024: 174 / 35 / 32 / 65,
+    // 4096: 675 / 132 / 99 / 76 us.
+    const int64_t outs = a.heads * a.head_dim;
+    const int64_t n64 = ceil_div(a.tokens, 64) * (outs / 64), n128 = ceil_div(a.tokens, 128) * (outs / 128);
+    const int64_t n256 = ceil_div(a.tokens, 256) * (outs / 256);
+    const double us64 = std::max(14.0, 7.0 + 0.0275 * n64), us128 = std::max(32.0, 8.0 + 0.09 * n128);
+    const double us256 = 76.0 * ceil_div(n256, 256);
+    if (us64 <= us128 && us64 <= us256)
+      launch_gemm_shape<T, 64, 64, 2, 2>(a, stream);
+    else if (us128 <= us256)
+      launch_gemm_shape<T, 128, 128, 2, 2>(a, stream);
+    else
+      launch_gemm_shape<T, 256, 256, 4, 2>(a, stream);
+    return hipGetLastError();
+  }
   const dim3 grid(static_cast<uint32_t>(q_tiles), static_cast<uint32_t>(ceil_div(a.tokens, kTokPerGroup)));
   launch_kernel(kKernIdxProject, indexer_project_kernel<T>, grid, dim3(kProjThreads), stream, a, q_tiles);
   return hipGetLastError();
@@ -243,6 +744,20 @@ int64_t indexer_k_chunk() { return kKChunk; }
 hipError_t launch_indexer_project(const IndexerArgs& a, hipStream_t stream) {
   if (a.tokens == 0) return hipSuccess;
   return a.elem == Elem::kBf16 ? launch_project<Bf16>(a, stream) : launch_project<F16>(a, stream);
+}
+
+bool indexer_kw_supported(int64_t heads, int64_t hid) {
+  return (heads == 16 || heads == 32 || heads == 64) && hid > 0 && hid % kGemmK == 0;
+}
+
+size_t indexer_kw_workspace_bytes(int64_t tokens, int64_t heads, int64_t hid, bool with_k) {
+  return sizeof(float) * kw_slices(tokens, hid) * std::max<int64_t>(0, tokens) * ((with_k ? kKwDim : 0) + heads);
+}
+
+hipError_t launch_indexer_kw(const IndexerKwArgs& a, hipStream_t stream) {
+  if (a.tokens == 0) return hipSuccess;
+  if (a.wk != nullptr) return a.elem == Elem::kBf16 ? launch_kw<Bf16, true>(a, stream) : launch_kw<F16, true>(a, stream);
+  return a.elem == Elem::kBf16 ? launch_kw<Bf16, false>(a, stream) : launch_kw<F16, false>(a, stream);
 }
 
 hipError_t launch_indexer_rope(const RopeArgs& a, hipStream_t stream) {

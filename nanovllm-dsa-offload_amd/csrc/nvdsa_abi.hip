@@ -8,7 +8,7 @@
 #include <string>
 #include <vector>
 
-#include "../../include/nvdsa.h"
+#include "../../include/nvdsa_ext.h"
 #include "nvdsa_common.h"
 #include "nvdsa_kernels.h"
 
@@ -184,7 +184,8 @@ const char* nvdsa_kernel_name(int32_t kernel_id) {
                                 "lim_threshold_kernel",  "lim_mtp_victims_kernel", "lim_mtp_pass_b_kernel",
                                 "sfa_mtp_overlap_kernel", "sfa_split_kernel_copied", "indexer_project_kernel",
                                 "indexer_rope_kernel", "persist_blocks_kernel", "lim_classify_kernel",
-                                "lim_chunks_kernel",   "lim_resolve_kernel"};
+                                "lim_chunks_kernel",   "lim_resolve_kernel",
+                                "indexer_kw_kernel",   "indexer_kw_finish_kernel"};
   static_assert(sizeof(names) / sizeof(names[0]) == nvdsa::kKernCount, "one name per kernel id");
   if (kernel_id < 0 || kernel_id >= nvdsa::kKernCount) return "unknown";
   return names[kernel_id];
@@ -1102,6 +1103,92 @@ int nvdsa_dsa_indexer_project_query_only(const nvdsa_tensor* hidden_states, cons
   a.elem = elem_of(hidden_states);
   return launch_status(nvdsa::launch_indexer_project(a, static_cast<hipStream_t>(stream)),
                        "dsa_indexer_project_query_only");
+}
+
+// ------------------------------------------------------------------------
+size_t nvdsa_dsa_indexer_project_kw_workspace_size(int64_t tokens, int64_t n_head, int64_t hidden_size, int32_t with_k) {
+  if (tokens < 0 || n_head <= 0 || hidden_size <= 0) return 0;
+  return nvdsa::indexer_kw_workspace_bytes(tokens, n_head, hidden_size, with_k != 0);
+}
+
+int nvdsa_dsa_indexer_project_kw(const nvdsa_tensor* hidden_states, const nvdsa_tensor* cos, const nvdsa_tensor* sin,
+                                 const nvdsa_tensor* wk_weight, const nvdsa_tensor* k_norm_weight,
+                                 const nvdsa_tensor* k_norm_bias, const nvdsa_tensor* weights_proj_weight,
+                                 const nvdsa_tensor* index_k_out, const nvdsa_tensor* index_weights_out,
+                                 int64_t rope_dim, double score_scale, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+  const nvdsa_tensor* const req[] = {hidden_states, weights_proj_weight, index_weights_out};
+  if (!all_nonnull(req)) return fail(NVDSA_ERR_ARG, "dsa_indexer_project_kw: null tensor argument");
+  const bool with_k = wk_weight != nullptr;
+  if (with_k && !(cos && sin && k_norm_weight && index_k_out))
+    return fail(NVDSA_ERR_ARG, "dsa_indexer_project_kw: wk_weight, k_norm_weight, cos, sin and index_k_out go together");
+  Check c("dsa_indexer_project_kw");
+  const int64_t T = sz(hidden_states, 0), hid = sz(hidden_states, 1), heads = sz(weights_proj_weight, 0);
+  const int dt = hidden_states->dtype;
+  c.need(dims_are(hidden_states, 2) && dims_are(weights_proj_weight, 2) && sz(weights_proj_weight, 1) == hid &&
+             dims_are(index_weights_out, 2) && sz(index_weights_out, 0) == T && sz(index_weights_out, 1) == heads,
+         NVDSA_ERR_SHAPE, "hidden_states [T, hidden], weights_proj_weight [n_head, hidden], index_weights_out [T, n_head]")
+      .need(nvdsa::indexer_kw_supported(heads, hid), NVDSA_ERR_SHAPE,
+            "n_head must be 16, 32 or 64 and hidden_size a positive multiple of 64")
+      .need(is_half(hidden_states) && index_weights_out->dtype == dt &&
+                (weights_proj_weight->dtype == dt || weights_proj_weight->dtype == NVDSA_FLOAT32),
+            NVDSA_ERR_DTYPE, "16-bit activations and outputs; weights_proj_weight in fp32 or their dtype");
+  if (with_k)
+    c.need(dims_are(wk_weight, 2) && sz(wk_weight, 0) == 128 && sz(wk_weight, 1) == hid && dims_are(index_k_out, 2) &&
+               sz(index_k_out, 0) == T && sz(index_k_out, 1) == 128 && numel(k_norm_weight) == 128 &&
+               (!k_norm_bias || numel(k_norm_bias) == 128),
+           NVDSA_ERR_SHAPE, "wk_weight must be [128, hidden], index_k_out [T, 128], the norm's vectors [128]")
+        .need(rope_dim > 0 && rope_dim <= 128 && rope_dim % 2 == 0, NVDSA_ERR_ARG,
+              "rope_dim must be positive, even and at most 128")
+        .need(T == 0 || (numel(cos) % T == 0 && numel(sin) == numel(cos) && numel(cos) / T >= rope_dim &&
+                         numel(cos) / T % 2 == 0),
+              NVDSA_ERR_SHAPE, "cos/sin must hold an even number of at least rope_dim values per token")
+        .need(wk_weight->dtype == dt && k_norm_weight->dtype == dt && (!k_norm_bias || k_norm_bias->dtype == dt) &&
+                  cos->dtype == dt && sin->dtype == dt && index_k_out->dtype == dt,
+              NVDSA_ERR_DTYPE, "all tensors but weights_proj_weight must share one 16-bit dtype");
+  if (c.ok()) {
+    check_common(c, req, hidden_states->device);
+    c.need(hidden_states->device >= 0, NVDSA_ERR_DEVICE, "tensors must be on a GPU")
+        .need(aligned16(hidden_states) && aligned16(weights_proj_weight), NVDSA_ERR_LAYOUT,
+              "inputs and projection weights must be 16-byte aligned");
+    if (with_k) {
+      const nvdsa_tensor* const ks[] = {wk_weight, k_norm_weight, cos, sin, index_k_out};
+      check_common(c, ks, hidden_states->device);
+      if (k_norm_bias) {
+        const nvdsa_tensor* const kb[] = {k_norm_bias};
+        check_common(c, kb, hidden_states->device);
+      }
+      c.need(aligned16(wk_weight) && aligned4(k_norm_weight) && (!k_norm_bias || aligned4(k_norm_bias)) &&
+                 aligned4(cos) && aligned4(sin) && aligned4(index_k_out),
+             NVDSA_ERR_LAYOUT, "wk_weight must be 16-byte aligned, the other tensors 4-byte");
+    }
+    const size_t need = nvdsa::indexer_kw_workspace_bytes(T, heads, hid, with_k);
+    c.need(need == 0 || (workspace != nullptr && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0),
+           NVDSA_ERR_WORKSPACE, "workspace too small");
+  }
+  if (!c.ok()) return c.finish();
+  nvdsa::IndexerKwArgs a{};
+  a.hidden = hidden_states->data;
+  a.w_proj = weights_proj_weight->data;
+  a.w_out = index_weights_out->data;
+  a.partial = static_cast<float*>(workspace);
+  a.tokens = T;
+  a.hid = hid;
+  a.heads = heads;
+  a.score_scale = static_cast<float>(score_scale);
+  a.w_fp32 = weights_proj_weight->dtype == NVDSA_FLOAT32 ? 1 : 0;
+  a.elem = elem_of(hidden_states);
+  if (with_k) {
+    a.wk = wk_weight->data;
+    a.norm_weight = k_norm_weight->data;
+    a.norm_bias = k_norm_bias ? k_norm_bias->data : nullptr;
+    a.cos = cos->data;
+    a.sin = sin->data;
+    a.k_out = index_k_out->data;
+    a.rope_dim = rope_dim;
+    a.cos_stride = T > 0 ? numel(cos) / T : 0;
+  }
+  return launch_status(nvdsa::launch_indexer_kw(a, static_cast<hipStream_t>(stream)), "dsa_indexer_project_kw");
 }
 
 // ------------------------------------------------------------------------

@@ -62,6 +62,13 @@ struct Bf16 {
     u += 0x7fffu + ((u >> 16) & 1u);
     return static_cast<uint16_t>(u >> 16);
   }
+  // Two values rounded to nearest even into one 32-bit word (v_cvt_pk_bf16_f32:
+  // one instruction for what from_float does in six per value).
+  __device__ static inline uint32_t pack2(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+  }
   // Leading part of a hi + lo split: truncation (the lo part takes the rest).
   __device__ static inline uint16_t hi_part(float f) { return static_cast<uint16_t>(__float_as_uint(f) >> 16); }
   __device__ static inline f32x16_t mfma32(vec8 a, vec8 b, f32x16_t c) {
@@ -83,6 +90,9 @@ struct F16 {
     return __builtin_bit_cast(uint16_t, h);
   }
   __device__ static inline uint16_t from_finite(float f) { return from_float(f); }
+  __device__ static inline uint32_t pack2(float a, float b) {
+    return static_cast<uint32_t>(from_float(a)) | (static_cast<uint32_t>(from_float(b)) << 16);
+  }
   __device__ static inline uint16_t hi_part(float f) { return from_float(f); }
   __device__ static inline f32x16_t mfma32(vec8 a, vec8 b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);

@@ -33,7 +33,9 @@ enum KernelId : int {
   kKernLimClassify = 17,
   kKernLimChunks = 18,
   kKernLimResolve = 19,
-  kKernCount = 20
+  kKernIdxKw = 20,
+  kKernIdxKwFinish = 21,
+  kKernCount = 22
 };
 // Timing events for the next launch of `kernel_id` when instrumentation is
 // on for the calling thread (nvdsa_profile_begin); both null otherwise.
@@ -202,6 +204,28 @@ struct IndexerArgs {
 // K extents (rank, hid) must be multiples of this.
 int64_t indexer_k_chunk();
 hipError_t launch_indexer_project(const IndexerArgs& a, hipStream_t stream);
+
+// Products of hidden_states for many tokens: the index key (wk != null) and
+// the head weights.
+struct IndexerKwArgs {
+  const void* hidden;       // [tokens, hid] 16-bit
+  const void* wk;           // [128, hid] 16-bit, or null: no key
+  const void* norm_weight;  // [128] 16-bit
+  const void* norm_bias;    // [128] 16-bit, or null
+  const void* w_proj;       // [heads, hid] fp32 (w_fp32) or 16-bit
+  const void* cos;          // [tokens, cos_stride]
+  const void* sin;
+  void* k_out;              // [tokens, 128]
+  void* w_out;              // [tokens, heads]
+  float* partial;           // workspace
+  int64_t tokens, hid, heads, rope_dim, cos_stride;
+  float score_scale;
+  int w_fp32;
+  Elem elem;
+};
+bool indexer_kw_supported(int64_t heads, int64_t hid);
+size_t indexer_kw_workspace_bytes(int64_t tokens, int64_t heads, int64_t hid, bool with_k);
+hipError_t launch_indexer_kw(const IndexerKwArgs& a, hipStream_t stream);
 
 struct RopeArgs {
   void* q;              // [rows = tokens * heads, head_dim], rotated in place

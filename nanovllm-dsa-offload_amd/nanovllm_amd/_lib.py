@@ -83,6 +83,12 @@ SIGNATURES = {
     "nvdsa_xcd_roles_record": ([ctypes.c_int32], None),
 }
 
+# include/nvdsa_ext.h
+EXT_SIGNATURES = {
+    "nvdsa_dsa_indexer_project_kw_workspace_size": ([_I64, _I64, _I64, ctypes.c_int32], _SZ),
+    "nvdsa_dsa_indexer_project_kw": ([_P] * 9 + [_I64, _DBL, _VP, _SZ, _VP], ctypes.c_int),
+}
+
 
 def _load() -> ctypes.CDLL:
     if not LIB_PATH.exists():
@@ -91,7 +97,7 @@ def _load() -> ctypes.CDLL:
             "(or nanovllm-dsa-offload_amd/csrc/build.py) first."
         )
     lib = ctypes.CDLL(str(LIB_PATH), mode=ctypes.RTLD_GLOBAL)
-    for name, (argtypes, restype) in SIGNATURES.items():
+    for name, (argtypes, restype) in {**SIGNATURES, **EXT_SIGNATURES}.items():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = restype

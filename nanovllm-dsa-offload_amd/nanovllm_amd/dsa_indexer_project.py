@@ -67,18 +67,52 @@ def _weights_fp32(hidden_states, weights_proj_weight, score_scale: float) -> tor
     return weights.to(hidden_states.dtype)
 
 
+def _plain(t, shape, dtypes, device, align=16) -> bool:
+    """A contiguous tensor of this shape that the HIP kernels read as it is."""
+    return (t.shape == shape and t.dtype in dtypes and t.device == device and t.is_contiguous()
+            and t.data_ptr() % align == 0)
+
+
+def _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, n_head) -> bool:
+    """Whether the head weights can come from the fp32-product kernel
+    (nvdsa_dsa_indexer_project_kw): plain tensors of the indexer's shapes;
+    any other form keeps the library GEMM."""
+    if hidden_states.dim() != 2 or weights_proj_weight.dim() != 2 or hidden_states.shape[0] == 0:
+        return False
+    hidden = hidden_states.shape[1]
+    dtype, device = hidden_states.dtype, hidden_states.device
+    return (dtype in (torch.bfloat16, torch.float16) and n_head in (16, 32, 64) and hidden > 0 and hidden % 64 == 0
+            and _plain(hidden_states, hidden_states.shape, (dtype,), device)
+            and _plain(weights_proj_weight, (n_head, hidden), (dtype, torch.float32), device)
+            and _plain(index_weights_out, (hidden_states.shape[0], n_head), (dtype,), device, 2)
+            and not (torch.is_grad_enabled() and (hidden_states.requires_grad or weights_proj_weight.requires_grad)))
+
+
+# Tokens of one group of the fused decode launch; past it q comes from the
+# tiled GEMM and the head weights from their own kernel.
+_GROUP_TOKENS = 64
+
+
 def dsa_indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, weights_proj_weight, q_index_out,
                                    index_weights_out, *, n_head, head_dim, rope_dim, score_scale, wq_b_bmm_t=None,
                                    enable_q_bmm=False):
     """Decode-only indexer projection (reference dsa_indexer_project.py:296-355)."""
     del wq_b_bmm_t, enable_q_bmm  # the fused kernel reads wq_b_weight directly
-    if q_index_out.shape != (hidden_states.shape[0], n_head, head_dim):
-        raise ValueError(f"q_index_out shape must be {(hidden_states.shape[0], n_head, head_dim)}, "
-                         f"got {tuple(q_index_out.shape)}")
-    if index_weights_out.shape != (hidden_states.shape[0], n_head):
-        raise ValueError(f"index_weights_out shape must be {(hidden_states.shape[0], n_head)}, "
-                         f"got {tuple(index_weights_out.shape)}")
+    tokens = hidden_states.shape[0]
+    if q_index_out.shape != (tokens, n_head, head_dim):
+        raise ValueError(f"q_index_out shape must be {(tokens, n_head, head_dim)}, got {tuple(q_index_out.shape)}")
+    if index_weights_out.shape != (tokens, n_head):
+        raise ValueError(f"index_weights_out shape must be {(tokens, n_head)}, got {tuple(index_weights_out.shape)}")
     same = weights_proj_weight.dtype == hidden_states.dtype
+    # One launch for both up to a group of tokens; more tokens (or fp32 head
+    # weights) take the head weights' own kernel where it reads their form.
+    if ((not same or tokens > _GROUP_TOKENS)
+            and _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, n_head)):
+        ops.indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, None, q_index_out, None, n_head,
+                                       head_dim, rope_dim, score_scale)
+        ops.indexer_project_kw(hidden_states, None, None, None, None, None, weights_proj_weight, None,
+                               index_weights_out, rope_dim, score_scale)
+        return q_index_out, index_weights_out
     ops.indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, weights_proj_weight if same else None,
                                    q_index_out, index_weights_out if same else None, n_head, head_dim, rope_dim,
                                    score_scale)
@@ -98,6 +132,20 @@ def dsa_indexer_project(hidden_states, q_c, cos, sin, wq_b_weight, wk_weight, k_
     # q: projection + RoPE in one launch (no weights part).
     ops.indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, None, q_index_out, None, n_head,
                                    head_dim, rope_dim, 1.0)
+    # k and the head weights: one pass over hidden_states where every tensor
+    # has the plain form that the kernels read (weights_proj_weight in fp32,
+    # or in 16 bits, which only the library path widens before the product).
+    dtype, device = hidden_states.dtype, hidden_states.device
+    norm = [t for t in (k_norm_weight, k_norm_bias) if t is not None]
+    if (weights_proj_weight.dtype == torch.float32 and int(head_dim) == 128 and k_norm_weight is not None
+            and _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, int(n_head))
+            and _plain(wk_weight, (128, hidden_states.shape[1]), (dtype,), device)
+            and all(_plain(t, (128,), (dtype,), device, 4) for t in norm)
+            and (cos.numel() // tokens) % 2 == 0 and index_k_out.data_ptr() % 4 == 0
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in (wk_weight, *norm)))):
+        ops.indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias, weights_proj_weight,
+                               index_k_out, index_weights_out, int(rope_dim), score_scale)
+        return q_index_out, index_k_out, index_weights_out
     # k: library projection and layer norm, then the RoPE kernel on [T, 1, D].
     k = F.linear(hidden_states, wk_weight)
     k = F.layer_norm(k, (int(head_dim),), k_norm_weight, k_norm_bias, eps=1e-6)

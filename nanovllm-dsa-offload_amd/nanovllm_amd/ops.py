@@ -255,6 +255,22 @@ def indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, weight
         int(n_head), int(head_dim), int(rope_dim), float(score_scale), _stream_of(q_c)))
 
 
+def indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias, weights_proj_weight, index_k_out,
+                       index_weights_out, rope_dim, score_scale) -> None:
+    """nvdsa_dsa_indexer_project_kw on the current stream: the index key and
+    the head weights of many tokens.  Pass the key's tensors (cos, sin,
+    wk_weight, k_norm_weight, k_norm_bias, index_k_out) as None to compute
+    the head weights only."""
+    descs = [_D(t) if t is not None else None for t in (hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias,
+                                                         weights_proj_weight, index_k_out, index_weights_out)]
+    nbytes = _L.nvdsa_dsa_indexer_project_kw_workspace_size(hidden_states.shape[0], weights_proj_weight.shape[0],
+                                                            hidden_states.shape[1], int(wk_weight is not None))
+    ws = _workspace(hidden_states.device, nbytes)
+    _lib.check(_L.nvdsa_dsa_indexer_project_kw(*(None if d is None else _ref(d) for d in descs), int(rope_dim),
+                                               float(score_scale), ws.data_ptr(), ws.numel(),
+                                               _stream_of(hidden_states)))
+
+
 def persist_prefill_blocks(hbm_kv_cache, hbm_k_rope, dram_kv_cache, dram_k_rope, hbm_block_ids,
                            dram_block_ids) -> None:
     """nvdsa_persist_prefill_blocks on the current stream (no host sync)."""

@@ -233,3 +233,89 @@ def test_project_errors():
                                        torch.empty(T, H, D, dtype=dtype, device="cuda"),
                                        torch.empty(T, H, dtype=dtype, device="cuda"), n_head=H, head_dim=D,
                                        rope_dim=ROPE, score_scale=1.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,heads,head_dim,rank,rope", [
+    (65, 16, 16, 256, 6),        # 64 x 64 tiles, one token in the last
+    (1000, 16, 48, 256, 18),     # heads that end inside a 32-wide tile
+    (15999, 16, 16, 512, 16),    # 128 x 128 tiles, all dims rotated
+    (49001, 16, 16, 256, 10),    # 256 x 256 tiles
+    (300, 32, 128, 2048, 64),    # the GLM indexer's shape
+])
+def test_project_many_tokens_close(dtype, T, heads, head_dim, rank, rope):
+    """The tiled GEMM path (more than 64 tokens), every tile shape, ragged
+    token counts; guard rows around the output stay untouched."""
+    from nanovllm_amd import ops
+
+    print(f"PROJECT GEMM {dtype} T={T} heads={heads}x{head_dim} rank={rank} rope={rope}", flush=True)
+    rng = np.random.default_rng(T)
+    qc = _to_bits(rng.standard_normal((T, rank)), dtype)
+    wq = _to_bits(rng.standard_normal((heads * head_dim, rank)) / np.sqrt(rank), dtype)
+    c, s = _cos_sin(T, dtype, rope, seed=T)
+    buf = torch.full((T + 2, heads, head_dim), 7.0, dtype=dtype, device="cuda")
+    hidden = torch.zeros(T, 64, dtype=dtype, device="cuda")
+    ops.indexer_project_query_only(hidden, _dev(qc, dtype), _dev(c, dtype), _dev(s, dtype), _dev(wq, dtype), None,
+                                   buf[1:T + 1], None, heads, head_dim, rope, 1.0)
+    torch.cuda.synchronize()
+    eq, _ = I.project_query_only(np.zeros((T, 64), np.uint16), qc, c, s, wq, np.zeros((heads, 64), np.float32), heads,
+                                 head_dim, rope, 1.0, dname(dtype))
+    got = bits(buf)
+    seven = _to_bits(np.full((heads, head_dim), 7.0), dtype)
+    assert np.array_equal(got[0], seven) and np.array_equal(got[T + 1], seven)
+    if rope < head_dim:
+        _close(got[1:T + 1][..., rope:], eq[..., rope:], dtype)
+    _close(got[1:T + 1][..., :rope], eq[..., :rope], dtype, min_exact=0.95, pairs=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,heads,hid,fp32,bias", [(1, 16, 64, True, True), (127, 32, 6144, True, False),
+                                                   (128, 64, 192, False, True), (129, 32, 6144, True, True),
+                                                   (700, 64, 1088, True, True), (33000, 16, 128, False, False)])
+def test_project_key_and_weights_kernel(dtype, T, heads, hid, fp32, bias):
+    """Index key and head weights of many tokens against the fp64 oracle:
+    token tiles' edges, one to many hidden_size slices, fp32 and 16-bit head
+    weights."""
+    from nanovllm_amd import ops
+
+    print(f"PROJECT kw {dtype} T={T} heads={heads} hid={hid} fp32={fp32}", flush=True)
+    rng = np.random.default_rng(T + heads)
+    hidden = _to_bits(rng.standard_normal((T, hid)), dtype)
+    wk = _to_bits(rng.standard_normal((D, hid)) / np.sqrt(hid), dtype)
+    wp = np.asarray(rng.standard_normal((heads, hid)) / np.sqrt(hid), np.float32)
+    wp_bits = None if fp32 else _to_bits(wp, dtype)
+    kw = _to_bits(rng.uniform(0.75, 1.25, D), dtype)
+    kb = _to_bits(rng.uniform(-0.125, 0.125, D), dtype) if bias else None
+    c, s = _cos_sin(T, dtype, ROPE, seed=T)
+    k_out = torch.full((T + 2, D), 7.0, dtype=dtype, device="cuda")
+    w_out = torch.full((T + 2, heads), 7.0, dtype=dtype, device="cuda")
+    wp_dev = torch.from_numpy(wp).to("cuda") if fp32 else _dev(wp_bits, dtype)
+    ops.indexer_project_kw(_dev(hidden, dtype), _dev(c, dtype), _dev(s, dtype), _dev(wk, dtype), _dev(kw, dtype),
+                           _dev(kb, dtype) if bias else None, wp_dev, k_out[1:T + 1], w_out[1:T + 1], ROPE, 0.25)
+    only_w = torch.empty(T, heads, dtype=dtype, device="cuda")
+    ops.indexer_project_kw(_dev(hidden, dtype), None, None, None, None, None, wp_dev, None, only_w, ROPE, 0.25)
+    torch.cuda.synchronize()
+    qc, wq = np.zeros((T, 16), np.uint16), np.zeros((heads * D, 16), np.uint16)
+    _, ek, ew = I.project_full(hidden, qc, c, s, wq, wk, kw, kb, wp, heads, D, ROPE, 0.25, dname(dtype))
+    if not fp32:
+        _, ew = I.project_query_only(hidden, qc, c, s, wq, wp_bits, heads, D, ROPE, 0.25, dname(dtype))
+    gk, gw = bits(k_out), bits(w_out)
+    for g in (gk, gw):
+        assert np.array_equal(g[0], _to_bits(np.full(g.shape[1], 7.0), dtype))
+        assert np.array_equal(g[T + 1], _to_bits(np.full(g.shape[1], 7.0), dtype))
+    _close(gw[1:T + 1], ew, dtype)
+    _close(bits(only_w), ew, dtype)
+    # A key value is (x - mean) rstd g + b of a sum x rounded to 16 bits.  The
+    # fp32 sum may round one step of x away: 2^-8 (bf16) or 2^-11 (fp16) of |x|
+    # on either side of a power of two, so 2^-7 / 2^-10 of |x| at most, times
+    # rstd g.  With 128 sums of unit variance |mean| stays below 0.5 (5.6
+    # sigma), |rstd g| below 1.25 * 1.3, and |b| below 0.125, so
+    # |x rstd g| <= |y| + 0.125 + 0.5 * 1.63 < |y| + 0.95.  The value's own
+    # rounding adds one step of |y|, the rotation mixes a pair's two values.
+    rel = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    g64 = O.bits_to_f32(gk[1:T + 1], dname(dtype)).astype(np.float64)
+    e64 = O.bits_to_f32(ek, dname(dtype)).astype(np.float64)
+    mag = np.repeat(np.hypot(e64[:, 0::2], e64[:, 1::2]), 2, axis=-1)
+    excess = np.abs(g64 - e64) - rel * (2 * mag + 1.41 * 0.95)
+    assert np.all(excess <= 0), float(excess.max())
+    assert np.mean(gk[1:T + 1] == ek) >= 0.9
