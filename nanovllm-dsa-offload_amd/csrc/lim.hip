@@ -418,28 +418,29 @@ __device__ __forceinline__ SelectOut radix_select_visit(int k, uint32_t kmin, ui
     __syncthreads();
     // Thread tid owns bins [tb*kBinsPerThread, +kBinsPerThread), threads in
     // descending bin order; find the bin holding the remaining-th largest.
+    // (The thread that holds it reads its bins again: kept in registers across
+    // the scan they are 16 more for every caller.)
     const int tb = kManageThreads - 1 - tid;
-    int cnt[kBinsPerThread];
+    uint32_t* own = hist + tb * kBinsPerThread;
     int sum = 0;
 #pragma unroll
-    for (int j = 0; j < kBinsPerThread; ++j) {
-      cnt[j] = static_cast<int>(hist[tb * kBinsPerThread + j]);
-      hist[tb * kBinsPerThread + j] = 0u;  // ready for the next pass / call
-      sum += cnt[j];
-    }
+    for (int j = 0; j < kBinsPerThread; ++j) sum += static_cast<int>(own[j]);
     int total;
     int acc = block_exclusive_scan(sum, scratch, &total);
     if (acc < remaining && remaining <= acc + sum) {
-#pragma unroll
+#pragma unroll 1
       for (int j = kBinsPerThread - 1; j >= 0; --j) {
-        if (acc < remaining && remaining <= acc + cnt[j]) {
+        const int cnt = static_cast<int>(own[j]);
+        if (acc < remaining && remaining <= acc + cnt) {
           bcast[0] = tb * kBinsPerThread + j;
           bcast[1] = acc;
-          bcast[2] = cnt[j];
+          bcast[2] = cnt;
         }
-        acc += cnt[j];
+        acc += cnt;
       }
     }
+#pragma unroll
+    for (int j = 0; j < kBinsPerThread; ++j) own[j] = 0u;  // ready for the next pass / call
     __syncthreads();
     prefix |= static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(bcast[0])) << lo;
     pmask |= dmask << lo;
@@ -485,7 +486,7 @@ __device__ __forceinline__ SelectOut radix_select_visit(int k, uint32_t kmin, ui
 // Same, with the keys supplied in groups of four: load(i, key[4], inc[4])
 // for group i < ngroups, groups strided over the workgroup.
 template <typename Load>
-__device__ SelectOut radix_select(int ngroups, int k, uint32_t kmin, uint32_t kmax, Load load, uint32_t* hist,
+__device__ __forceinline__ SelectOut radix_select(int ngroups, int k, uint32_t kmin, uint32_t kmax, Load load, uint32_t* hist,
                                   int* scratch, int* bcast) {
   return radix_select_visit(
       k, kmin, kmax,
@@ -762,6 +763,48 @@ __device__ __forceinline__ void load_slot_states(const uint32_t* stab, uint32_t 
   }
 }
 
+// The victims among this thread's ITEMS slots [tid * ITEMS, +ITEMS) (bit e =
+// slot tid * ITEMS + e) when only some of the non-hit slots `nh` are taken:
+// the m with the largest inverted keys, ties at the threshold to the lower
+// slots.  Requires 0 < m < non-hit slots of the workgroup.
+template <int ITEMS, bool LDS_ONLY>
+__device__ __forceinline__ unsigned victim_mask(int m, unsigned nh, const uint32_t (&key)[ITEMS], uint32_t* hist,
+                                                int* scratch, int* bcast, uint32_t* red) {
+  uint32_t lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+  for (int e = 0; e < ITEMS; ++e)
+    if ((nh >> e) & 1u) {
+      lo = min(lo, key[e]);
+      hi = max(hi, key[e]);
+    }
+  block_minmax(lo, hi, red);
+  const SelectOut sel = radix_select_visit(
+      m, lo, hi,
+      [&](auto&& fn) {
+#pragma unroll
+        for (int e = 0; e < ITEMS; ++e)
+          if ((nh >> e) & 1u) fn(key[e]);
+      },
+      hist, scratch, bcast);
+  unsigned vmask = 0u, eqmask = 0u;
+#pragma unroll
+  for (int e = 0; e < ITEMS; ++e)
+    if ((nh >> e) & 1u) {
+      if (key[e] > sel.thresh) vmask |= 1u << e;
+      if (key[e] == sel.thresh) eqmask |= 1u << e;
+    }
+  if (sel.cnt_eq == sel.need_eq) return vmask | eqmask;
+  int tot;
+  int r = block_exclusive_scan<LDS_ONLY>(__popc(eqmask), scratch, &tot);
+#pragma unroll
+  for (int e = 0; e < ITEMS; ++e)
+    if ((eqmask >> e) & 1u) {
+      if (r < sel.need_eq) vmask |= 1u << e;
+      ++r;
+    }
+  return vmask;
+}
+
 // select_victims with the slot states and keys held in registers (from
 // load_slot_regs): thread t owns slots [t*ITEMS, (t+1)*ITEMS) (slot order =
 // thread-major order).  Same result as select_victims; requires
@@ -781,50 +824,8 @@ __device__ __forceinline__ int select_victims_in_regs(int c, int m, const uint32
     key[e] = ~(state == kStateFree ? 0u : kv[e]);  // smallest score = largest inverted key; free slots first
     if (i0 + e < c && state != kStateHit) nh |= 1u << e;
   }
-  uint32_t lo = 0xffffffffu, hi = 0u;
-#pragma unroll
-  for (int e = 0; e < ITEMS; ++e)
-    if ((nh >> e) & 1u) {
-      lo = min(lo, key[e]);
-      hi = max(hi, key[e]);
-    }
   const int nonhit = block_sum<LDS_ONLY>(__popc(nh), scratch);
-  const bool take_all = m >= nonhit;
-  SelectOut sel{0, 0, 0};
-  if (!take_all) {
-    block_minmax(lo, hi, red);
-    sel = radix_select_visit(
-        m, lo, hi,
-        [&](auto&& fn) {
-#pragma unroll
-          for (int e = 0; e < ITEMS; ++e)
-            if ((nh >> e) & 1u) fn(key[e]);
-        },
-        hist, scratch, bcast);
-  }
-  unsigned vmask = 0u, eqmask = 0u;
-  if (take_all) {
-    vmask = nh;
-  } else {
-#pragma unroll
-    for (int e = 0; e < ITEMS; ++e)
-      if ((nh >> e) & 1u) {
-        if (key[e] > sel.thresh) vmask |= 1u << e;
-        if (key[e] == sel.thresh) eqmask |= 1u << e;
-      }
-    if (sel.cnt_eq != sel.need_eq) {  // ties at the threshold: lowest slots first
-      int tot;
-      int r = block_exclusive_scan<LDS_ONLY>(__popc(eqmask), scratch, &tot);
-#pragma unroll
-      for (int e = 0; e < ITEMS; ++e)
-        if ((eqmask >> e) & 1u) {
-          if (r < sel.need_eq) vmask |= 1u << e;
-          ++r;
-        }
-    } else {
-      vmask |= eqmask;
-    }
-  }
+  const unsigned vmask = m >= nonhit ? nh : victim_mask<ITEMS, LDS_ONLY>(m, nh, key, hist, scratch, bcast, red);
   int tot;
   int pos = block_exclusive_scan<LDS_ONLY>(__popc(vmask), scratch, &tot);
 #pragma unroll
@@ -1465,24 +1466,40 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
     }
   }
   // The slot table, cim and the in-bin miss list are complete.  Only the
-  // global slot table's readers (the streamed paths) need the full barrier.
+  // global slot table's readers (larger budgets, the streamed classification)
+  // need the full barrier.
   if (direct && slots_in_regs)
     lds_barrier();
   else
     __syncthreads();
-  // The slot states in registers (their keys only where victims are
-  // selected, below).
+  // The slot states in registers, thread t owning slots [t * ITEMS, +ITEMS):
+  // 4 per thread for budgets up to 2048 (from the patched LDS copy; their keys
+  // only where victims are selected, below), 16 up to 8192.  Larger budgets
+  // walk the slot table in memory on every pass.  At C = 8192 the walked form
+  // took 36 of the kernel's 65 us (24 requests of 65536): a dozen dependent
+  // passes of one workgroup over 64 KB, each with its own block scan; the
+  // register form takes the kernel to 35 us.  The wide form keeps masks of its
+  // slots, not the states: with 16 states and 16 keys live the kernel passes
+  // its 128 registers, and scratch memory costs every launch 1.5 us.
+  constexpr int kSlotRegsWide = 16;
+  const bool slots_wide = !slots_in_regs && c <= kSlotRegsWide * kManageThreads;
   uint32_t st[kSlotRegs];
-  if (slots_in_regs) {
-    const uint32_t* src = direct ? lst : stab;  // (the global table after the streamed classification)
+  unsigned nh = 0u, hm = 0u, cand = 0u;  // this thread's non-hit and hit slots below c; slots of unselected tokens
+  auto slot_masks = [&](const auto& states, auto items) {
 #pragma unroll
-    for (int j = 0; j < kSlotRegs; j += 4) {
-      const uint4 v = *reinterpret_cast<const uint4*>(src + tid * kSlotRegs + j);
-      st[j] = v.x;
-      st[j + 1] = v.y;
-      st[j + 2] = v.z;
-      st[j + 3] = v.w;
+    for (int e = 0; e < decltype(items)::value; ++e) {
+      const uint32_t state = states[e] >> kStateShift;
+      if (tid * decltype(items)::value + e < c) (state == kStateHit ? hm : nh) |= 1u << e;
+      if (state == kStateCand) cand |= 1u << e;
     }
+  };
+  if (slots_in_regs) {
+    load_slot_states<kSlotRegs>(direct ? lst : stab, st);  // (the global table after the streamed classification)
+    slot_masks(st, std::integral_constant<int, kSlotRegs>{});
+  } else if (slots_wide) {
+    uint32_t states[kSlotRegsWide];
+    load_slot_states<kSlotRegsWide>(stab, states);
+    slot_masks(states, std::integral_constant<int, kSlotRegsWide>{});
   }
 
   // 4. Misses per chunk, their bases, and the victims.  With the slots in
@@ -1491,18 +1508,6 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
   //    every non-hit slot is a victim (C = 2048 with a full pool) the victims
   //    come straight from it, in ascending slot order.
   const int mine = tid < active ? L.cdm[tid] + L.cim[tid] : 0;
-  const int i0 = tid * kSlotRegs;
-  unsigned nh = 0u, hm = 0u;  // this thread's non-hit and hit slots below c
-  if (slots_in_regs) {
-#pragma unroll
-    for (int e = 0; e < kSlotRegs; ++e)
-      if (i0 + e < c) {
-        if ((st[e] >> kStateShift) == kStateHit)
-          hm |= 1u << e;
-        else
-          nh |= 1u << e;
-      }
-  }
   // Fields: misses [42, 64), non-hit slots [21, 42), hits [0, 21) (block
   // totals stay below 2^21: at most 512 chunks of 4096 tokens, c < 2^14).
   uint64_t tot4;
@@ -1524,7 +1529,7 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
 #pragma unroll
     for (int e = 0; e < kSlotRegs; ++e)
       if ((nh >> e) & 1u) {
-        L.vsl[pos] = i0 + e;
+        L.vsl[pos] = tid * kSlotRegs + e;
         L.vev[pos] = (st[e] >> kStateShift) == kStateCand ? static_cast<int>(st[e] & kTokenMask) : -1;
         ++pos;
       }
@@ -1533,9 +1538,7 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
     uint32_t kv[kSlotRegs];
     if (slots_in_regs) {
       if (keyed) {
-        const uint32_t* src = direct ? lkv : skey;
-#pragma unroll
-        for (int e = 0; e < kSlotRegs; ++e) kv[e] = src[tid * kSlotRegs + e];
+        load_slot_states<kSlotRegs>(direct ? lkv : skey, kv);
       } else {
         // c = kTopK with more non-hit slots than misses (a pool naming one
         // slot twice): no key table was kept, a candidate slot's key is its
@@ -1551,6 +1554,31 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
     lds_barrier();
     if (slots_in_regs) {
       nv = select_victims_in_regs<kSlotRegs, true>(c, m, st, kv, L.vsl, hist, L.scratch, L.bcast, L.red, L.vev);
+    } else if (slots_wide) {
+      unsigned vmask = nh;
+      if (m < nonhit) {
+        vmask = 0u;
+        if (m > 0) {
+          uint32_t key[kSlotRegsWide];
+          load_slot_states<kSlotRegsWide>(skey, key);
+#pragma unroll
+          for (int e = 0; e < kSlotRegsWide; ++e) key[e] = ~((cand >> e) & 1u ? key[e] : 0u);  // free slots first
+          vmask = victim_mask<kSlotRegsWide, true>(m, nh, key, hist, L.scratch, L.bcast, L.red);
+        }
+      }
+      int pos = block_exclusive_scan<true>(__popc(vmask), L.scratch, &nv);
+      nv = min(nv, m);
+#pragma unroll
+      for (int e = 0; e < kSlotRegsWide; ++e)
+        if ((vmask >> e) & 1u) {
+          if (pos < nv) L.vsl[pos] = tid * kSlotRegsWide + e;
+          ++pos;
+        }
+      lds_barrier();
+      for (int i = tid; i < nv; i += kManageThreads) {
+        const uint32_t ent = stab[L.vsl[i]];
+        L.vev[i] = (ent >> kStateShift) == kStateCand ? static_cast<int>(ent & kTokenMask) : -1;
+      }
     } else {
       nv = select_victims(c, m, stab, skey, L.vsl, hist, L.scratch, L.bcast, L.red, L.vev);
     }
@@ -1661,26 +1689,30 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
   }
 
   // 7. Then the hits by descending old slot (reference BuildHitMissKey order).
-  if (!slots_in_regs) {
+  if (!slots_in_regs && !slots_wide) {
     write_hit_rows(a, b, c, m, stab, L.scratch);
     return;
   }
-  unsigned hm7 = 0u;
+  int above = nhits - L.cim[tid] - __popc(hm);  // hits in higher slots (cim: in lower ones, this thread's own word)
+  auto place_hits = [&](const auto& states, auto items) {
 #pragma unroll
-  for (int e = 0; e < kSlotRegs; ++e)
-    if (i0 + e < c && (st[e] >> kStateShift) == kStateHit) hm7 |= 1u << e;
-  const int below = L.cim[tid];                 // hits in lower slots (this thread's own word)
-  int above = nhits - below - __popc(hm7);      // hits in higher slots
-#pragma unroll
-  for (int e = kSlotRegs - 1; e >= 0; --e)
-    if ((hm7 >> e) & 1u) {
-      const int pos = m + above;
-      if (pos < kTopK) {
-        out_src[pos] = static_cast<int32_t>(st[e] & kTokenMask);
-        out_dst[pos] = i0 + e;
+    for (int e = decltype(items)::value - 1; e >= 0; --e)
+      if ((hm >> e) & 1u) {
+        const int pos = m + above;
+        if (pos < kTopK) {
+          out_src[pos] = static_cast<int32_t>(states[e] & kTokenMask);
+          out_dst[pos] = tid * decltype(items)::value + e;
+        }
+        ++above;
       }
-      ++above;
-    }
+  };
+  if (slots_in_regs) {
+    place_hits(st, std::integral_constant<int, kSlotRegs>{});
+  } else {
+    uint32_t states[kSlotRegsWide];
+    load_slot_states<kSlotRegsWide>(stab, states);  // (hit entries: no longer written)
+    place_hits(states, std::integral_constant<int, kSlotRegsWide>{});
+  }
   // Positions a corrupt pool (duplicate slots) left unfilled.
   for (int pos = m + nhits + tid; pos < kTopK; pos += kManageThreads) {
     out_src[pos] = -1;

@@ -130,6 +130,29 @@ def test_lim_closed_form_and_repeat(heads, batch, seq_len, cache_tokens, miss):
     _validate(d, pool1, seq_len, cache_tokens, 0)
 
 
+@pytest.mark.parametrize("cache_tokens,miss,fill", [
+    (2049, 1, "full"), (2049, 2048, "full"), (2560, 0, "full"), (4000, 700, "free"), (8191, 2047, "full"),
+    (8192, 300, "full"), (8192, 2048, "cold"), (8193, 300, "free"), (16383, 2048, "full"),
+])
+def test_lim_victims_by_budget_bit_exact(cache_tokens, miss, fill):
+    """Victim selection either side of every budget class (2048, 8192 slots):
+    slots all held, some free, a cold pool row (every victim key equal);
+    integers and pool against the oracle."""
+    print(f"LIM victims C={cache_tokens} miss={miss} fill={fill}", flush=True)
+    case = _structured_case(32, 2, 20480, cache_tokens, miss, seed=cache_tokens + miss)
+    pool = case["cache_slots_pool"]
+    held = (pool[1] >= 0).nonzero().view(-1)
+    lower = held[held < 20480 - TOPK]  # unselected tokens
+    if fill == "free":
+        pool[1, lower[::3]] = -1
+    elif fill == "cold":
+        pool[1].fill_(-1)
+    expect = oracle_lim(case)
+    d = case.to_device(torch.device("cuda", 0))
+    _run_lim(d)
+    _assert_matches(d, expect, False)
+
+
 @pytest.mark.parametrize("n_tokens,cache_tokens", [(12288, 2048), (20480, 6144)])
 def test_lim_cold_pool_rows_bit_exact(n_tokens, cache_tokens):
     """Pool rows with nothing cached (every selected token a miss, every
