@@ -38,6 +38,27 @@ int nvdsa_dsa_indexer_project_kw(const nvdsa_tensor* hidden_states,
                                  size_t workspace_bytes,
                                  void* stream);
 
+/* One row-wise copy of nvdsa_stage_inputs: rows [0, real) of dst (dst_bytes
+ * apart) take src_bytes of src's row (src_stride bytes apart) and the 32-bit
+ * pattern `fill` after them, rows [real, rows) the pattern alone.  All sizes
+ * and addresses are multiples of 2 (of 4 unless the pattern's halves are
+ * equal). */
+typedef struct nvdsa_stage_item {
+  void* dst;
+  const void* src;
+  int64_t rows;
+  int64_t real;
+  int64_t dst_bytes;
+  int64_t src_bytes;
+  int64_t src_stride;
+  int64_t fill;
+} nvdsa_stage_item;
+/* Up to 16 such copies in one launch: the inputs of a decode step into a
+ * captured graph's fixed buffers (reference
+ * nanovllm/engine/full_decode_graph.py:546-720 copies them one by one).  No
+ * item may read what another one writes. */
+int nvdsa_stage_inputs(const nvdsa_stage_item* items, int64_t count, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

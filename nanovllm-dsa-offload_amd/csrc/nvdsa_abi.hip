@@ -185,7 +185,8 @@ const char* nvdsa_kernel_name(int32_t kernel_id) {
                                 "sfa_mtp_overlap_kernel", "sfa_split_kernel_copied", "indexer_project_kernel",
                                 "indexer_rope_kernel", "persist_blocks_kernel", "lim_classify_kernel",
                                 "lim_chunks_kernel",   "lim_resolve_kernel",
-                                "indexer_kw_kernel",   "indexer_kw_finish_kernel"};
+                                "indexer_kw_kernel",   "indexer_kw_finish_kernel",
+                                "stage_inputs_kernel"};
   static_assert(sizeof(names) / sizeof(names[0]) == nvdsa::kKernCount, "one name per kernel id");
   if (kernel_id < 0 || kernel_id >= nvdsa::kKernCount) return "unknown";
   return names[kernel_id];
@@ -1235,6 +1236,33 @@ int nvdsa_persist_prefill_blocks(const nvdsa_tensor* hbm_kv_cache, const nvdsa_t
   a.dram_blocks = sz(dram_kv_cache, 0);
   if (a.count * 4 >= kMaxGridThreads / 256) return fail(NVDSA_ERR_SHAPE, "persist_prefill_blocks: too many blocks");
   return launch_status(nvdsa::launch_persist_blocks(a, static_cast<hipStream_t>(stream)), "persist_prefill_blocks");
+}
+
+// ------------------------------------------------------------------------
+int nvdsa_stage_inputs(const nvdsa_stage_item* items, int64_t count, void* stream) {
+  if (count < 0 || count > nvdsa::kMaxStageItems || (count > 0 && !items))
+    return fail(NVDSA_ERR_ARG, "stage_inputs: 0 to 16 items");
+  nvdsa::StageArgs a{};
+  for (int64_t i = 0; i < count; ++i) {
+    const nvdsa_stage_item& it = items[i];
+    if (it.rows < 0 || it.real < 0 || it.real > it.rows || it.src_bytes < 0 || it.src_bytes > it.dst_bytes ||
+        it.src_stride < 0)
+      return fail(NVDSA_ERR_SHAPE, "stage_inputs: rows or widths out of range");
+    if (it.rows == 0 || it.dst_bytes == 0) continue;
+    const bool reads = it.real > 0 && it.src_bytes > 0;
+    if (!it.dst || (reads && !it.src)) return fail(NVDSA_ERR_ARG, "stage_inputs: null data pointer");
+    const uint32_t f = static_cast<uint32_t>(it.fill);
+    const uintptr_t all = reinterpret_cast<uintptr_t>(it.dst) | static_cast<uintptr_t>(it.dst_bytes) |
+                          (reads ? reinterpret_cast<uintptr_t>(it.src) | static_cast<uintptr_t>(it.src_bytes) |
+                                       static_cast<uintptr_t>(it.src_stride)
+                                 : 0);
+    if ((all & 1) != 0 || ((all & 3) != 0 && (f >> 16) != (f & 0xffffu)))
+      return fail(NVDSA_ERR_LAYOUT, "stage_inputs: addresses and widths must be multiples of 2 (4 with a 32-bit pattern)");
+    nvdsa::StageItem& d = a.items[a.count++];
+    d = {it.dst, reads ? it.src : nullptr, it.rows, reads ? it.real : 0, it.dst_bytes, reads ? it.src_bytes : 0,
+         reads ? it.src_stride : 0, static_cast<int32_t>(f), 0};
+  }
+  return launch_status(nvdsa::launch_stage_inputs(a, static_cast<hipStream_t>(stream)), "stage_inputs");
 }
 
 // ------------------------------------------------------------------------

@@ -35,7 +35,8 @@ enum KernelId : int {
   kKernLimResolve = 19,
   kKernIdxKw = 20,
   kKernIdxKwFinish = 21,
-  kKernCount = 22
+  kKernStage = 22,
+  kKernCount = 23
 };
 // Timing events for the next launch of `kernel_id` when instrumentation is
 // on for the calling thread (nvdsa_profile_begin); both null otherwise.
@@ -247,5 +248,24 @@ struct PersistArgs {
   int64_t count, hbm_blocks, dram_blocks;
 };
 hipError_t launch_persist_blocks(const PersistArgs& a, hipStream_t stream);
+
+// ---- staging of a captured graph's inputs ---------------------------------
+// Rows [0, real) take src_bytes from src (src_stride bytes apart) and `fill`
+// (32-bit pattern; its low half for 2-byte units) after them; rows
+// [real, rows) take `fill` alone.  Rows of dst lie dst_bytes apart.
+struct StageItem {
+  void* dst;
+  const void* src;
+  int64_t rows, real, dst_bytes, src_bytes, src_stride;
+  int32_t fill;
+  int32_t unit;  // 16, 4 or 2 bytes, set by the launch
+};
+constexpr int kMaxStageItems = 16;
+struct StageArgs {
+  StageItem items[kMaxStageItems];
+  int32_t first_block[kMaxStageItems];
+  int32_t count;
+};
+hipError_t launch_stage_inputs(StageArgs& a, hipStream_t stream);
 
 }  // namespace nvdsa

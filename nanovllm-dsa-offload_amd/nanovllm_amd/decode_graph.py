@@ -20,17 +20,21 @@ layer-step ``fused_li_manage(_mtp) -> fused_copy_sfa(_mtp)``.
 * The KV caches, index keys and the LIDU pool are the caller's persistent
   tensors; their addresses are baked into the graph, as in the reference.
 
-Inputs are copied with ordinary eager torch copies on the current stream
-before each replay; nothing inside the graph is a memset.
+Inputs are copied on the current stream before each replay, all in one
+launch (``nvdsa_stage_inputs``; with a tensor of another device, dtype or
+layout among them, by ordinary torch copies); nothing inside the graph is a
+memset.
 """
 
 from __future__ import annotations
 
+import math
 from typing import Iterable
 
 import torch
 
 from . import dsa_offload_ops as ops
+from . import ops as _op_impl
 
 MTP_QUERIES = 4
 TOPK = 2048
@@ -90,17 +94,30 @@ class DsaLayerGraph:
         self.persistent = dict(index_key_cache=index_key_cache, cache_slots_pool=cache_slots_pool,
                                hbm_k_rope=hbm_k_rope, hbm_kv_cache=hbm_kv_cache, dram_k_rope=dram_k_rope,
                                dram_kv_cache=dram_kv_cache)
-        self.inputs = {
-            "query_index": torch.zeros(rows, index_heads, 128, **f16),
-            "index_weights": torch.zeros(rows, index_heads, **f16),
-            "query_rope": torch.zeros(rows, heads, 64, **f16),
-            "query": torch.zeros(rows, heads, 512, **f16),
-            "index_block_table": torch.zeros(B, index_block_columns, **i32),
-            "hbm_block_table": torch.zeros(B, hbm_block_columns, **i32),
-            "dram_block_table": torch.zeros(B, dram_block_columns, **i32),
+        shapes = {
+            "query_index": ((rows, index_heads, 128), dtype),
+            "index_weights": ((rows, index_heads), dtype),
+            "query_rope": ((rows, heads, 64), dtype),
+            "query": ((rows, heads, 512), dtype),
+            "index_block_table": ((B, index_block_columns), torch.int32),
+            "hbm_block_table": ((B, hbm_block_columns), torch.int32),
+            "dram_block_table": ((B, dram_block_columns), torch.int32),
+            **{name: ((B,), torch.int32) for name in _ROW_INPUTS},
         }
+        # One block of memory holds every static input (256-byte steps), so
+        # whether a runtime tensor lies in any of them is one comparison.
+        self._nbytes = {k: math.prod(shape) * dt.itemsize for k, (shape, dt) in shapes.items()}
+        offsets, total = {}, 0
+        for k, n in self._nbytes.items():
+            offsets[k] = total
+            total += -(-n // 256) * 256
+        self._block = torch.zeros(max(total, 256), dtype=torch.uint8, device=dev)
+        self._span = (self._block.data_ptr(), self._block.data_ptr() + self._block.numel())
+        self._address = {k: self._span[0] + o for k, o in offsets.items()}
+        self.inputs = {k: self._block[offsets[k]:offsets[k] + self._nbytes[k]].view(dt).view(shape)
+                       for k, (shape, dt) in shapes.items()}
         for name, pad in _ROW_INPUTS.items():
-            self.inputs[name] = torch.full((B,), pad, **i32)
+            self.inputs[name].fill_(pad)
         self.outputs = {
             "topk_src_ids": torch.full((rows, 1, TOPK), -1, **i32),
             "topk_dst_slots": torch.full((rows, 1, TOPK), -1, **i32),
@@ -110,6 +127,7 @@ class DsaLayerGraph:
         if mtp:
             self.outputs["miss_src_ids"] = torch.full((B, MTP_QUERIES * TOPK), -1, **i32)
             self.outputs["miss_dst_slots"] = torch.full((B, MTP_QUERIES * TOPK), -1, **i32)
+        self._device = self._block.device
         self.graph: torch.cuda.CUDAGraph | None = None
         self.real_batch = 0
         self.replay_count = 0
@@ -147,6 +165,32 @@ class DsaLayerGraph:
         torch.cuda.current_stream().wait_stream(stream)
 
     # -- per-step inputs --------------------------------------------------------
+    def _stageable(self, name: str, src: torch.Tensor) -> bool:
+        """Whether the staging kernel may read ``src`` for buffer ``name``: a
+        plain tensor of the buffer's dtype on its device, outside the static
+        inputs' memory or the buffer itself."""
+        if type(src) is not torch.Tensor or src.dtype != self.inputs[name].dtype or src.device != self._device:
+            return False
+        at = src.data_ptr()
+        lo, hi = self._span
+        return (at == self._address[name] or not lo <= at < hi) and not (src.requires_grad or src.is_neg())
+
+    def _copy_inputs(self, runtime: dict[str, torch.Tensor], real: int) -> None:
+        """The same with torch copies (any device, dtype and layout)."""
+        q = MTP_QUERIES if self.mtp else 1
+        for name, pad in _ROW_INPUTS.items():
+            self.inputs[name][:real].copy_(runtime[name])
+            self.inputs[name][real:].fill_(pad)
+        for name in _TABLES:
+            src, dst = runtime[name], self.inputs[name]
+            dst[:real, :src.shape[1]].copy_(src)
+            dst[:real, src.shape[1]:].zero_()
+            dst[real:].zero_()
+        for name in _QUERY_INPUTS:
+            dst = self.inputs[name]
+            dst[:real * q].copy_(runtime[name])
+            dst[real * q:].zero_()
+
     def copy_runtime_inputs(self, **runtime: torch.Tensor) -> int:
         """Copy one step's inputs into the static buffers; returns the runtime
         batch.  Every name in ``_ROW_INPUTS``, ``_TABLES`` and
@@ -158,29 +202,42 @@ class DsaLayerGraph:
         if real > self.batch_size:
             raise ValueError(f"runtime batch {real} exceeds the graph's batch size {self.batch_size}")
         q = MTP_QUERIES if self.mtp else 1
+        # Every check first, then one launch that moves what the kernel reads
+        # as it is (same device and dtype, contiguous rows).  Anything else
+        # sends the whole step through torch copies, one after another.
+        staged: list[int] = []
+        plain = torch.cuda.current_device() == self._device.index
         for name, pad in _ROW_INPUTS.items():
             src = runtime[name]
             if src.shape != (real,):
                 raise ValueError(f"{name} must be [{real}], got {tuple(src.shape)}")
-            self.inputs[name][:real].copy_(src)
-            self.inputs[name][real:].fill_(pad)
+            plain = plain and self._stageable(name, src) and src.is_contiguous()
+            if plain:
+                staged += (self._address[name], src.data_ptr(), 1, 1, 4 * self.batch_size, 4 * real, 0, pad)
         for name in _TABLES:
-            src, dst = runtime[name], self.inputs[name]
-            if src.dim() != 2 or src.shape[0] != real:
-                raise ValueError(f"{name} must be rank 2 with {real} rows, got {tuple(src.shape)}")
-            if src.shape[1] > dst.shape[1]:
-                raise ValueError(f"{name} is wider than its graph buffer: runtime={src.shape[1]}, "
-                                 f"graph={dst.shape[1]}.")
-            dst[:real, :src.shape[1]].copy_(src)
-            dst[:real, src.shape[1]:].zero_()
-            dst[real:].zero_()
+            src, width = runtime[name], self.inputs[name].shape[1]
+            shape = src.shape
+            if len(shape) != 2 or shape[0] != real:
+                raise ValueError(f"{name} must be rank 2 with {real} rows, got {tuple(shape)}")
+            if shape[1] > width:
+                raise ValueError(f"{name} is wider than its graph buffer: runtime={shape[1]}, graph={width}.")
+            plain = plain and self._stageable(name, src) and src.stride(1) == 1
+            if plain:
+                staged += (self._address[name], src.data_ptr(), self.batch_size, real, 4 * width, 4 * shape[1],
+                           4 * src.stride(0), 0)
         for name in _QUERY_INPUTS:
             src, dst = runtime[name], self.inputs[name]
             if src.shape[0] != real * q or src.shape[1:] != dst.shape[1:]:
                 raise ValueError(f"{name} must be [{real * q}, {', '.join(map(str, dst.shape[1:]))}], "
                                  f"got {tuple(src.shape)}")
-            dst[:real * q].copy_(src)
-            dst[real * q:].zero_()
+            plain = plain and self._stageable(name, src) and src.is_contiguous()
+            if plain:
+                nbytes = self._nbytes[name]
+                staged += (self._address[name], src.data_ptr(), 1, 1, nbytes, nbytes // self.batch_size * real, 0, 0)
+        if plain:
+            _op_impl.stage_inputs(staged, self._block)
+        else:
+            self._copy_inputs(runtime, real)
         self.real_batch = real
         return real
 

@@ -25,6 +25,7 @@ or pinned CPU tensors; the GPU reads them over the host link.
 from __future__ import annotations
 
 import ctypes
+import struct
 
 import torch
 
@@ -269,6 +270,14 @@ def indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm
     _lib.check(_L.nvdsa_dsa_indexer_project_kw(*(None if d is None else _ref(d) for d in descs), int(rope_dim),
                                                float(score_scale), ws.data_ptr(), ws.numel(),
                                                _stream_of(hidden_states)))
+
+
+def stage_inputs(fields: list[int], like: torch.Tensor) -> None:
+    """nvdsa_stage_inputs on the current stream of ``like``'s device:
+    ``fields`` holds the eight numbers of each copy, in the order of
+    ``nvdsa_stage_item``."""
+    items = struct.pack(f"={len(fields)}q", *fields)
+    _lib.check(_L.nvdsa_stage_inputs(items, len(fields) // 8, _stream_of(like)))
 
 
 def persist_prefill_blocks(hbm_kv_cache, hbm_k_rope, dram_kv_cache, dram_k_rope, hbm_block_ids,

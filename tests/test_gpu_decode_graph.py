@@ -151,3 +151,61 @@ def test_many_captured_graphs_keep_their_workspaces():
         out = g.replay(**runtime)
         torch.cuda.synchronize()
         _check(out, t, exp, False, label)
+
+
+@pytest.mark.parametrize("mtp", [False, True])
+@pytest.mark.parametrize("batch,real,form", [(1, 1, "plain"), (5, 3, "plain"), (5, 5, "odd"), (4, 2, "strided"),
+                                             (3, 0, "plain"), (6, 4, "host"), (5, 4, "own"), (4, 4, "crossed")])
+def test_staged_inputs_match_copies(mtp, batch, real, form):
+    """The one-launch staging against what torch copies leave: odd batches and
+    addresses (2- and 4-byte units), tables that are columns of wider ones,
+    an empty batch, host tensors, a buffer's own memory, another buffer's."""
+    from nanovllm_amd import decode_graph as G
+
+    print(f"STAGE mtp={mtp} batch={batch} real={real} {form}", flush=True)
+    dev, q, heads = "cuda", 4 if mtp else 1, 6
+    gen = torch.Generator(device=dev).manual_seed(batch * 10 + real)
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)  # noqa: E731
+    g = G.DsaLayerGraph(batch, index_key_cache=z(1, 128, 1, 128), cache_slots_pool=torch.zeros(1, 1280, device=dev),
+                        hbm_k_rope=z(1, 128, 1, 64), hbm_kv_cache=z(1, 128, 1, 512), dram_k_rope=z(1, 128, 64),
+                        dram_kv_cache=z(1, 128, 512), hbm_block_columns=7, dram_block_columns=9, heads=heads,
+                        index_heads=32, scale=1.0, mtp=mtp)
+    ints_ = lambda *s: torch.randint(-5, 1000, s, generator=gen, device=dev, dtype=torch.int32)  # noqa: E731
+    half = lambda *s: torch.randn(*s, generator=gen, device=dev).to(torch.bfloat16)  # noqa: E731
+    runtime = {n: ints_(real) for n in G._ROW_INPUTS}
+    for n, cols in zip(G._TABLES, (10, 4, 9)):
+        runtime[n] = ints_(real, cols)
+    for n, tail in zip(G._QUERY_INPUTS, ((32, 128), (32,), (heads, 64), (heads, 512))):
+        runtime[n] = half(real * q, *tail)
+    if form == "odd":
+        for n in list(runtime):
+            t = runtime[n]
+            runtime[n] = torch.cat((t.view(-1)[:1], t.view(-1)))[1:].view(t.shape)
+    elif form == "strided":
+        for n in G._TABLES:
+            runtime[n] = torch.cat((runtime[n], ints_(real, 5)), 1)[:, :runtime[n].shape[1]]
+    elif form == "host":
+        runtime["hbm_block_table"] = runtime["hbm_block_table"].cpu()
+    elif form == "own":
+        g.inputs["query"].copy_(half(batch * q, heads, 512))
+        runtime["query"] = g.inputs["query"][:real * q]
+    elif form == "crossed":
+        g.inputs["num_cache_tokens"].copy_(ints_(batch))
+        runtime["num_candidate_tokens"] = g.inputs["num_cache_tokens"]
+    expect = {}
+    for n, pad in G._ROW_INPUTS.items():
+        expect[n] = torch.full((batch,), pad, dtype=torch.int32, device=dev)
+        expect[n][:real] = runtime[n]
+    for n in G._TABLES:
+        expect[n] = torch.zeros(batch, g.inputs[n].shape[1], dtype=torch.int32, device=dev)
+        expect[n][:real, :runtime[n].shape[1]] = runtime[n].to(dev)
+    for n in G._QUERY_INPUTS:
+        expect[n] = torch.zeros_like(g.inputs[n])
+        expect[n][:real * q] = runtime[n]
+    for n, t in g.inputs.items():  # whatever the last step left
+        if form not in ("own", "crossed"):
+            t.fill_(77)
+    assert g.copy_runtime_inputs(**runtime) == real
+    torch.cuda.synchronize()
+    for n, t in expect.items():
+        assert torch.equal(g.inputs[n], t), n
