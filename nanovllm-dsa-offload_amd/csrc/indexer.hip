@@ -401,31 +401,50 @@ void launch_gemm_shape(const IndexerArgs& a, hipStream_t stream) {
 // (w_proj in fp32, or 16-bit).  Both read hidden_states, the only large
 // operand, so one kernel reads it once: a workgroup owns 128 tokens x every
 // column x one slice of hidden_size (split so that about one workgroup per CU
-// runs), through LDS as above.  The key columns run on 32x32x16 MFMAs, the
-// head weights on 16x16x4 fp32 MFMAs: the 16-bit activations widened exactly,
-// so a product and its sum round as in an fp32 GEMM (the matrix cores' fp32
-// rate, 1/16 of the 16-bit one, is what bounds the kernel: 1.6 GFLOP at 4096
-// tokens, 10 us of the chip; measured 33 us, 40 us with one K step in flight:
-// the loads' latency).  It replaces two library GEMMs (27 + 24 us), the fp32
-// copy of hidden_states (22 us), a layer norm, the rotation and six small
-// copies and casts.  Slices leave fp32 partial sums; the finish
+// runs), through LDS as above.  Everything runs on 32x32x16 16-bit MFMAs.  An
+// fp32 head weight is cut into three bf16 parts by truncation, 8 mantissa bits
+// each, which hold it exactly (an fp16 activation likewise into two), so every
+// product is exact and only the fp32 sums round, as in an fp32 GEMM.  (On the
+// fp32 MFMA, at 1/16 of the rate, the kernel takes 33 us at 4096 tokens, this
+// form 28.6 us, both 2.0e-3 off fp64 in the rounded outputs; what bounds it
+// now is each CU's pull of 40 KB per K step.)  It replaces two library GEMMs (27 +
+// 24 us), the fp32 copy of hidden_states (22 us), a layer norm, the rotation
+// and six small copies and casts.  Slices leave fp32 partial sums; the finish
 // kernel adds them in slice order, rounds, and does the layer norm, the
 // rotation and the scale: one wave per token.
 constexpr int kKwTok = 128;
 constexpr int kKwThreads = 512;
 constexpr int kKwDim = 128;                   // index key width
 constexpr int kKwMaxSlices = 48;
-constexpr int kKwWRow = kGemmK + 4;            // fp32 LDS row of the head projection (floats)
+constexpr int kKwParts = 3;                    // bf16 parts of a head weight
 
-// HT: 16-head tiles.  K: the key columns too.
+// The bf16 parts of a value, truncated: v = p0 + p1 + p2 exactly.  (Infinities
+// and NaNs stay in p0.)
+__device__ __forceinline__ void bf16_parts(float v, uint16_t (&p)[kKwParts]) {
+  uint32_t u = __float_as_uint(v);
+  if ((u & 0x7f800000u) == 0x7f800000u) {
+    p[0] = static_cast<uint16_t>((u >> 16) | ((u & 0x007fffffu) != 0u ? 0x40u : 0u));
+    p[1] = p[2] = 0;
+    return;
+  }
+  p[0] = static_cast<uint16_t>(u >> 16);
+  const float r1 = v - __uint_as_float(u & 0xffff0000u);
+  p[1] = static_cast<uint16_t>(__float_as_uint(r1) >> 16);
+  const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+  p[2] = static_cast<uint16_t>(__float_as_uint(r2) >> 16);
+}
+
+// HT: 32-head tiles (16 heads: the upper half of the one tile is zeros).  K:
+// the key columns too.
 template <typename T, int HT, bool K>
 __global__ __launch_bounds__(kKwThreads) void indexer_kw_kernel(IndexerKwArgs a, int slices) {
-  constexpr int kHeads = 16 * HT;
-  constexpr int kCols = (K ? kKwDim : 0) + kHeads;
+  constexpr int kRows = 32 * HT;                 // head-weight rows in LDS
+  const int heads = static_cast<int>(a.heads);
+  const int cols = (K ? kKwDim : 0) + heads;
   constexpr int kX = kKwTok * kGemmK, kWk = K ? kKwDim * kGemmK : 0;  // elements of one buffer
   __shared__ __align__(16) uint16_t xs[2][kX];
   __shared__ __align__(16) uint16_t wks[2][K ? kWk : 8];
-  __shared__ __align__(16) float wps[2][kHeads * kKwWRow];
+  __shared__ __align__(16) uint16_t wps[2][kKwParts][kRows * kGemmK];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -439,7 +458,6 @@ __global__ __launch_bounds__(kKwThreads) void indexer_kw_kernel(IndexerKwArgs a,
 
   const int lrow = tid >> 3, lch = tid & 7;     // 64 rows of eight chunks per round
   constexpr int kXl = kKwTok / 64, kWl = K ? kKwDim / 64 : 0;
-  constexpr int kPl = (kHeads * kGemmK / 8 + kKwThreads - 1) / kKwThreads;  // runs of eight head-projection values
   const u32x4_t* xsrc[kXl];
   const u32x4_t* wsrc[kWl > 0 ? kWl : 1];
 #pragma unroll
@@ -452,23 +470,20 @@ __global__ __launch_bounds__(kKwThreads) void indexer_kw_kernel(IndexerKwArgs a,
                                                static_cast<int64_t>(lrow + 64 * j) * hid) + lch;
   const int lpos = lrow * kGemmK + ((lch ^ (lrow & 7)) * 8);
   // Two sets of staged loads: two K steps are in flight while one is multiplied.
-  u32x4_t xv[2][kXl], wv[2][kWl > 0 ? kWl : 1], pv[2][kPl][2];
+  u32x4_t xv[2][kXl], wv[2][kWl > 0 ? kWl : 1], pv[2][2];
   auto load = [&](int set, int s) {
 #pragma unroll
     for (int j = 0; j < kXl; ++j) xv[set][j] = xsrc[j][s * kGemmChunks];
 #pragma unroll
     for (int j = 0; j < kWl; ++j) wv[set][j] = wsrc[j][s * kGemmChunks];
-#pragma unroll
-    for (int j = 0; j < kPl; ++j) {
-      const int r = min(lrow + 64 * j, kHeads - 1);
-      const int64_t at = static_cast<int64_t>(r) * hid + s * kGemmK + lch * 8;
-      if (a.w_fp32) {  // uniform
-        const u32x4_t* p = reinterpret_cast<const u32x4_t*>(static_cast<const float*>(a.w_proj) + at);
-        pv[set][j][0] = p[0];
-        pv[set][j][1] = p[1];
-      } else {
-        pv[set][j][0] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.w_proj) + at);
-      }
+    // Head-weight row lrow (the kernel has at most 64), eight values.
+    const int64_t at = static_cast<int64_t>(min(lrow, heads - 1)) * hid + s * kGemmK + lch * 8;
+    if (a.w_fp32) {  // uniform
+      const u32x4_t* p = reinterpret_cast<const u32x4_t*>(static_cast<const float*>(a.w_proj) + at);
+      pv[set][0] = p[0];
+      pv[set][1] = p[1];
+    } else {
+      pv[set][0] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.w_proj) + at);
     }
   };
   auto store = [&](int set, int buf) {
@@ -476,44 +491,38 @@ __global__ __launch_bounds__(kKwThreads) void indexer_kw_kernel(IndexerKwArgs a,
     for (int j = 0; j < kXl; ++j) *reinterpret_cast<u32x4_t*>(&xs[buf][lpos + 64 * j * kGemmK]) = xv[set][j];
 #pragma unroll
     for (int j = 0; j < kWl; ++j) *reinterpret_cast<u32x4_t*>(&wks[buf][lpos + 64 * j * kGemmK]) = wv[set][j];
+    if (lrow < kRows) {
+      u32x4_t part[kKwParts] = {};
+      if (lrow < heads) {
 #pragma unroll
-    for (int j = 0; j < kPl; ++j) {
-      const int r = lrow + 64 * j;
-      if (r >= kHeads) continue;
-      u32x4_t lo = pv[set][j][0], hi = pv[set][j][1];
-      if (!a.w_fp32) {
+        for (int e = 0; e < 8; ++e) {
+          float v;
+          if (a.w_fp32)
+            v = __uint_as_float(pv[set][e >> 2][e & 3]);
+          else
+            v = T::to_float(static_cast<uint16_t>(pv[set][0][e >> 1] >> (16 * (e & 1))));
+          uint16_t q[kKwParts];
+          bf16_parts(v, q);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t w = pv[set][j][0][e];
-          const uint32_t f0 = __float_as_uint(T::to_float(static_cast<uint16_t>(w)));
-          const uint32_t f1 = __float_as_uint(T::to_float(static_cast<uint16_t>(w >> 16)));
-          if (e < 2) {
-            lo[2 * e] = f0;
-            lo[2 * e + 1] = f1;
-          } else {
-            hi[2 * e - 4] = f0;
-            hi[2 * e - 3] = f1;
-          }
+          for (int i = 0; i < kKwParts; ++i) part[i][e >> 1] |= static_cast<uint32_t>(q[i]) << (16 * (e & 1));
         }
       }
-      float* d = &wps[buf][r * kKwWRow + lch * 8];
-      *reinterpret_cast<u32x4_t*>(d) = lo;
-      *reinterpret_cast<u32x4_t*>(d + 4) = hi;
+#pragma unroll
+      for (int i = 0; i < kKwParts; ++i) *reinterpret_cast<u32x4_t*>(&wps[buf][i][lpos]) = part[i];
     }
   };
 
-  // Key columns: waves 4 (32 tokens) x 2 (64 columns).  Head weights: wave w
-  // takes tokens 16 w .. +15.
-  const int l32 = lane & 31, grp = lane >> 5, l16 = lane & 15, g = lane >> 4;
-  const int wt = wave >> 1, wo = wave & 1;
-  f32x16_t kacc[2];
+  // Waves 0-3: the key columns of 32 tokens each; waves 4-7: their head
+  // weights (a SIMD holds one of either).
+  const int l32 = lane & 31, grp = lane >> 5;
+  const int wt = wave & 3;
+  const bool key_wave = wave < 4;
+  constexpr int kAcc = K && 4 > HT ? 4 : HT;
+  f32x16_t acc[kAcc];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kAcc; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) kacc[i][e] = 0.f;
-  f32x4_t hacc[HT];
-#pragma unroll
-  for (int i = 0; i < HT; ++i) hacc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
   if (s_begin < s_end) {
     const int last = s_end - 1;
     load(0, s_begin);
@@ -523,39 +532,41 @@ __global__ __launch_bounds__(kKwThreads) void indexer_kw_kernel(IndexerKwArgs a,
     lds_barrier();
     auto step = [&](int s, auto parity) {
       constexpr int cur = decltype(parity)::value;  // this step's buffer; the next one's tile is in set cur ^ 1
-      if constexpr (K) {
 #pragma unroll
-        for (int kk = 0; kk < kGemmK / 16; ++kk) {
-          const int ch = ((2 * kk + grp) ^ (l32 & 7)) * 8;
-          const auto xf = *reinterpret_cast<const typename T::vec8*>(&xs[cur][(wt * 32 + l32) * kGemmK + ch]);
+      for (int kk = 0; kk < kGemmK / 16; ++kk) {
+        const int ch = ((2 * kk + grp) ^ (l32 & 7)) * 8;
+        const u32x4_t x8 = *reinterpret_cast<const u32x4_t*>(&xs[cur][(wt * 32 + l32) * kGemmK + ch]);
+        if (key_wave) {
+          if constexpr (K) {
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const auto wf =
-                *reinterpret_cast<const typename T::vec8*>(&wks[cur][(wo * 64 + i * 32 + l32) * kGemmK + ch]);
-            kacc[i] = T::mfma32(wf, xf, kacc[i]);
+            for (int i = 0; i < 4; ++i)
+              acc[i] = T::mfma32(*reinterpret_cast<const typename T::vec8*>(&wks[cur][(i * 32 + l32) * kGemmK + ch]),
+                                 __builtin_bit_cast(typename T::vec8, x8), acc[i]);
           }
-        }
-      }
-      // 32 K per block: lane group g holds K 8 g .. 8 g + 7 of it, and step m
-      // multiplies the four K values 8 g + m.
+        } else {
+          // The activations as bf16: themselves, or an fp16 value's two parts.
+          constexpr int kXParts = std::is_same<T, Bf16>::value ? 1 : 2;
+          u32x4_t xp[kXParts];
+          if constexpr (kXParts == 1) {
+            xp[0] = x8;
+          } else {
 #pragma unroll
-      for (int kb = 0; kb < kGemmK / 32; ++kb) {
-        const u32x4_t x8 = *reinterpret_cast<const u32x4_t*>(
-            &xs[cur][(wave * 16 + l16) * kGemmK + (((4 * kb + g) ^ (l16 & 7)) * 8)]);
-        float xf[8];
+            for (int e = 0; e < 4; ++e) {
+              uint16_t q0[kKwParts], q1[kKwParts];
+              bf16_parts(T::to_float(static_cast<uint16_t>(x8[e])), q0);
+              bf16_parts(T::to_float(static_cast<uint16_t>(x8[e] >> 16)), q1);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          xf[2 * e] = T::to_float(static_cast<uint16_t>(x8[e]));
-          xf[2 * e + 1] = T::to_float(static_cast<uint16_t>(x8[e] >> 16));
-        }
+              for (int h = 0; h < kXParts; ++h) xp[h][e] = static_cast<uint32_t>(q0[h]) | (static_cast<uint32_t>(q1[h]) << 16);
+            }
+          }
 #pragma unroll
-        for (int i = 0; i < HT; ++i) {
-          const float* wp = &wps[cur][(16 * i + l16) * kKwWRow + 32 * kb + 8 * g];
-          const f32x4_t w0 = *reinterpret_cast<const f32x4_t*>(wp);
-          const f32x4_t w1 = *reinterpret_cast<const f32x4_t*>(wp + 4);
+          for (int i = 0; i < HT; ++i)
 #pragma unroll
-          for (int m = 0; m < 8; ++m)
-            hacc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(m < 4 ? w0[m & 3] : w1[m & 3], xf[m], hacc[i], 0, 0, 0);
+            for (int p = 0; p < kKwParts; ++p) {
+              const auto wf = *reinterpret_cast<const bf16x8_t*>(&wps[cur][p][(i * 32 + l32) * kGemmK + ch]);
+#pragma unroll
+              for (int h = 0; h < kXParts; ++h) acc[i] = Bf16::mfma32(wf, __builtin_bit_cast(bf16x8_t, xp[h]), acc[i]);
+            }
         }
       }
       store(cur ^ 1, cur ^ 1);
@@ -568,25 +579,20 @@ __global__ __launch_bounds__(kKwThreads) void indexer_kw_kernel(IndexerKwArgs a,
     }
   }
   // Partial sums [slice][token][column]: the key columns, then the heads.
-  float* out = a.partial + static_cast<int64_t>(slice) * ntok * kCols;
-  if constexpr (K) {
-    const int t = tok0 + wt * 32 + l32;
-    if (t < ntok) {
+  // (Columns from the wave's first one; heads end inside the tile at 16.)
+  const int t = tok0 + wt * 32 + l32;
+  if (t >= ntok || (key_wave && !K)) return;
+  float* out = a.partial + (static_cast<int64_t>(slice) * ntok + t) * cols + (K && !key_wave ? kKwDim : 0);
+  const int width = key_wave ? kKwDim : heads;
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kAcc; ++i)
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4)
-          *reinterpret_cast<float4*>(out + static_cast<int64_t>(t) * kCols + wo * 64 + i * 32 + 8 * g4 + 4 * grp) =
-              make_float4(kacc[i][4 * g4], kacc[i][4 * g4 + 1], kacc[i][4 * g4 + 2], kacc[i][4 * g4 + 3]);
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const int col = i * 32 + 8 * g4 + 4 * grp;
+      if (col < width)
+        *reinterpret_cast<float4*>(out + col) =
+            make_float4(acc[i][4 * g4], acc[i][4 * g4 + 1], acc[i][4 * g4 + 2], acc[i][4 * g4 + 3]);
     }
-  }
-  const int t = tok0 + wave * 16 + l16;  // head 16 i + 4 g + e of token l16
-  if (t < ntok) {
-#pragma unroll
-    for (int i = 0; i < HT; ++i)
-      *reinterpret_cast<float4*>(out + static_cast<int64_t>(t) * kCols + (K ? kKwDim : 0) + 16 * i + 4 * g) =
-          make_float4(hacc[i][0], hacc[i][1], hacc[i][2], hacc[i][3]);
-  }
 }
 
 // One wave per token: lane l holds key dims 2 l, 2 l + 1 (the rotation's
@@ -671,9 +677,9 @@ hipError_t launch_kw_shape(const IndexerKwArgs& a, hipStream_t stream) {
 template <typename T, bool K>
 hipError_t launch_kw(const IndexerKwArgs& a, hipStream_t stream) {
   switch (a.heads) {
-    case 16: return launch_kw_shape<T, 1, K>(a, stream);
-    case 32: return launch_kw_shape<T, 2, K>(a, stream);
-    default: return launch_kw_shape<T, 4, K>(a, stream);
+    case 16:
+    case 32: return launch_kw_shape<T, 1, K>(a, stream);
+    default: return launch_kw_shape<T, 2, K>(a, stream);
   }
 }
 
