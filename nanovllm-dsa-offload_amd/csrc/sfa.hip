@@ -655,12 +655,12 @@ __device__ __forceinline__ void sfa_split_body(const SfaArgs& a, const Partials&
         // does not shrink with it.)
         typename T::vec8 pb_hi, pb_lo;
         uint16_t* phs = reinterpret_cast<uint16_t*>(&pb_hi);
-        uint16_t* pls = reinterpret_cast<uint16_t*>(&pb_lo);
+        uint32_t* plw = reinterpret_cast<uint32_t*>(&pb_lo);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          phs[i] = T::hi_part(p[i]);
-          pls[i] = T::from_finite(p[i] - T::to_float(phs[i]));
-        }
+        for (int i = 0; i < 8; ++i) phs[i] = T::hi_part(p[i]);
+#pragma unroll
+        for (int i = 0; i < 8; i += 2)
+          plw[i / 2] = T::pack2(p[i] - T::to_float(phs[i]), p[i + 1] - T::to_float(phs[i + 1]));
 #pragma unroll
         for (int dt = 0; dt < kVDims / 16; ++dt) {
           const auto af = __builtin_bit_cast(typename T::vec8, make_uint4(vlo[dt].x, vlo[dt].y, vhi[dt].x, vhi[dt].y));
