@@ -1160,7 +1160,8 @@ def measure_lidu_init(torch, np, dev, seed: int, reps: int = 5):
             for _ in range(reps):
                 ops.initialize_lidu_row(**kw)
             torch.cuda.synchronize()
-        km = _kernel_means(kt, ("lim_score_kernel", "lidu_init_kernel", "scatter_copy_kernel"))
+        km = _kernel_means(kt, ("lim_score_kernel", "lim_hist_kernel", "lim_chunks_kernel", "lidu_init_kernel",
+                                "scatter_copy_kernel"))
         out[f"C{c}"] = {"kernels_us": km, "copy_h2d_GBs": round(c * ROW_BYTES / (km["scatter_copy_kernel"] * 1e-6)
                                                                  / 1e9, 2)}
     # A shared layer's copy of the owner's C = 8192 mapping, the pool row as
@@ -1192,7 +1193,8 @@ def measure_lidu_init(torch, np, dev, seed: int, reps: int = 5):
         for _ in range(reps):
             ops.initialize_lidu_row(**kw)
         torch.cuda.synchronize()
-    out["n65536_C2048"] = {"kernels_us": _kernel_means(kt, ("lim_score_kernel", "lidu_init_kernel"))}
+    out["n65536_C2048"] = {"kernels_us": _kernel_means(kt, ("lim_score_kernel", "lim_hist_kernel", "lim_chunks_kernel",
+                                                            "lidu_init_kernel"))}
     del keys, dkpe, dckv, keys64, dkpe64, dckv64
     torch.cuda.empty_cache()
     return out

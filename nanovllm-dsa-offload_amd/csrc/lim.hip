@@ -155,9 +155,9 @@ __host__ __device__ constexpr int score_tokens_per_wave(int q) { return q > 1 ? 
 // RELU = false is the first-decode initialisation score (no ReLU,
 // nanovllm/models/dsa_offload_ops.py:306-311); there `fixed_n` >= 0 gives the
 // candidate count of the single request and the row guards do not apply.
-// For MTP0 management (Q == 1, RELU, side.ranges set) each wave also writes
-// its block's smallest and largest score key, and the workgroups of a request
-// zero the request's state of the chunked management kernels.
+// With one query (side.ranges set) each wave also writes its block's smallest
+// and largest score key, and the workgroups of a request zero the request's
+// state of the chunked selection kernels.
 template <typename T, int HEADS, int Q, bool RELU>
 __global__ __launch_bounds__(kScoreWaves * kWave) void lim_score_kernel(LimArgs a, float* scores, int mtp,
                                                                         int fixed_n, LimWs side) {
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kScoreWaves * kWave) void lim_score_kernel(LimArgs 
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 
-  constexpr bool kRanges = Q == 1 && RELU;
+  constexpr bool kRanges = Q == 1;
   const int64_t cap = a.source_capacity;
   if constexpr (kRanges) {
     if (side.ranges != nullptr) {
@@ -1116,6 +1116,67 @@ __device__ inline void load_keys8(const float* s, int n, int t0, uint32_t* u, bo
   }
 }
 
+// The float whose key `score_key` gives.
+__device__ inline float key_score(uint32_t key) {
+  return __uint_as_float((key & 0x80000000u) ? key & 0x7fffffffu : ~key);
+}
+
+// First digits of a row of linear scores: the scores of both signs that the
+// first decode ranks spread their key range over every exponent down to zero,
+// and the top bits of a key would put hundreds of tokens around the C-th
+// largest into one bin.  The digit is the score's place in [lo, hi] instead,
+// in kHistBins steps: each operation is monotone, so digits order as scores
+// do.  A range that is not finite (or empty) puts every token into bin 0,
+// where the select works on the exact keys.
+struct LinearDigits {
+  float lo, steps;
+  __device__ LinearDigits(uint32_t lo_key, uint32_t hi_key) : lo(key_score(lo_key)) {
+    const float range = key_score(hi_key) - lo;
+    steps = range > 0.f && range <= FLT_MAX ? static_cast<float>(kHistBins) / range : 0.f;
+    if (!(steps <= FLT_MAX)) steps = 0.f;  // (a range of denormals)
+  }
+  __device__ uint32_t operator()(uint32_t key) const {
+    if (steps == 0.f) return 0u;  // (uniform)
+    return min(static_cast<uint32_t>((key_score(key) - lo) * steps), static_cast<uint32_t>(kHistBins - 1));
+  }
+};
+
+// One chunk's share of a row's first-digit histogram `gh`: the row's key range
+// from its blocks' ranges `rg` (part 0 leaves the smallest key and the shift,
+// or the largest key for linear digits, in rowsel), the chunk's digits counted
+// in LDS, then added.
+template <bool LINEAR>
+__device__ __forceinline__ void chunk_first_digits(const float* s, int n, int part, const uint2* rg, uint32_t* gh,
+                                                   uint32_t* rowsel, uint32_t* hist, uint32_t* red) {
+  const int tid = threadIdx.x;
+  uint32_t u[kItems];
+  bool in[kItems];
+  load_keys8(s, n, part * kChunk + tid * kItems, u, in);
+  const int nblocks = static_cast<int>(ceil_div(n, kBlock));
+  uint32_t lo = 0xffffffffu, hi = 0u;
+  for (int i = tid; i < nblocks; i += kManageThreads) {
+    const uint2 v = rg[i];
+    lo = min(lo, v.x);
+    hi = max(hi, v.y);
+  }
+  for (int i = tid; i < kHistBins; i += kManageThreads) hist[i] = 0u;
+  block_minmax<true>(lo, hi, red);  // its barriers also order the clearing before the counts (the key loads stay in flight)
+  const int shift = hist_shift(lo, hi);
+  if (part == 0 && tid == 0) {
+    rowsel[0] = lo;
+    rowsel[1] = LINEAR ? hi : static_cast<uint32_t>(shift);
+  }
+  const LinearDigits digit(lo, hi);
+#pragma unroll
+  for (int e = 0; e < kItems; ++e)
+    if (in[e]) atomicAdd(&hist[LINEAR ? digit(u[e]) : (u[e] - lo) >> shift], 1u);
+  __syncthreads();
+  for (int i = tid; i < kHistBins; i += kManageThreads) {
+    const uint32_t v = hist[i];
+    if (v != 0u) atomicAdd(&gh[i], v);
+  }
+}
+
 __global__ __launch_bounds__(kManageThreads) void lim_hist_kernel(LimArgs a, LimWs w, int parts) {
   __shared__ uint32_t hist[kHistBins];
   __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
@@ -1133,33 +1194,9 @@ __global__ __launch_bounds__(kManageThreads) void lim_hist_kernel(LimArgs a, Lim
   for (int i = part * kManageThreads + tid; i < c; i += parts * kManageThreads) stab[i] = kStateFree;
   if (part * kChunk >= n) return;
   const int64_t cap = a.source_capacity;
-  uint32_t u[kItems];
-  bool in[kItems];
-  load_keys8(w.scores + static_cast<int64_t>(b) * cap, n, part * kChunk + tid * kItems, u, in);
-  const uint2* rg = w.ranges + static_cast<int64_t>(b) * (cap / kBlock);
-  const int nblocks = static_cast<int>(ceil_div(n, kBlock));
-  uint32_t lo = 0xffffffffu, hi = 0u;
-  for (int i = tid; i < nblocks; i += kManageThreads) {
-    const uint2 v = rg[i];
-    lo = min(lo, v.x);
-    hi = max(hi, v.y);
-  }
-  for (int i = tid; i < kHistBins; i += kManageThreads) hist[i] = 0u;
-  block_minmax<true>(lo, hi, red);  // its barriers also order the clearing before the counts (the key loads stay in flight)
-  const int shift = hist_shift(lo, hi);
-  if (part == 0 && tid == 0) {
-    w.rowsel[4 * b] = lo;
-    w.rowsel[4 * b + 1] = static_cast<uint32_t>(shift);
-  }
-#pragma unroll
-  for (int e = 0; e < kItems; ++e)
-    if (in[e]) atomicAdd(&hist[(u[e] - lo) >> shift], 1u);
-  __syncthreads();
-  uint32_t* gh = w.hist + static_cast<int64_t>(b) * kHistBins;
-  for (int i = tid; i < kHistBins; i += kManageThreads) {
-    const uint32_t v = hist[i];
-    if (v != 0u) atomicAdd(&gh[i], v);
-  }
+  chunk_first_digits<false>(w.scores + static_cast<int64_t>(b) * cap, n, part,
+                            w.ranges + static_cast<int64_t>(b) * (cap / kBlock),
+                            w.hist + static_cast<int64_t>(b) * kHistBins, w.rowsel + 4 * b, hist, red);
 }
 
 // The hit half of an MTP0 output row: positions m, m+1, ... get the hits by
@@ -1721,6 +1758,52 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
   if (tid == 0) a.miss_counts[b] = m;
 }
 
+// The first-digit bin holding the k-th largest key of a row, and the count of
+// keys above it: thread tid owns bins [P tb, P tb + P), P = kHistPerThread, tb
+// = 511 - tid, so ascending threads scan descending bins.  (Barriers order LDS
+// only: the caller's loads stay in flight.)
+__device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int* scratch, int* bcast, int& bin,
+                                                int& above) {
+  const int tid = threadIdx.x;
+  constexpr int P = kHistPerThread;
+  const int tb = kManageThreads - 1 - tid;
+  const uint32_t* gh = hist + P * tb;
+  int cnt[P];
+  if constexpr (P == 2) {
+    const uint2 h = *reinterpret_cast<const uint2*>(gh);
+    cnt[0] = static_cast<int>(h.x);
+    cnt[1] = static_cast<int>(h.y);
+  } else {
+#pragma unroll
+    for (int j = 0; j < P; j += 4) {
+      const uint4 h = *reinterpret_cast<const uint4*>(gh + j);
+      cnt[j] = static_cast<int>(h.x);
+      cnt[j + 1] = static_cast<int>(h.y);
+      cnt[j + 2] = static_cast<int>(h.z);
+      cnt[j + 3] = static_cast<int>(h.w);
+    }
+  }
+  int sum = 0;
+#pragma unroll
+  for (int j = 0; j < P; ++j) sum += cnt[j];
+  if (tid == 0) bcast[0] = bcast[1] = 0;  // ordered before the writes below by the scan's barriers
+  int total;
+  int acc = block_exclusive_scan<true>(sum, scratch, &total);  // the token loads stay in flight
+  if (acc < k && k <= acc + sum) {
+#pragma unroll
+    for (int j = P - 1; j >= 0; --j) {
+      if (acc < k && k <= acc + cnt[j]) {
+        bcast[0] = P * tb + j;
+        bcast[1] = acc;
+      }
+      acc += cnt[j];
+    }
+  }
+  lds_barrier();
+  bin = __builtin_amdgcn_readfirstlane(bcast[0]);
+  above = __builtin_amdgcn_readfirstlane(bcast[1]);
+}
+
 // One 4096-token chunk of an MTP0 request (every launch shape): the row's
 // first-digit bin holding the 2048th largest key (from the request's
 // histogram) and the count above it; the chunk's cached tokens go to the slot
@@ -1742,49 +1825,8 @@ __device__ __forceinline__ ChunkSel classify_chunk(const LimArgs& a, const LimWs
   int32_t slot[kItems];
   bool in[kItems];
   load_tokens8(w.scores + static_cast<int64_t>(b) * cap, a.pool + static_cast<int64_t>(r) * cap, n, t0, u, slot, in);
-  // The first-digit bin holding the 2048th largest key: thread tid owns bins
-  // [P tb, P tb + P), P = kHistPerThread, tb = 511 - tid, so ascending threads
-  // scan descending bins.
-  int bin = 0, above = 0;
-  {
-    constexpr int P = kHistPerThread;
-    const int tb = kManageThreads - 1 - tid;
-    const uint32_t* gh = w.hist + static_cast<int64_t>(b) * kHistBins + P * tb;
-    int cnt[P];
-    if constexpr (P == 2) {
-      const uint2 h = *reinterpret_cast<const uint2*>(gh);
-      cnt[0] = static_cast<int>(h.x);
-      cnt[1] = static_cast<int>(h.y);
-    } else {
-#pragma unroll
-      for (int j = 0; j < P; j += 4) {
-        const uint4 h = *reinterpret_cast<const uint4*>(gh + j);
-        cnt[j] = static_cast<int>(h.x);
-        cnt[j + 1] = static_cast<int>(h.y);
-        cnt[j + 2] = static_cast<int>(h.z);
-        cnt[j + 3] = static_cast<int>(h.w);
-      }
-    }
-    int sum = 0;
-#pragma unroll
-    for (int j = 0; j < P; ++j) sum += cnt[j];
-    if (tid == 0) bcast[0] = bcast[1] = 0;  // ordered before the writes below by the scan's barriers
-    int total;
-    int acc = block_exclusive_scan<true>(sum, scratch, &total);  // the token loads stay in flight
-    if (acc < kTopK && kTopK <= acc + sum) {
-#pragma unroll
-      for (int j = P - 1; j >= 0; --j) {
-        if (acc < kTopK && kTopK <= acc + cnt[j]) {
-          bcast[0] = P * tb + j;
-          bcast[1] = acc;
-        }
-        acc += cnt[j];
-      }
-    }
-    lds_barrier();
-    bin = __builtin_amdgcn_readfirstlane(bcast[0]);
-    above = __builtin_amdgcn_readfirstlane(bcast[1]);
-  }
+  int bin, above;
+  first_digit_bin(w.hist + static_cast<int64_t>(b) * kHistBins, kTopK, scratch, bcast, bin, above);
   uint32_t* stab = w.slot_table + static_cast<int64_t>(b) * kTableStride;
   uint32_t* skey = w.slot_key + static_cast<int64_t>(b) * kTableStride;
   unsigned missm = 0u, inbin = 0u;
@@ -2187,164 +2229,123 @@ __global__ __launch_bounds__(kManageThreads) void lim_mtp_pass_b_kernel(LimArgs 
 // 3. First-decode LIDU initialisation (nanovllm/models/dsa_offload_ops.py:251-411).
 
 struct InitWs {
-  float* scores;  // [S_cap]
-  int32_t* src;   // [16384] selected tokens, ascending
-  int32_t* dst;   // [16384] their slots
-  int32_t* count; // list length
+  float* scores;     // [S_cap]
+  int32_t* src;      // [16384] selected tokens, ascending
+  int32_t* dst;      // [16384] their slots
+  int32_t* count;    // list length
+  uint2* ranges;     // [S_cap/128] smallest and largest score key of each 128-token block
+  uint32_t* hist;    // [kHistBins] first-digit histogram
+  uint32_t* rowsel;  // [4] smallest key, first-digit shift, bin of the C-th largest key, keys above it
+  int32_t* counts;   // [parts, 2] keys above the bin, in-bin tokens of each chunk
+  uint2* gather;     // [parts, kGatherPart] in-bin (token, key) of each chunk
+  int32_t* done;     // (cleared by the score kernel)
 };
 
-InitWs carve_init(void* base, int64_t cap) {
-  char* p = static_cast<char*>(base);
-  InitWs w;
-  w.scores = reinterpret_cast<float*>(p);
-  p += align256(sizeof(float) * cap);
-  w.src = reinterpret_cast<int32_t*>(p);
-  p += align256(sizeof(int32_t) * kSlotStride);
-  w.dst = reinterpret_cast<int32_t*>(p);
-  p += align256(sizeof(int32_t) * kSlotStride);
-  w.count = reinterpret_cast<int32_t*>(p);
+// Layout for a pool row of `cap` tokens; with base == nullptr only *bytes is meaningful.
+InitWs init_layout(void* base, int64_t cap, size_t* bytes) {
+  const uintptr_t p0 = reinterpret_cast<uintptr_t>(base);
+  uintptr_t p = p0;
+  auto take = [&](size_t n) {
+    const uintptr_t q = p;
+    p += align256(n);
+    return q;
+  };
+  const size_t n = static_cast<size_t>(cap);
+  InitWs w{};
+  w.scores = reinterpret_cast<float*>(take(sizeof(float) * n));
+  w.src = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * kSlotStride));
+  w.dst = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * kSlotStride));
+  w.count = reinterpret_cast<int32_t*>(take(sizeof(int32_t)));
+  w.ranges = reinterpret_cast<uint2*>(take(sizeof(uint2) * ceil_div(cap, kBlock)));
+  w.hist = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * kHistBins));
+  w.rowsel = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * 4));
+  w.counts = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * 2 * mtp_parts(cap)));
+  w.gather = reinterpret_cast<uint2*>(take(sizeof(uint2) * kGatherPart * mtp_parts(cap)));
+  w.done = reinterpret_cast<int32_t*>(take(sizeof(int32_t)));
+  if (bytes != nullptr) *bytes = p - p0;
   return w;
 }
 
-// Tokens per group of the first-decode selection: 8 chunks of kChunk, thread
-// tid holding tokens gbase + k * kChunk + tid * kItems + e of group gbase.
-constexpr int kInitGroup = 8;
+InitWs carve_init(void* base, int64_t cap) { return init_layout(base, cap, nullptr); }
 
-// Byte range of the buffer resource over the score region: align256(4 row_len)
-// (a multiple of the 16-byte loads), capped at 1 GiB so it fits the 32-bit
-// field; every load offset stays below 4 (n + one group) < 9 MB (n < 2^21).
-__device__ inline int init_score_range(int64_t row_len) {
-  return static_cast<int>(min<size_t>(align256(sizeof(float) * row_len), size_t(1) << 30));
+// The C largest linear scores of tokens [0, n) (ties at the threshold to the
+// lower tokens), slot i to the i-th smallest selected token, the pool row
+// rewritten over its whole length (-1 outside the selection), and the (token,
+// slot) copy list: three kernels of one 512-thread workgroup per 4096-token
+// chunk, on the key ranges that the score kernel leaves.
+//   lidu_hist    the row's first-digit histogram, as lim_hist.
+//   lidu_chunks  the bin holding the C-th largest key; each chunk's count of
+//                keys above it, and its tokens in it (count and list).
+//   lidu_init    every chunk ranks the in-bin tokens of all chunks (a few
+//                dozen), which gives the threshold, the tie cutoff and the
+//                selected tokens before the chunk, and places its own.
+// One workgroup for the row kept every pass on one CU: 25.6 us at 32768
+// tokens (keys in registers), 55 us at 65536 (re-read by each pass); the three
+// kernels take 16 us at 32768 tokens (initialize_lidu_row: 78.5 -> 68 us with the
+// copy).
+
+// Chunk p's keys above the bin and in-bin tokens: counts[2 p], counts[2 p + 1];
+// the first kGatherPart in-bin (token, key) pairs, in token order, at
+// gather[p * kGatherPart].
+__global__ __launch_bounds__(kManageThreads) void lidu_hist_kernel(const float* s, int n, InitWs w) {
+  __shared__ uint32_t hist[kHistBins];
+  __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
+  chunk_first_digits<true>(s, n, blockIdx.x, w.ranges, w.hist, w.rowsel, hist, red);
 }
 
-// One group's score keys: 16 loads per thread in flight together, through a
-// buffer resource over the workspace's score region (align256(4 row_len)
-// bytes, a multiple of the 16-byte loads, so loads past it return zeros
-// without a branch; keys of tokens >= n are never used), turned into
-// order-preserving keys in place.
-__device__ __forceinline__ void load_init_group(__amdgpu_buffer_rsrc_t rsrc, int64_t gbase,
-                                                u32x4_t (&key)[kInitGroup][2]) {
+__global__ __launch_bounds__(kManageThreads) void lidu_chunks_kernel(const float* s, int n, int c, InitWs w) {
+  __shared__ int scratch[kManageThreads / 64 + 1];
+  __shared__ uint64_t scratch64[kManageThreads / 64 + 1];
+  __shared__ int bcast[4];
+  const int part = blockIdx.x, tid = threadIdx.x;
+  const int t0 = part * kChunk + tid * kItems;
+  uint32_t u[kItems];
+  bool in[kItems];
+  load_keys8(s, n, t0, u, in);
+  const LinearDigits digit(w.rowsel[0], w.rowsel[1]);
+  int bin, above;
+  first_digit_bin(w.hist, c, scratch, bcast, bin, above);
+  unsigned inbin = 0u;
+  int over = 0;
 #pragma unroll
-  for (int k = 0; k < kInitGroup; ++k)
+  for (int e = 0; e < kItems; ++e) {
+    if (!in[e]) continue;
+    const uint32_t d = digit(u[e]);
+    if (d == static_cast<uint32_t>(bin)) inbin |= 1u << e;
+    if (d > static_cast<uint32_t>(bin)) ++over;
+  }
+  uint64_t tot;
+  const uint64_t pos =
+      block_exclusive_scan4<true>(static_cast<uint64_t>(over) << 16 | __popc(inbin), scratch64, &tot);
+  int idx = static_cast<int>(pos & 0xffffu);
+  uint2* gl = w.gather + static_cast<int64_t>(part) * kGatherPart;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      key[k][h] = __builtin_amdgcn_raw_buffer_load_b128(
-          rsrc, static_cast<int>((gbase + k * kChunk + threadIdx.x * kItems + 4 * h) * 4), 0, 0);
-#pragma unroll
-  for (int k = 0; k < kInitGroup; ++k)
-#pragma unroll
-    for (int e = 0; e < kItems; ++e) key[k][e >> 2][e & 3] = score_key(__uint_as_float(key[k][e >> 2][e & 3]));
-}
-
-// f(key) for every key of tokens < n in a group: chunks below kfull are
-// whole, chunk kfull is cut at n (element e exists iff e < lim), the ones
-// above lie past n; kfull is uniform, so the element checks stay in the one
-// cut chunk.
-template <typename F>
-__device__ __forceinline__ void visit_init_group(const u32x4_t (&key)[kInitGroup][2], int kfull, int lim, const F& f) {
-#pragma unroll
-  for (int k = 0; k < kInitGroup; ++k) {
-    if (k < kfull) {
-#pragma unroll
-      for (int e = 0; e < kItems; ++e) f(key[k][e >> 2][e & 3]);
-    } else if (k == kfull) {
-#pragma unroll
-      for (int e = 0; e < kItems; ++e)
-        if (e < lim) f(key[k][e >> 2][e & 3]);
+  for (int e = 0; e < kItems; ++e)
+    if ((inbin >> e) & 1u) {
+      if (idx < kGatherPart) gl[idx] = make_uint2(static_cast<uint32_t>(t0 + e), u[e]);
+      ++idx;
+    }
+  if (tid == 0) {
+    w.counts[2 * part] = static_cast<int>((tot >> 16) & 0xffffu);
+    w.counts[2 * part + 1] = static_cast<int>(tot & 0xffffu);
+    if (part == 0) {
+      w.rowsel[2] = static_cast<uint32_t>(bin);
+      w.rowsel[3] = static_cast<uint32_t>(above);
     }
   }
 }
 
-// Smallest and largest key of the group's tokens < n (kfull, lim as for
-// visit_init_group), folded into lo and hi.
-__device__ __forceinline__ void group_minmax(const u32x4_t (&key)[kInitGroup][2], int kfull, int lim, uint32_t& lo,
-                                             uint32_t& hi) {
-#pragma unroll
-  for (int k = 0; k < kInitGroup; ++k) {
-    if (k < kfull) {
-#pragma unroll
-      for (int e = 0; e < kItems; ++e) {
-        lo = min(lo, key[k][e >> 2][e & 3]);
-        hi = max(hi, key[k][e >> 2][e & 3]);
-      }
-    } else if (k == kfull) {
-#pragma unroll
-      for (int e = 0; e < kItems; ++e)
-        if (e < lim) {
-          lo = min(lo, key[k][e >> 2][e & 3]);
-          hi = max(hi, key[k][e >> 2][e & 3]);
-        }
-    }
-  }
-}
-
-// The ordered pass over one group: slot positions of its selected tokens
-// from one 8-counter block scan (two when tied keys must be ranked: only the
-// lowest need_eq tokens equal to the threshold are selected; `eq_run` counts
-// the ties of earlier groups), the pool entries (-1 elsewhere; 16-byte stores
-// when the row allows) and the copy list.  Token order is chunk-major, so the
-// tokens before this thread's chunk-k ones are the earlier chunks' totals
-// plus the chunk-k counts of the lower threads.  Returns the group's count.
-__device__ __forceinline__ int init_group_order(const u32x4_t (&key)[kInitGroup][2], int kfull, int lim,
-                                                const SelectOut& sel, int64_t gbase, int run, int& eq_run,
-                                                int32_t* pool_row, int64_t row_len, bool vec_ok, const InitWs& w,
-                                                uint64_t* scan64) {
+__global__ __launch_bounds__(kManageThreads) void lidu_init_kernel(const float* s, int n, int c, int32_t* pool_row,
+                                                                   int64_t row_len, InitWs w) {
+  __shared__ uint32_t hist[kBins];  // the ranking lists, or the streamed select's histogram
+  __shared__ int scratch[kManageThreads / 64 + 1];
+  __shared__ int bcast[4];
+  __shared__ int goff[kManageThreads], cim[kManageThreads];
   const int tid = threadIdx.x;
-  unsigned selm[kInitGroup], eqm[kInitGroup];
-#pragma unroll
-  for (int k = 0; k < kInitGroup; ++k) {
-    selm[k] = 0u;
-    eqm[k] = 0u;
-    if (k > kfull) continue;  // uniform
-#pragma unroll
-    for (int e = 0; e < kItems; ++e) {
-      if (k == kfull && e >= lim) continue;
-      if (key[k][e >> 2][e & 3] > sel.thresh) selm[k] |= 1u << e;
-      if (key[k][e >> 2][e & 3] == sel.thresh) eqm[k] |= 1u << e;
-    }
-  }
-  if (sel.cnt_eq != sel.need_eq) {
-    uint64_t ec[2] = {0, 0}, etot[2];
-#pragma unroll
-    for (int k = 0; k < kInitGroup; ++k) ec[k >> 2] |= static_cast<uint64_t>(__popc(eqm[k])) << (16 * (k & 3));
-    block_exclusive_scan8(ec, scan64, etot);
-#pragma unroll
-    for (int k = 0; k < kInitGroup; ++k) {
-      int rk = eq_run + lane16x8(ec, k);
-#pragma unroll
-      for (int e = 0; e < kItems; ++e)
-        if ((eqm[k] >> e) & 1u) {
-          if (rk < sel.need_eq) selm[k] |= 1u << e;
-          ++rk;
-        }
-      eq_run += lane16x8(etot, k);
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < kInitGroup; ++k) selm[k] |= eqm[k];
-  }
-  uint64_t sc[2] = {0, 0}, stot[2];
-#pragma unroll
-  for (int k = 0; k < kInitGroup; ++k) sc[k >> 2] |= static_cast<uint64_t>(__popc(selm[k])) << (16 * (k & 3));
-  block_exclusive_scan8(sc, scan64, stot);
-  int count = 0;
-#pragma unroll
-  for (int k = 0; k < kInitGroup; ++k) {
-    const int64_t t0 = gbase + static_cast<int64_t>(k) * kChunk + tid * kItems;
-    int pos = run + count + lane16x8(sc, k);
-    int pv[kItems];
-#pragma unroll
-    for (int e = 0; e < kItems; ++e) {
-      pv[e] = -1;
-      if ((selm[k] >> e) & 1u) {
-        pv[e] = pos;
-        if (pos < kSlotStride) {
-          w.src[pos] = static_cast<int32_t>(t0 + e);
-          w.dst[pos] = pos;
-        }
-        ++pos;
-      }
-    }
+  const int part = blockIdx.x;
+  const int64_t t0 = static_cast<int64_t>(part) * kChunk + tid * kItems;
+  const bool vec_ok = (reinterpret_cast<uintptr_t>(pool_row) & 15) == 0;  // uniform
+  auto store_pool = [&](const int (&pv)[kItems]) {
     if (vec_ok && t0 + kItems <= row_len) {
       *reinterpret_cast<int4*>(pool_row + t0) = make_int4(pv[0], pv[1], pv[2], pv[3]);
       *reinterpret_cast<int4*>(pool_row + t0 + 4) = make_int4(pv[4], pv[5], pv[6], pv[7]);
@@ -2353,93 +2354,117 @@ __device__ __forceinline__ int init_group_order(const u32x4_t (&key)[kInitGroup]
       for (int e = 0; e < kItems; ++e)
         if (t0 + e < row_len) pool_row[t0 + e] = pv[e];
     }
-    count += lane16x8(stot, k);
-  }
-  return count;
-}
-
-// One workgroup: the C largest linear scores of tokens [0, n) (ties at the
-// threshold to the lower tokens), slot i to the i-th smallest selected token,
-// the pool row rewritten over its whole length (-1 outside the selection),
-// and the (token, slot) copy list.  Any n: every pass (range, radix digits,
-// ordered pass) walks the scores group by group, one load round trip per
-// group of 32768 tokens.
-__global__ __launch_bounds__(kManageThreads) void lidu_init_kernel(const float* s, int n, int c, int32_t* pool_row,
-                                                                   int64_t row_len, InitWs w) {
-  __shared__ uint32_t hist[kBins];
-  __shared__ int scratch[kManageThreads / 64 + 1];
-  __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
-  __shared__ int bcast[4];
-  __shared__ uint64_t scan64[2 * (kManageThreads / 64)];
-  const int tid = threadIdx.x;
-  const __amdgpu_buffer_rsrc_t srsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(s), 0, init_score_range(row_len), kBufferFlags);
-  for (int i = tid; i < kBins; i += kManageThreads) hist[i] = 0u;
-  constexpr int kGroupTokens = kInitGroup * kChunk;
-  auto each_key = [&](auto f) {
-    for (int gbase = 0; gbase < n; gbase += kGroupTokens) {
-      u32x4_t key[kInitGroup][2];
-      load_init_group(srsrc, gbase, key);
-      const int kfull = (n - gbase) / kChunk;
-      visit_init_group(key, kfull, n - gbase - kfull * kChunk - tid * kItems, f);
-    }
   };
-  uint32_t lo = 0xffffffffu, hi = 0u;
-  for (int gbase = 0; gbase < n; gbase += kGroupTokens) {
-    u32x4_t key[kInitGroup][2];
-    load_init_group(srsrc, gbase, key);
-    const int kfull = (n - gbase) / kChunk;
-    group_minmax(key, kfull, n - gbase - kfull * kChunk - tid * kItems, lo, hi);
+  if (static_cast<int64_t>(part) * kChunk >= n) {  // past the source: nothing selected
+    const int none[kItems] = {-1, -1, -1, -1, -1, -1, -1, -1};
+    store_pool(none);
+    return;
   }
-  block_minmax(lo, hi, red);
-  const SelectOut sel = radix_select_visit(c, lo, hi, each_key, hist, scratch, bcast);
-  const bool vec_ok = (reinterpret_cast<uintptr_t>(pool_row) & 15) == 0;  // uniform
-  int run = 0, eq_run = 0;
-  for (int64_t gbase = 0; gbase < row_len; gbase += kGroupTokens) {
-    if (gbase >= n) {  // past the source: nothing selected
-      for (int64_t t = gbase + tid; t < min<int64_t>(row_len, gbase + kGroupTokens); t += kManageThreads)
-        pool_row[t] = -1;
-      continue;
+  uint32_t u[kItems];
+  bool in[kItems];
+  load_keys8(s, n, static_cast<int>(t0), u, in);
+  const int active = static_cast<int>(ceil_div(n, kChunk));  // <= kManageThreads (n < 2^21)
+  const int above = tid < active ? w.counts[2 * tid] : 0;
+  const int ni = tid < active ? w.counts[2 * tid + 1] : 0;
+  const uint32_t lo = w.rowsel[0], hi = w.rowsel[1], bin = w.rowsel[2];
+  const int k = c - static_cast<int>(w.rowsel[3]);  // in-bin tokens to select
+  cim[tid] = 0;
+  int g;
+  const int off = block_exclusive_scan<true>(ni, scratch, &g);
+  if (tid < active) goff[tid] = off;
+  const bool direct = block_or_lds(ni > kGatherPart ? 1u : 0u, scratch) == 0u && g <= kRankDirect;
+  uint32_t thr;
+  int cutoff = INT_MAX;
+  int before;  // selected tokens of the chunks before this one
+  if (direct) {
+    uint32_t* lkey = hist;
+    int* ltok = reinterpret_cast<int*>(hist + kRankDirect);
+    if (tid < g) {
+      const int p = chunk_of(goff, active, tid);
+      const uint2 x = w.gather[static_cast<int64_t>(p) * kGatherPart + (tid - goff[p])];
+      ltok[tid] = static_cast<int>(x.x);
+      lkey[tid] = x.y;
     }
-    u32x4_t key[kInitGroup][2];
-    load_init_group(srsrc, gbase, key);
-    const int kfull = static_cast<int>((n - gbase) / kChunk);
-    run += init_group_order(key, kfull, static_cast<int>(n - gbase - kfull * kChunk - tid * kItems), sel, gbase, run,
-                            eq_run, pool_row, row_len, vec_ok, w, scan64);
+    lds_barrier();
+    if (tid < g) {  // key descending, then token ascending
+      const int my_t = ltok[tid];
+      const uint32_t my_k = lkey[tid];
+      int rank = 0;
+      for (int j = 0; j < g; ++j) rank += (lkey[j] > my_k || (lkey[j] == my_k && ltok[j] < my_t)) ? 1 : 0;
+      if (rank < k) atomicAdd(&cim[my_t / kChunk], 1);
+      if (rank == k - 1) {  // the last selected token: the threshold and the tie cutoff
+        bcast[0] = static_cast<int>(my_k);
+        bcast[1] = my_t;
+      }
+    }
+    lds_barrier();
+    thr = static_cast<uint32_t>(bcast[0]);
+    cutoff = bcast[1];
+    before = block_sum<true>(tid < part ? above + cim[tid] : 0, scratch);
+  } else {
+    // More in-bin tokens than the lists hold (heavy ties): every chunk selects
+    // from the whole row by itself.
+    for (int i = tid; i < kBins; i += kManageThreads) hist[i] = 0u;
+    __syncthreads();
+    const LinearDigits digit(lo, hi);
+    const int ngroups = static_cast<int>(ceil_div(n, 4));
+    auto load_bin = [&](int gi, uint32_t* key, bool* inc) {
+      load_score_keys(s, n, 4 * gi, key, inc);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) inc[e] = inc[e] && digit(key[e]) == bin;
+    };
+    const SelectOut sel = radix_select(ngroups, k, lo, hi, load_bin, hist, scratch, bcast);
+    thr = sel.thresh;
+    // Ties in token order up to the last one selected (its token is the
+    // cutoff), and the selected tokens before this chunk on the way.
+    int ties = 0, mine = 0;
+    for (int g0 = 0; g0 < ngroups; g0 += kManageThreads) {
+      const int gi = g0 + tid;
+      unsigned eqm = 0u;
+      if (gi < ngroups) {
+        uint32_t key[4];
+        bool inc[4];
+        load_score_keys(s, n, 4 * gi, key, inc);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (inc[e] && key[e] == thr) eqm |= 1u << e;
+          if (inc[e] && key[e] > thr && 4 * gi + e < part * kChunk) ++mine;
+        }
+      }
+      ties = tie_cutoff_step(eqm, 4 * gi, sel.need_eq - 1, ties, scratch, bcast);
+    }
+    __syncthreads();
+    cutoff = bcast[3];
+    for (int gi = tid; 4 * gi < part * kChunk; gi += kManageThreads) {
+      uint32_t key[4];
+      bool inc[4];
+      load_score_keys(s, n, 4 * gi, key, inc);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mine += inc[e] && key[e] == thr && 4 * gi + e <= cutoff ? 1 : 0;
+    }
+    before = block_sum(mine, scratch);
   }
-  if (tid == 0) *w.count = run;
-}
-
-// lidu_init_kernel for sources of at most one group (32768 tokens): the
-// group's keys stay in registers across the range, the radix passes and the
-// ordered pass instead of being re-read for each.
-__global__ __launch_bounds__(kManageThreads) void lidu_init_reg_kernel(const float* s, int n, int c,
-                                                                       int32_t* pool_row, int64_t row_len, InitWs w) {
-  __shared__ uint32_t hist[kBins];
-  __shared__ int scratch[kManageThreads / 64 + 1];
-  __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
-  __shared__ int bcast[4];
-  __shared__ uint64_t scan64[2 * (kManageThreads / 64)];
-  const int tid = threadIdx.x;
-  const __amdgpu_buffer_rsrc_t srsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(s), 0, init_score_range(row_len), kBufferFlags);
-  u32x4_t key[kInitGroup][2];
-  load_init_group(srsrc, 0, key);
-  for (int i = tid; i < kBins; i += kManageThreads) hist[i] = 0u;
-  const int kfull = n / kChunk;
-  const int lim = n - kfull * kChunk - tid * kItems;
-  auto each_key = [&](auto f) { visit_init_group(key, kfull, lim, f); };
-  uint32_t lo = 0xffffffffu, hi = 0u;
-  group_minmax(key, kfull, lim, lo, hi);
-  block_minmax(lo, hi, red);
-  const SelectOut sel = radix_select_visit(c, lo, hi, each_key, hist, scratch, bcast);
-  int eq_run = 0;
-  const int run = init_group_order(key, kfull, lim, sel, 0, 0, eq_run, pool_row, row_len,
-                                   (reinterpret_cast<uintptr_t>(pool_row) & 15) == 0, w, scan64);
-  // The rest of the pool row lies past the source: nothing selected there.
-  for (int64_t t = static_cast<int64_t>(kInitGroup) * kChunk + tid; t < row_len; t += kManageThreads)
-    pool_row[t] = -1;
-  if (tid == 0) *w.count = run;
+  unsigned selm = 0u;
+#pragma unroll
+  for (int e = 0; e < kItems; ++e)
+    if (in[e] && mtp0_selected(u[e], static_cast<int>(t0) + e, thr, cutoff)) selm |= 1u << e;
+  int tot;
+  int pos = before + block_exclusive_scan<true>(__popc(selm), scratch, &tot);
+  int pv[kItems];
+#pragma unroll
+  for (int e = 0; e < kItems; ++e) {
+    pv[e] = -1;
+    if ((selm >> e) & 1u) {
+      pv[e] = pos;
+      if (pos < kSlotStride) {
+        w.src[pos] = static_cast<int32_t>(t0 + e);
+        w.dst[pos] = pos;
+      }
+      ++pos;
+    }
+  }
+  store_pool(pv);
+  if (tid == 0 && part == active - 1) *w.count = before + tot;
 }
 
 // One workgroup: the (token, slot) list of every entry >= 0 of an owner's
@@ -2513,13 +2538,17 @@ hipError_t launch_lidu_scores(const LiduInitArgs& a, const InitWs& w, hipStream_
   la.source_capacity = a.row_len;
   la.heads = a.heads;
   la.batch = 1;
+  LimWs side{};
+  side.ranges = w.ranges;
+  side.hist = w.hist;
+  side.done = w.done;
   const dim3 grid(static_cast<uint32_t>(ceil_div(ceil_div(a.n, kBlock), kScoreWaves)), 1);
   if (a.heads == 32) {
     launch_kernel(kKernLimScore, lim_score_kernel<T, 32, 1, false>, grid, dim3(kScoreWaves * kWave), stream, la,
-                  w.scores, 0, static_cast<int>(a.n), LimWs{});
+                  w.scores, 0, static_cast<int>(a.n), side);
   } else {
     launch_kernel(kKernLimScore, lim_score_kernel<T, 64, 1, false>, grid, dim3(kScoreWaves * kWave), stream, la,
-                  w.scores, 0, static_cast<int>(a.n), LimWs{});
+                  w.scores, 0, static_cast<int>(a.n), side);
   }
   return hipGetLastError();
 }
@@ -2579,7 +2608,9 @@ size_t lim_workspace_bytes(int64_t batch, int64_t source_capacity, int queries) 
 }
 
 size_t lidu_init_workspace_bytes(int64_t source_capacity) {
-  return align256(sizeof(float) * source_capacity) + 2 * align256(sizeof(int32_t) * kSlotStride) + 256;
+  size_t bytes = 0;
+  (void)init_layout(nullptr, source_capacity, &bytes);
+  return bytes;
 }
 
 int64_t lidu_list_capacity() { return kSlotStride; }
@@ -2590,14 +2621,12 @@ hipError_t launch_lidu_init(const LiduInitArgs& a, hipStream_t stream) {
   if (e != hipSuccess) return e;
   const float* s = static_cast<const float*>(w.scores);
   const int n = static_cast<int>(a.n), c = static_cast<int>(a.c);
-  // Sources of up to one group (32768 tokens) keep their keys in registers
-  // (64 per thread; at 128 the compiler moved the array to scratch memory).
-  if (a.n <= kInitGroup * kChunk)
-    launch_kernel(kKernLiduInit, lidu_init_reg_kernel, dim3(1), dim3(kManageThreads), stream, s, n, c, a.pool_row,
-                  a.row_len, w);
-  else
-    launch_kernel(kKernLiduInit, lidu_init_kernel, dim3(1), dim3(kManageThreads), stream, s, n, c, a.pool_row,
-                  a.row_len, w);
+  const dim3 chunks(static_cast<uint32_t>(ceil_div(a.n, kChunk))), block(kManageThreads);
+  if (chunks.x > kManageThreads) return hipErrorInvalidValue;  // (the chunk counts are scanned one per thread)
+  launch_kernel(kKernLimHist, lidu_hist_kernel, chunks, block, stream, s, n, w);
+  launch_kernel(kKernLimChunks, lidu_chunks_kernel, chunks, block, stream, s, n, c, w);
+  launch_kernel(kKernLiduInit, lidu_init_kernel, dim3(static_cast<uint32_t>(ceil_div(a.row_len, kChunk))), block, stream,
+                s, n, c, a.pool_row, a.row_len, w);
   return hipGetLastError();
 }
 

@@ -245,6 +245,40 @@ def test_gpu_initialize_lidu_row_matches_oracle(seed, n_blocks, c, heads, dtype,
     assert np.array_equal(bits(g["hbm_kpe"]), hkpe)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_blocks,c,extra,ties", [
+    (16, 2048, 0, 0),       # everything selected
+    (32, 2049, 7, 0),       # one whole chunk, a row that ends inside the next one
+    (33, 4096, 4095, 0),    # a chunk of one block
+    (97, 2048, 4100, 90),   # in-bin tokens in several chunks, a chunk past the source
+    (160, 8192, 1, 500),    # ties that fill the lists
+    (160, 2500, 3, 700),    # more ties than the lists hold: the streamed select
+])
+def test_gpu_initialize_lidu_row_chunk_edges(n_blocks, c, extra, ties):
+    """Chunk and list edges of the first-decode selection: sources and pool
+    rows that end inside chunks, threshold ties spread over the source."""
+    from nanovllm_amd import dsa_offload_ops as ops
+
+    case = _init_case(n_blocks, n_blocks, c, 32, "bf16", True)
+    n = case["n"]
+    if ties:  # `ties` tokens around the C-th largest share its key row
+        keys = case["keys"].reshape(-1, 128)
+        rng = np.random.default_rng(n_blocks)
+        rows = lambda t: case["table"][t // 128] * 128 + t % 128  # noqa: E731
+        same = rng.choice(np.arange(n - c - ties, n - c + ties // 2), ties, replace=False)
+        keys[rows(same)] = keys[rows(np.array([n - c]))]
+    row = np.full(n + extra, -5, np.int32)
+    case = dict(case, slots=row)
+    print(f"LIDU-INIT edges n={n} c={c} row={row.size} ties={ties}", flush=True)
+    slots, hkpe, hckv = _oracle_init(case)
+    g = _to_gpu(case)
+    ops.initialize_lidu_row(candidate_len=n, cache_tokens=c, block_size=128, **g)
+    torch.cuda.synchronize()
+    assert np.array_equal(ints(g["cache_slots_row"]), slots)
+    assert np.array_equal(bits(g["hbm_ckv"]), hckv)
+    assert np.array_equal(bits(g["hbm_kpe"]), hkpe)
+
+
 def _unaligned(t: torch.Tensor) -> torch.Tensor:
     """A copy of 1-D ``t`` whose data starts 4 bytes into an allocation (not
     16-byte aligned), so the kernels take their element-wise path."""
