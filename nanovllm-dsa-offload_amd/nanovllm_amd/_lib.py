@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from pathlib import Path
 
 import torch  # noqa: F401  -- must precede the CDLL load (shared HIP runtime)
@@ -107,6 +108,22 @@ def _load() -> ctypes.CDLL:
 
 lib = _load()
 
+
+class _PackedCalls:
+    """The entry points taking descriptors as plain addresses (from
+    :func:`pack`) instead of pointers to ctypes structures."""
+
+    def __init__(self) -> None:
+        for name, (argtypes, restype) in {**SIGNATURES, **EXT_SIGNATURES}.items():
+            if _P in argtypes:
+                fn = lib[name]  # a function object of its own
+                fn.argtypes = [_VP if a is _P else a for a in argtypes]
+                fn.restype = restype
+                setattr(self, name, fn)
+
+
+packed = _PackedCalls()
+
 _DTYPE_CODES = {
     torch.int32: INT32,
     torch.float16: FLOAT16,
@@ -132,6 +149,47 @@ def describe(t: torch.Tensor) -> NvdsaTensor:
     else:
         d.device = _NOT_DEVICE
     return d
+
+
+# Packed descriptors: NvdsaTensor's layout, the zeros that fill a shape to four
+# entries, and the descriptor arrays by length.
+_ITEM = "Qii4qii"
+_ITEM_BYTES = ctypes.sizeof(NvdsaTensor)
+assert struct.calcsize("=" + _ITEM) == _ITEM_BYTES
+_FILL = ((0, 0, 0, 0), (0, 0, 0), (0, 0), (0,), (), ())
+_NO_TENSOR = (0,) * 9
+_MAX_PACKED = 24
+_PACKERS = tuple((struct.Struct("=" + _ITEM * k), ctypes.c_char * (_ITEM_BYTES * k)) for k in range(_MAX_PACKED + 1))
+
+
+def pack(*tensors: torch.Tensor | None):
+    """The tensors' descriptors in one buffer: (buffer, addresses), None for a
+    None.  The same fields as :func:`describe`, which builds a ctypes structure
+    per tensor, at a third of its host time (a fused step describes 27
+    tensors); the buffer has to outlive the call that reads it."""
+    values: list[int] = []
+    for t in tensors:
+        if t is None:
+            values += _NO_TENSOR
+            continue
+        shape = t.shape
+        n = len(shape)
+        if n > 4:
+            n, shape = 5, shape[:4]
+        values += (t.data_ptr(), _DTYPE_CODES.get(t.dtype, -1), n, *shape, *_FILL[n], t.is_contiguous(),
+                   t.get_device() if t.is_cuda else _host_device(t))
+    packer, buffer_type = _PACKERS[len(tensors)]
+    buf = buffer_type()
+    packer.pack_into(buf, 0, *values)
+    base = ctypes.addressof(buf)
+    at = [base + i * _ITEM_BYTES for i in range(len(tensors))]
+    if any(t is None for t in tensors):
+        at = [None if t is None else p for t, p in zip(tensors, at)]
+    return buf, at
+
+
+def _host_device(t: torch.Tensor) -> int:
+    return HOST_MAPPED_DEVICE if t.device.type == "cpu" and _is_pinned(t) else _NOT_DEVICE
 
 
 def _is_pinned(t: torch.Tensor) -> bool:

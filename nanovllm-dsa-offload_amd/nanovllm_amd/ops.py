@@ -24,7 +24,6 @@ or pinned CPU tensors; the GPU reads them over the host link.
 
 from __future__ import annotations
 
-import ctypes
 import struct
 
 import torch
@@ -100,12 +99,9 @@ SCHEMAS = {
     ),
 }
 
-_D = _lib.describe
 _L = _lib.lib
-
-
-def _ref(d: _lib.NvdsaTensor):
-    return ctypes.byref(d)
+_C = _lib.packed
+_pack = _lib.pack
 
 
 def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
@@ -121,125 +117,116 @@ def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_of(t: torch.Tensor) -> int:
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _fused_li_manage(query, index_weights, index_key_cache, index_block_table, num_candidate_tokens,
                      num_cache_tokens, req_pool_entries, cache_slots_pool, topk_src_ids, topk_dst_slots,
                      miss_counts) -> None:
-    descs = [_D(t) for t in (query, index_weights, index_key_cache, index_block_table, num_candidate_tokens,
-                             num_cache_tokens, req_pool_entries, cache_slots_pool, topk_src_ids, topk_dst_slots,
-                             miss_counts)]
+    buf, at = _pack(query, index_weights, index_key_cache, index_block_table, num_candidate_tokens,
+                    num_cache_tokens, req_pool_entries, cache_slots_pool, topk_src_ids, topk_dst_slots, miss_counts)
     nbytes = _L.nvdsa_fused_li_manage_workspace_size(query.shape[0] if query.dim() else 0,
                                                      index_block_table.shape[-1] * 128 if index_block_table.dim() == 2 else 0,
                                                      query.shape[1] if query.dim() > 1 else 0)
     ws = _workspace(query.device, nbytes)
-    _lib.check(_L.nvdsa_fused_li_manage(*map(_ref, descs), ws.data_ptr(), ws.numel(), _stream_of(query)))
+    _lib.check(_C.nvdsa_fused_li_manage(*at, ws.data_ptr(), ws.numel(), _stream_of(query)))
 
 
 def _fused_li_manage_mtp(query, index_weights, index_key_cache, index_block_table, num_candidate_tokens,
                          num_cache_tokens, req_pool_entries, cache_slots_pool, topk_src_ids, topk_dst_slots,
                          miss_src_ids, miss_dst_slots, miss_counts) -> None:
-    descs = [_D(t) for t in (query, index_weights, index_key_cache, index_block_table, num_candidate_tokens,
-                             num_cache_tokens, req_pool_entries, cache_slots_pool, topk_src_ids, topk_dst_slots,
-                             miss_src_ids, miss_dst_slots, miss_counts)]
+    buf, at = _pack(query, index_weights, index_key_cache, index_block_table, num_candidate_tokens,
+                    num_cache_tokens, req_pool_entries, cache_slots_pool, topk_src_ids, topk_dst_slots,
+                    miss_src_ids, miss_dst_slots, miss_counts)
     batch = req_pool_entries.shape[0] if req_pool_entries.dim() == 1 else 0
     nbytes = _L.nvdsa_fused_li_manage_mtp_workspace_size(
         batch, index_block_table.shape[-1] * 128 if index_block_table.dim() == 2 else 0,
         query.shape[1] if query.dim() > 1 else 0)
     ws = _workspace(query.device, nbytes)
-    _lib.check(_L.nvdsa_fused_li_manage_mtp(*map(_ref, descs), ws.data_ptr(), ws.numel(), _stream_of(query)))
+    _lib.check(_C.nvdsa_fused_li_manage_mtp(*at, ws.data_ptr(), ws.numel(), _stream_of(query)))
 
 
 def _scatter_copy(src_ids, dst_slots, copy_counts, hbm_block_table, dram_block_table, hbm_k_rope, hbm_kv_cache,
                   dram_k_rope, dram_kv_cache) -> None:
-    descs = [_D(t) for t in (src_ids, dst_slots, copy_counts, hbm_block_table, dram_block_table, hbm_k_rope,
-                             hbm_kv_cache, dram_k_rope, dram_kv_cache)]
-    _lib.check(_L.nvdsa_scatter_copy(*map(_ref, descs), _stream_of(hbm_kv_cache)))
+    buf, at = _pack(src_ids, dst_slots, copy_counts, hbm_block_table, dram_block_table, hbm_k_rope, hbm_kv_cache,
+                    dram_k_rope, dram_kv_cache)
+    _lib.check(_C.nvdsa_scatter_copy(*at, _stream_of(hbm_kv_cache)))
 
 
-def _attention_workspace(query: torch.Tensor) -> torch.Tensor:
+def _attend(entry, query, scale_value, *tensors) -> None:
+    """One of the attention entry points: its tensors in schema order, the
+    scale, then the output (the last of ``tensors``)."""
+    buf, at = _pack(*tensors)
     rows = query.shape[0] if query.dim() == 3 else 0
     heads = query.shape[1] if query.dim() == 3 else 0
-    nbytes = _L.nvdsa_sparse_tail_attention_workspace_size(rows, heads, 0)
-    return _workspace(query.device, nbytes)
+    ws = _workspace(query.device, _L.nvdsa_sparse_tail_attention_workspace_size(rows, heads, 0))
+    _lib.check(entry(*at[:-1], float(scale_value), at[-1], ws.data_ptr(), ws.numel(), _stream_of(query)))
 
 
 def _sparse_tail_attention(query_rope, query, actual_seq_lengths_query, actual_seq_lengths_kv, num_cache_tokens,
                            topk_dst_slots, hbm_block_table, hbm_k_rope, hbm_kv_cache, scale_value,
                            attention_out) -> None:
-    descs = [_D(t) for t in (query_rope, query, actual_seq_lengths_query, actual_seq_lengths_kv, num_cache_tokens,
-                             topk_dst_slots, hbm_block_table, hbm_k_rope, hbm_kv_cache)]
-    out = _D(attention_out)
-    ws = _attention_workspace(query)
-    _lib.check(_L.nvdsa_sparse_tail_attention(*map(_ref, descs), float(scale_value), _ref(out), ws.data_ptr(),
-                                              ws.numel(), _stream_of(query)))
+    _attend(_C.nvdsa_sparse_tail_attention, query, scale_value, query_rope, query, actual_seq_lengths_query,
+            actual_seq_lengths_kv, num_cache_tokens, topk_dst_slots, hbm_block_table, hbm_k_rope, hbm_kv_cache,
+            attention_out)
 
 
 def _sparse_tail_attention_mtp(query_rope, query, actual_seq_lengths_query, actual_seq_lengths_kv,
                                num_cache_tokens, topk_dst_slots, hbm_block_table, hbm_k_rope, hbm_kv_cache,
                                scale_value, attention_out) -> None:
-    descs = [_D(t) for t in (query_rope, query, actual_seq_lengths_query, actual_seq_lengths_kv, num_cache_tokens,
-                             topk_dst_slots, hbm_block_table, hbm_k_rope, hbm_kv_cache)]
-    out = _D(attention_out)
-    ws = _attention_workspace(query)
-    _lib.check(_L.nvdsa_sparse_tail_attention_mtp(*map(_ref, descs), float(scale_value), _ref(out), ws.data_ptr(),
-                                                  ws.numel(), _stream_of(query)))
+    _attend(_C.nvdsa_sparse_tail_attention_mtp, query, scale_value, query_rope, query, actual_seq_lengths_query,
+            actual_seq_lengths_kv, num_cache_tokens, topk_dst_slots, hbm_block_table, hbm_k_rope, hbm_kv_cache,
+            attention_out)
 
 
 def _fused_copy_sfa(query_rope, query, actual_seq_lengths_query, actual_seq_lengths_kv, num_cache_tokens,
                     topk_dst_slots, topk_src_ids, miss_counts, hbm_block_table, dram_block_table, hbm_k_rope,
                     hbm_kv_cache, dram_k_rope, dram_kv_cache, scale_value, attention_out) -> None:
-    descs = [_D(t) for t in (query_rope, query, actual_seq_lengths_query, actual_seq_lengths_kv, num_cache_tokens,
-                             topk_dst_slots, topk_src_ids, miss_counts, hbm_block_table, dram_block_table,
-                             hbm_k_rope, hbm_kv_cache, dram_k_rope, dram_kv_cache)]
-    out = _D(attention_out)
-    ws = _attention_workspace(query)
-    _lib.check(_L.nvdsa_fused_copy_sfa(*map(_ref, descs), float(scale_value), _ref(out), ws.data_ptr(),
-                                       ws.numel(), _stream_of(query)))
+    _attend(_C.nvdsa_fused_copy_sfa, query, scale_value, query_rope, query, actual_seq_lengths_query,
+            actual_seq_lengths_kv, num_cache_tokens, topk_dst_slots, topk_src_ids, miss_counts, hbm_block_table,
+            dram_block_table, hbm_k_rope, hbm_kv_cache, dram_k_rope, dram_kv_cache, attention_out)
 
 
 def _fused_copy_sfa_mtp(query_rope, query, actual_seq_lengths_query, actual_seq_lengths_kv, num_cache_tokens,
                         topk_dst_slots, topk_src_ids, miss_src_ids, miss_dst_slots, miss_counts, hbm_block_table,
                         dram_block_table, hbm_k_rope, hbm_kv_cache, dram_k_rope, dram_kv_cache, scale_value,
                         attention_out) -> None:
-    descs = [_D(t) for t in (query_rope, query, actual_seq_lengths_query, actual_seq_lengths_kv, num_cache_tokens,
-                             topk_dst_slots, topk_src_ids, miss_src_ids, miss_dst_slots, miss_counts,
-                             hbm_block_table, dram_block_table, hbm_k_rope, hbm_kv_cache, dram_k_rope,
-                             dram_kv_cache)]
-    out = _D(attention_out)
-    ws = _attention_workspace(query)
-    _lib.check(_L.nvdsa_fused_copy_sfa_mtp(*map(_ref, descs), float(scale_value), _ref(out), ws.data_ptr(),
-                                           ws.numel(), _stream_of(query)))
+    _attend(_C.nvdsa_fused_copy_sfa_mtp, query, scale_value, query_rope, query, actual_seq_lengths_query,
+            actual_seq_lengths_kv, num_cache_tokens, topk_dst_slots, topk_src_ids, miss_src_ids, miss_dst_slots,
+            miss_counts, hbm_block_table, dram_block_table, hbm_k_rope, hbm_kv_cache, dram_k_rope, dram_kv_cache,
+            attention_out)
 
 
 def lidu_init_row(query, weights, index_cache, index_block_table, candidate_len, cache_tokens, cache_slots_row,
                   hbm_kpe, hbm_ckv, dram_kpe, dram_ckv, hbm_block_table, dram_block_table, block_size) -> None:
     """nvdsa_initialize_lidu_row on the current stream (no host sync)."""
-    descs = [_D(t) for t in (query, weights, index_cache, index_block_table)]
-    rest = [_D(t) for t in (cache_slots_row, hbm_kpe, hbm_ckv, dram_kpe, dram_ckv, hbm_block_table,
-                            dram_block_table)]
+    buf, at = _pack(query, weights, index_cache, index_block_table, cache_slots_row, hbm_kpe, hbm_ckv, dram_kpe,
+                    dram_ckv, hbm_block_table, dram_block_table)
     nbytes = _L.nvdsa_initialize_lidu_row_workspace_size(cache_slots_row.shape[0] if cache_slots_row.dim() else 0)
     ws = _workspace(query.device, nbytes)
-    _lib.check(_L.nvdsa_initialize_lidu_row(*map(_ref, descs), int(candidate_len), int(cache_tokens),
-                                            *map(_ref, rest), int(block_size), ws.data_ptr(), ws.numel(),
-                                            _stream_of(query)))
+    _lib.check(_C.nvdsa_initialize_lidu_row(*at[:4], int(candidate_len), int(cache_tokens), *at[4:], int(block_size),
+                                            ws.data_ptr(), ws.numel(), _stream_of(query)))
 
 
 def lidu_init_row_shared(cache_slots_row, cache_tokens, hbm_kpe, hbm_ckv, dram_kpe, dram_ckv, hbm_block_table,
                          dram_block_table) -> None:
     """nvdsa_initialize_lidu_row_shared (synchronises the current stream once)."""
-    descs = [_D(t) for t in (hbm_kpe, hbm_ckv, dram_kpe, dram_ckv, hbm_block_table, dram_block_table)]
+    buf, at = _pack(cache_slots_row, hbm_kpe, hbm_ckv, dram_kpe, dram_ckv, hbm_block_table, dram_block_table)
     nbytes = _L.nvdsa_initialize_lidu_row_workspace_size(cache_slots_row.shape[0] if cache_slots_row.dim() else 0)
     ws = _workspace(hbm_kpe.device, nbytes)
-    _lib.check(_L.nvdsa_initialize_lidu_row_shared(_ref(_D(cache_slots_row)), int(cache_tokens), *map(_ref, descs),
-                                                   ws.data_ptr(), ws.numel(), _stream_of(hbm_kpe)))
+    _lib.check(_C.nvdsa_initialize_lidu_row_shared(at[0], int(cache_tokens), *at[1:], ws.data_ptr(), ws.numel(),
+                                                   _stream_of(hbm_kpe)))
 
 
 def _dsa_indexer_query_rope_inplace(q_inout, cos, sin, rope_dim) -> None:
-    descs = [_D(t) for t in (q_inout, cos, sin)]
-    _lib.check(_L.nvdsa_dsa_indexer_query_rope_inplace(*map(_ref, descs), int(rope_dim), _stream_of(q_inout)))
+    buf, at = _pack(q_inout, cos, sin)
+    _lib.check(_C.nvdsa_dsa_indexer_query_rope_inplace(*at, int(rope_dim), _stream_of(q_inout)))
 
 
 def indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, weights_proj_weight, q_index_out,
@@ -247,13 +234,9 @@ def indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, weight
     """nvdsa_dsa_indexer_project_query_only on the current stream.  Pass
     ``weights_proj_weight`` and ``index_weights_out`` as None to project q
     only."""
-    descs = [_D(t) for t in (hidden_states, q_c, cos, sin, wq_b_weight)]
-    wp = _D(weights_proj_weight) if weights_proj_weight is not None else None
-    qo = _D(q_index_out)
-    wo = _D(index_weights_out) if index_weights_out is not None else None
-    _lib.check(_L.nvdsa_dsa_indexer_project_query_only(
-        *map(_ref, descs), _ref(wp) if wp is not None else None, _ref(qo), _ref(wo) if wo is not None else None,
-        int(n_head), int(head_dim), int(rope_dim), float(score_scale), _stream_of(q_c)))
+    buf, at = _pack(hidden_states, q_c, cos, sin, wq_b_weight, weights_proj_weight, q_index_out, index_weights_out)
+    _lib.check(_C.nvdsa_dsa_indexer_project_query_only(*at, int(n_head), int(head_dim), int(rope_dim),
+                                                       float(score_scale), _stream_of(q_c)))
 
 
 def indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias, weights_proj_weight, index_k_out,
@@ -262,13 +245,12 @@ def indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm
     the head weights of many tokens.  Pass the key's tensors (cos, sin,
     wk_weight, k_norm_weight, k_norm_bias, index_k_out) as None to compute
     the head weights only."""
-    descs = [_D(t) if t is not None else None for t in (hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias,
-                                                         weights_proj_weight, index_k_out, index_weights_out)]
+    buf, at = _pack(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias, weights_proj_weight, index_k_out,
+                    index_weights_out)
     nbytes = _L.nvdsa_dsa_indexer_project_kw_workspace_size(hidden_states.shape[0], weights_proj_weight.shape[0],
                                                             hidden_states.shape[1], int(wk_weight is not None))
     ws = _workspace(hidden_states.device, nbytes)
-    _lib.check(_L.nvdsa_dsa_indexer_project_kw(*(None if d is None else _ref(d) for d in descs), int(rope_dim),
-                                               float(score_scale), ws.data_ptr(), ws.numel(),
+    _lib.check(_C.nvdsa_dsa_indexer_project_kw(*at, int(rope_dim), float(score_scale), ws.data_ptr(), ws.numel(),
                                                _stream_of(hidden_states)))
 
 
@@ -283,8 +265,8 @@ def stage_inputs(fields: list[int], like: torch.Tensor) -> None:
 def persist_prefill_blocks(hbm_kv_cache, hbm_k_rope, dram_kv_cache, dram_k_rope, hbm_block_ids,
                            dram_block_ids) -> None:
     """nvdsa_persist_prefill_blocks on the current stream (no host sync)."""
-    descs = [_D(t) for t in (hbm_kv_cache, hbm_k_rope, dram_kv_cache, dram_k_rope, hbm_block_ids, dram_block_ids)]
-    _lib.check(_L.nvdsa_persist_prefill_blocks(*map(_ref, descs), _stream_of(hbm_kv_cache)))
+    buf, at = _pack(hbm_kv_cache, hbm_k_rope, dram_kv_cache, dram_k_rope, hbm_block_ids, dram_block_ids)
+    _lib.check(_C.nvdsa_persist_prefill_blocks(*at, _stream_of(hbm_kv_cache)))
 
 
 IMPLS = {
