@@ -210,7 +210,10 @@ __global__ __launch_bounds__(kProjThreads) void indexer_project_kernel(IndexerAr
 // K steps of 64 (128-byte rows of eight 16-byte chunks, chunk c of row r kept
 // at c ^ (r & 7): the operand reads of eight consecutive rows touch all
 // banks), two buffers: the next step's loads are issued before this step's
-// MFMAs and stored after them, one barrier per step.  Wave tiles are
+// MFMAs and stored after them, one barrier per step.  At 4096 tokens a step of
+// a 256 x 256 tile takes 1.7 us (4.1k cycles, half of them MFMA): its 64 KB
+// arrive at the ~16 bytes per clock that one CU pulls, whatever the order of
+// loads, stores and MFMAs in it (five orders within 3%).  Wave tiles are
 // TOK/WT x OUT/WO of 32x32x16 MFMAs, the weight rows as the A operand, so a
 // lane holds runs of four consecutive outputs of one token (the rotation's
 // pairs).  The rotated 16-bit tile is turned through LDS and stored in whole
@@ -358,33 +361,60 @@ __global__ __launch_bounds__(64 * WT * WO) void indexer_project_gemm_kernel(Inde
   // Then rotated and stored by 16-byte chunks (eight outputs of one token,
   // within one head).  A rolled loop: unrolled over the accumulators the
   // rotation is tens of KB of straight-line code, and fetching it cost more
-  // than running it (a 256 x 256 tile's epilogue 30 us, 16 us of it after the
-  // cheaper conversion; now a few).
+  // than running it (30 us of a launch of 256 x 256 tiles).
   constexpr int kRowChunks = OUT / 8;
   const int head_dim = static_cast<int>(a.head_dim), rope = static_cast<int>(a.rope_dim);
   const int64_t row_elems = a.heads * a.head_dim;
-  for (int c = tid; c < TOK * kRowChunks; c += S::kThreads) {
-    const int r = c / kRowChunks, ch = c % kRowChunks;
-    const int64_t t = tok0 + r;
-    if (t >= ntok) break;  // (r does not decrease along the loop)
-    u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[r * S::kOutStride + ch * 8]);
-    const int d = (out0 + ch * 8) % head_dim;
-    if (d < rope) {
-      const uint32_t* cp = reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.cos) + t * a.cos_stride + d);
-      const uint32_t* sp = reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.sin) + t * a.cos_stride + d);
+  // Batches of kBatch chunks per thread, every cos and sin load of a batch in
+  // flight together, 16 bytes each where the rows allow it (one chunk at a
+  // time the loop is a chain of round trips: 7 of 76 us at 4096 tokens).
+  constexpr int kIters = TOK * kRowChunks / S::kThreads;
+  constexpr int kBatch = kIters < 4 ? kIters : 4;
+  static_assert(TOK * kRowChunks % S::kThreads == 0 && kIters % kBatch == 0, "epilogue tiling");
+  const bool vec = (a.cos_stride & 7) == 0 && ((reinterpret_cast<uintptr_t>(a.cos) | reinterpret_cast<uintptr_t>(a.sin)) & 15) == 0;
+#pragma unroll 1
+  for (int c0 = 0; c0 < kIters; c0 += kBatch) {
+    u32x4_t v[kBatch], cv[kBatch], sv[kBatch];
+    int64_t t[kBatch];
+    int d[kBatch];
+    const int ch = tid % kRowChunks;  // (kThreads is a multiple of kRowChunks: the same chunk of every row)
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int r = ((c0 + i) * S::kThreads + tid) / kRowChunks;
+      t[i] = tok0 + r;
+      d[i] = (out0 + ch * 8) % head_dim;
+      v[i] = *reinterpret_cast<const u32x4_t*>(&lds[r * S::kOutStride + ch * 8]);
+      const int64_t at = min<int64_t>(t[i], ntok - 1) * a.cos_stride + d[i];
+      const uint16_t* cp = static_cast<const uint16_t*>(a.cos) + at;
+      const uint16_t* sp = static_cast<const uint16_t*>(a.sin) + at;
+      if (vec && d[i] + 8 <= rope) {
+        cv[i] = *reinterpret_cast<const u32x4_t*>(cp);
+        sv[i] = *reinterpret_cast<const u32x4_t*>(sp);
+      } else {
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          if (d[i] + 2 * h < rope) {
+            cv[i][h] = reinterpret_cast<const uint32_t*>(cp)[h];
+            sv[i][h] = reinterpret_cast<const uint32_t*>(sp)[h];
+          }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
 #pragma unroll
       for (int h = 0; h < 4; ++h) {
-        if (d + 2 * h < rope) {
-          const uint32_t x2 = v[h], c2 = cp[h], s2 = sp[h];
+        if (d[i] + 2 * h < rope) {
+          const uint32_t x2 = v[i][h], c2 = cv[i][h], s2 = sv[i][h];
           float y0, y1;
           rope_pair(T::to_float(static_cast<uint16_t>(x2)), T::to_float(static_cast<uint16_t>(x2 >> 16)),
                     T::to_float(static_cast<uint16_t>(c2)), T::to_float(static_cast<uint16_t>(c2 >> 16)),
                     T::to_float(static_cast<uint16_t>(s2)), T::to_float(static_cast<uint16_t>(s2 >> 16)), y0, y1);
-          v[h] = T::pack2(y0, y1);
+          v[i][h] = T::pack2(y0, y1);
         }
       }
+      if (t[i] < ntok)
+        *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(a.q_out) + t[i] * row_elems + out0 + ch * 8) = v[i];
     }
-    *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(a.q_out) + t * row_elems + out0 + ch * 8) = v;
   }
 }
 
@@ -712,22 +742,22 @@ hipError_t launch_project(const IndexerArgs& a, hipStream_t stream) {
     // More than one 64-token group: the tiled GEMM (n_head and head_dim are
     // multiples of 16, so its output tiles divide the rows of wq_b).  Its
     // tile by the time each would take, measured at 4096 outputs of K 2048: a
-    // launch's 64 x 64 tiles fill the chip's 256 CUs at 14 us and then cost
-    // 27.5 ns each, 128 x 128 ones 32 us and 93 ns, 256 x 256 ones 76 us per
+    // launch's 64 x 64 tiles fill the chip's 256 CUs at 13 us and then cost
+    // 26.5 ns each, 128 x 128 ones 29.5 us and 75 ns, 256 x 256 ones 69 us per
     // round of 256.  64-token groups / 64 / 128 / 256 tiles: 65 tokens 15.8 /
-    // 14.2 / 32 / 60 us, 512: 89 / 22 / 34 / 66, 1024: 174 / 35 / 32 / 65,
-    // 4096: 675 / 132 / 99 / 76 us.
+    // 12.2 / 26 / 56 us, 512: 89 / 22 / 33 / 60, 1024: 174 / 34 / 29.5 / 59,
+    // 2048: 339 / 63 / 46 / 60, 4096: 675 / 120 / 85 / 69 us.
     const int64_t outs = a.heads * a.head_dim;
     const int64_t n64 = ceil_div(a.tokens, 64) * (outs / 64), n128 = ceil_div(a.tokens, 128) * (outs / 128);
     const int64_t n256 = ceil_div(a.tokens, 256) * (outs / 256);
-    const double us64 = std::max(14.0, 7.0 + 0.0275 * n64), us128 = std::max(32.0, 8.0 + 0.09 * n128);
-    const double us256 = 76.0 * ceil_div(n256, 256);
+    const double us64 = std::max(13.0, 7.0 + 0.0265 * n64), us128 = std::max(29.5, 8.0 + 0.075 * n128);
+    const double us256 = 69.0 * ceil_div(n256, 256);
     if (us64 <= us128 && us64 <= us256)
       launch_gemm_shape<T, 64, 64, 2, 2>(a, stream);
     else if (us128 <= us256)
       launch_gemm_shape<T, 128, 128, 2, 2>(a, stream);
     else
-      launch_gemm_shape<T, 256, 256, 4, 2>(a, stream);
+      launch_gemm_shape<T, 256, 256, 2, 4>(a, stream);
     return hipGetLastError();
   }
   const dim3 grid(static_cast<uint32_t>(q_tiles), static_cast<uint32_t>(ceil_div(a.tokens, kTokPerGroup)));
