@@ -418,8 +418,8 @@ __device__ __forceinline__ SelectOut radix_select_visit(int k, uint32_t kmin, ui
     __syncthreads();
     // Thread tid owns bins [tb*kBinsPerThread, +kBinsPerThread), threads in
     // descending bin order; find the bin holding the remaining-th largest.
-    // (The thread that holds it reads its bins again: kept in registers across
-    // the scan they are 16 more for every caller.)
+    // (The thread that holds it reads its bins again, four at a time: kept in
+    // registers across the scan they are 16 more for every caller.)
     const int tb = kManageThreads - 1 - tid;
     uint32_t* own = hist + tb * kBinsPerThread;
     int sum = 0;
@@ -429,14 +429,19 @@ __device__ __forceinline__ SelectOut radix_select_visit(int k, uint32_t kmin, ui
     int acc = block_exclusive_scan(sum, scratch, &total);
     if (acc < remaining && remaining <= acc + sum) {
 #pragma unroll 1
-      for (int j = kBinsPerThread - 1; j >= 0; --j) {
-        const int cnt = static_cast<int>(own[j]);
-        if (acc < remaining && remaining <= acc + cnt) {
-          bcast[0] = tb * kBinsPerThread + j;
-          bcast[1] = acc;
-          bcast[2] = cnt;
+      for (int j = kBinsPerThread - 4; j >= 0; j -= 4) {
+        const uint4 c4 = *reinterpret_cast<const uint4*>(own + j);
+        const uint32_t cnt[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+        for (int e = 3; e >= 0; --e) {
+          const int n = static_cast<int>(cnt[e]);
+          if (acc < remaining && remaining <= acc + n) {
+            bcast[0] = tb * kBinsPerThread + j + e;
+            bcast[1] = acc;
+            bcast[2] = n;
+          }
+          acc += n;
         }
-        acc += cnt;
       }
     }
 #pragma unroll
@@ -1007,11 +1012,14 @@ __device__ __forceinline__ SelectOut row_threshold(const float* s, int n, int64_
 }
 
 // Top-2048 threshold of one (request, query) score row, written to the
-// workspace for the MTP3 management kernels.  One workgroup per row; RES > 0
-// keeps the row's keys in registers (RES chunks of 4096 tokens).
-template <int RES>
-__global__ __launch_bounds__(kManageThreads) void lim_threshold_kernel(LimArgs a, LimWs w, int queries, int min_n) {
-  __shared__ uint32_t hist[kBins + kWave];  // (+ the bins that keys past n count into)
+// workspace for the MTP3 management kernels.  One workgroup per row, which
+// keeps its keys in registers (kThresholdChunks chunks of 4096 tokens) or, if
+// it is longer, reads it on every pass.  The row's own length decides, not the
+// tables' width: 40960 tokens on tables of 131072 take the same 22 us as on
+// 65536 (33 us when every row of a wider table was streamed).
+constexpr int kThresholdChunks = 16;
+__global__ __launch_bounds__(kManageThreads) void lim_threshold_kernel(LimArgs a, LimWs w, int queries) {
+  __shared__ __align__(16) uint32_t hist[kBins + kWave];  // (+ the bins that keys past n count into)
   __shared__ int scratch[kManageThreads / 64 + 1];
   __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
   __shared__ int bcast[4];
@@ -1023,11 +1031,13 @@ __global__ __launch_bounds__(kManageThreads) void lim_threshold_kernel(LimArgs a
   const int r = a.pool_entries[b];
   const bool valid = queries > 1 ? lim_mtp_row_valid(n, c, r, a.source_capacity, a.pool_rows)
                                  : lim_row_valid(n, c, r, a.source_capacity, a.pool_rows);
-  if (!valid || n < min_n) return;
+  if (!valid) return;
   const int64_t cap = a.source_capacity;
   const float* s = w.scores + (static_cast<int64_t>(b) * queries + q) * cap;
   for (int i = tid; i < kBins + kWave; i += kManageThreads) hist[i] = 0u;
-  const SelectOut sel = row_threshold<RES>(s, n, cap, hist, scratch, bcast, red);
+  const SelectOut sel = n <= kThresholdChunks * kChunk  // (uniform)
+                            ? row_threshold<kThresholdChunks>(s, n, cap, hist, scratch, bcast, red)
+                            : row_threshold<0>(s, n, cap, hist, scratch, bcast, red);
   // Ties at the threshold go to the lowest tokens: a token with key ==
   // thresh is selected iff token <= cutoff (INT_MAX when all ties are taken).
   int cutoff = INT_MAX;
@@ -1884,7 +1894,7 @@ __device__ __forceinline__ ChunkSel classify_chunk(const LimArgs& a, const LimWs
 // LDS allows.  Used while every chunk of the launch is resident at once
 // (kResidentChunks); larger launches take lim_chunks_kernel + lim_resolve_kernel.
 __global__ __launch_bounds__(kManageThreads, 4) void lim_classify_kernel(LimArgs a, LimWs w, int parts) {
-  __shared__ uint32_t region[kBins];
+  __shared__ __align__(16) uint32_t region[kBins];
   __shared__ int scratch[kManageThreads / 64 + 1];
   __shared__ uint64_t scratch64[kManageThreads / 64 + 1];
   __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
@@ -1944,7 +1954,7 @@ __global__ __launch_bounds__(kManageThreads) void lim_chunks_kernel(LimArgs a, L
 }
 
 __global__ __launch_bounds__(kManageThreads, 4) void lim_resolve_kernel(LimArgs a, LimWs w, int parts) {
-  __shared__ uint32_t region[kBins];
+  __shared__ __align__(16) uint32_t region[kBins];
   __shared__ int scratch[kManageThreads / 64 + 1];
   __shared__ uint64_t scratch64[kManageThreads / 64 + 1];
   __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
@@ -2074,7 +2084,7 @@ __global__ __launch_bounds__(kManageThreads) void lim_mtp_pass_a_kernel(LimArgs 
 }
 
 __global__ __launch_bounds__(kManageThreads) void lim_mtp_victims_kernel(LimArgs a, LimWs w, int parts) {
-  __shared__ uint32_t hist[kBins];
+  __shared__ __align__(16) uint32_t hist[kBins];
   __shared__ int scratch[kManageThreads / 64 + 1];
   __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
   __shared__ int bcast[4];
@@ -2337,7 +2347,7 @@ __global__ __launch_bounds__(kManageThreads) void lidu_chunks_kernel(const float
 
 __global__ __launch_bounds__(kManageThreads) void lidu_init_kernel(const float* s, int n, int c, int32_t* pool_row,
                                                                    int64_t row_len, InitWs w) {
-  __shared__ uint32_t hist[kBins];  // the ranking lists, or the streamed select's histogram
+  __shared__ __align__(16) uint32_t hist[kBins];  // the ranking lists, or the streamed select's histogram
   __shared__ int scratch[kManageThreads / 64 + 1];
   __shared__ int bcast[4];
   __shared__ int goff[kManageThreads], cim[kManageThreads];
@@ -2587,10 +2597,7 @@ hipError_t launch_lim(const LimArgs& a, hipStream_t stream) {
     return hipGetLastError();
   }
   // MTP3: thresholds first, one workgroup per (request, query) score row.
-  if (a.source_capacity <= 16 * kChunk)
-    launch_kernel(kKernLimThreshold, lim_threshold_kernel<16>, tgrid, mblock, stream, a, w, Q, 0);
-  else
-    launch_kernel(kKernLimThreshold, lim_threshold_kernel<0>, tgrid, mblock, stream, a, w, Q, 0);
+  launch_kernel(kKernLimThreshold, lim_threshold_kernel, tgrid, mblock, stream, a, w, Q);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   launch_kernel(kKernLimMtpPassA, lim_mtp_pass_a_kernel, pgrid, mblock, stream, a, w, parts);

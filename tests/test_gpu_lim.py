@@ -252,6 +252,24 @@ def test_lim_mtp_bit_exact(heads):
     assert np.array_equal(ints(d["cache_slots_pool"]), expect["pool"])
 
 
+def test_lim_mtp_long_and_short_rows_on_wide_tables_bit_exact():
+    """131072-token tables: a row of 65536 candidates (keys in registers, the
+    longest), one block more (read on every pass) and a short one, each by
+    its own length."""
+    from nanovllm_amd.workloads import STRUCTURED_ORDERS, make_chain_case
+
+    orders = [STRUCTURED_ORDERS[k] for k in ("t", "d0", "d1", "d0d2")]
+    case = make_chain_case(3, [65536, 65664, 8320], [8192, 8192, 8192], [5, 9, 4], mtp=True, guard=False, seed=5,
+                           structured_scores=True, structured_orders=orders, source_capacity=131072, fast_fill=True,
+                           attn_heads=4, miss_frac=(0.1, 0.2))
+    print("LIM MTP wide tables", flush=True)
+    expect = oracle_lim(case, mtp=True)
+    assert (expect["miss_counts"][:2] > 0).all()
+    d = case.to_device("cuda", host_mapped=False)
+    _run_lim(d, mtp=True)
+    _assert_matches(d, expect, True)
+
+
 def _tie_case(mtp: bool, positives, seed=11, n_tokens=12288):
     """Scores with exact ties at the top-2048 threshold: query row j of a
     request reads key dim j only, and key dim j is positive for `positives[j]`
