@@ -10,15 +10,18 @@ buffers and ``ValueError`` conditions):
   ``weights_proj_weight`` shares the activations' dtype (the decode graph's
   cached low-precision copy, nanovllm/models/glm_mla.py:262-271) both come
   from one fused gfx950 launch (``nvdsa_dsa_indexer_project_query_only``).
-  Otherwise q comes from that launch and the weights from an fp32 library
-  GEMM then one cast, as the reference computes them (:82-86).
-  ``wq_b_bmm_t`` / ``enable_q_bmm`` are accepted for signature parity; the
-  fused kernel reads ``wq_b_weight`` in its natural [H*D, R] layout, so the
-  transposed BMM copy (an Ascend layout, :102-130) is not used.
+  fp32 weights, and any weights of more than 64 tokens, take a launch of
+  their own (``nvdsa_dsa_indexer_project_kw``: exact products, fp32 sums, one
+  cast, as the reference computes them, :82-86) where the tensors are plain
+  (contiguous, aligned, no gradient asked for), and an fp32 library GEMM
+  otherwise.  ``wq_b_bmm_t`` / ``enable_q_bmm`` are accepted for signature
+  parity; the kernels read ``wq_b_weight`` in its natural [H*D, R] layout, so
+  the transposed BMM copy (an Ascend layout, :102-130) is not used.
 * :func:`dsa_indexer_project` (reference :245-293), the prefill path: q as
-  above, ``index_k = RoPE(LayerNorm(hidden . wk^T))`` and fp32 weights.  The
-  k projection and layer norm are library calls; both RoPEs are the HIP
-  kernel behind ``torch.ops.nanovllm_dsa.dsa_indexer_query_rope_inplace``.
+  above, ``index_k = RoPE(LayerNorm(hidden . wk^T))`` and fp32 weights in one
+  pass over ``hidden_states`` under the same conditions.  Otherwise the k
+  projection and layer norm are library calls and its RoPE the HIP kernel
+  behind ``torch.ops.nanovllm_dsa.dsa_indexer_query_rope_inplace``.
 
 RoPE is the interleaved-pair rotation of the reference's AscendC kernel
 (ops/dsa_indexer_project/op_kernel/dsa_indexer_project_kernel.cpp:105-176):
