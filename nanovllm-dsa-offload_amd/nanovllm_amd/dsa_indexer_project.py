@@ -88,7 +88,8 @@ def _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out,
             and _plain(hidden_states, hidden_states.shape, (dtype,), device)
             and _plain(weights_proj_weight, (n_head, hidden), (dtype, torch.float32), device)
             and _plain(index_weights_out, (hidden_states.shape[0], n_head), (dtype,), device, 2)
-            and not (torch.is_grad_enabled() and (hidden_states.requires_grad or weights_proj_weight.requires_grad)))
+            and not (torch.is_grad_enabled() and (hidden_states.requires_grad or weights_proj_weight.requires_grad
+                                                  or index_weights_out.requires_grad)))
 
 
 # Tokens of one group of the fused decode launch; past it q comes from the
@@ -109,7 +110,9 @@ def dsa_indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, we
     same = weights_proj_weight.dtype == hidden_states.dtype
     # One launch for both up to a group of tokens; more tokens (or fp32 head
     # weights) take the head weights' own kernel where it reads their form.
-    if ((not same or tokens > _GROUP_TOKENS)
+    # (16-bit weights only in the sizes that the one launch takes too).
+    if ((not same or (tokens > _GROUP_TOKENS and hidden_states.shape[-1] % 512 == 0
+                      and index_weights_out.data_ptr() % 4 == 0))
             and _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, n_head)):
         ops.indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, None, q_index_out, None, n_head,
                                        head_dim, rope_dim, score_scale)
@@ -145,7 +148,7 @@ def dsa_indexer_project(hidden_states, q_c, cos, sin, wq_b_weight, wk_weight, k_
             and _plain(wk_weight, (128, hidden_states.shape[1]), (dtype,), device)
             and all(_plain(t, (128,), (dtype,), device, 4) for t in norm)
             and (cos.numel() // tokens) % 2 == 0 and index_k_out.data_ptr() % 4 == 0
-            and not (torch.is_grad_enabled() and any(t.requires_grad for t in (wk_weight, *norm)))):
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in (wk_weight, index_k_out, *norm)))):
         ops.indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias, weights_proj_weight,
                                index_k_out, index_weights_out, int(rope_dim), score_scale)
         return q_index_out, index_k_out, index_weights_out
