@@ -434,7 +434,8 @@ void launch_gemm_shape(const IndexerArgs& a, hipStream_t stream) {
 // runs), through LDS as above.  Everything runs on 32x32x16 16-bit MFMAs.  An
 // fp32 head weight is cut into three bf16 parts by truncation, 8 mantissa bits
 // each, which hold it exactly (an fp16 activation likewise into two), so every
-// product is exact and only the fp32 sums round, as in an fp32 GEMM.  (On the
+// product is exact and only the fp32 sums round, as in an fp32 GEMM; sums that
+// an infinity makes NaN are taken again by the finish kernel.  (On the
 // fp32 MFMA, at 1/16 of the rate, the kernel takes 33 us at 4096 tokens, this
 // form 28.6 us, both 2.0e-3 off fp64 in the rounded outputs; what bounds it
 // now is each CU's pull of 40 KB per K step.)  It replaces two library GEMMs (27 +
@@ -646,16 +647,17 @@ __global__ __launch_bounds__(256) void indexer_kw_finish_kernel(IndexerKwArgs a,
     }
     if (lane < heads) w += p[s * stride + (K ? kKwDim : 0) + lane];
   }
-  if (lane < heads) {
-    uint16_t* out = static_cast<uint16_t*>(a.w_out) + t * heads + lane;
+  const auto store_weight = [&](int head, float v) {
+    uint16_t* out = static_cast<uint16_t*>(a.w_out) + t * heads + head;
     if (a.w_fp32) {
-      *out = T::from_float(w * a.score_scale);
+      *out = T::from_float(v * a.score_scale);
     } else {  // rounded after the projection and again after the scale
-      uint16_t o = T::from_float(w);
+      uint16_t o = T::from_float(v);
       if (a.score_scale != 1.f) o = T::from_float(T::to_float(o) * a.score_scale);
       *out = o;
     }
-  }
+  };
+  if (lane < heads) store_weight(lane, w);
   if constexpr (K) {
     // The projection is rounded to 16 bits, then the layer norm in fp32
     // (eps 1e-6), rounded, then the rotation.
@@ -683,6 +685,24 @@ __global__ __launch_bounds__(256) void indexer_kw_finish_kernel(IndexerKwArgs a,
       o = T::pack2(r0, r1);
     }
     static_cast<uint32_t*>(a.k_out)[t * (kKwDim / 2) + lane] = o;
+  }
+  // An infinite operand times another's zero part is NaN where the product
+  // itself is infinite: a NaN sum is taken again in whole values (a wave per
+  // head; only non-finite operands or overflowing sums come here).  After the
+  // stores: in front of them it cost finite inputs 4 us at 4096 tokens, here none.
+  uint64_t again = __ballot(lane < heads && w != w);
+  while (__builtin_expect(again != 0, 0)) {
+    const int h = __ffsll(static_cast<unsigned long long>(again)) - 1;
+    again &= again - 1;
+    const uint16_t* x = static_cast<const uint16_t*>(a.hidden) + t * a.hid;
+    const int64_t wrow = h * a.hid;
+    float sum = 0.f;
+#pragma unroll 1
+    for (int64_t i = lane; i < a.hid; i += 64)
+      sum += T::to_float(x[i]) * (a.w_fp32 ? static_cast<const float*>(a.w_proj)[wrow + i]
+                                           : T::to_float(static_cast<const uint16_t*>(a.w_proj)[wrow + i]));
+    sum = wave_all_op(sum, AddOp{});
+    if (lane == h) store_weight(h, sum);
   }
 }
 

@@ -319,3 +319,31 @@ def test_project_key_and_weights_kernel(dtype, T, heads, hid, fp32, bias):
     excess = np.abs(g64 - e64) - rel * (2 * mag + 1.41 * 0.95)
     assert np.all(excess <= 0), float(excess.max())
     assert np.mean(gk[1:T + 1] == ek) >= 0.9
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fp32", [True, False])
+def test_project_weights_infinities(dtype, fp32):
+    """Infinite and NaN activations and head weights give the infinities and
+    NaNs of the products themselves (a NaN only where inf * 0, inf - inf or a
+    NaN is summed); the other tokens and heads are those of finite inputs."""
+    from nanovllm_amd import ops
+
+    print(f"PROJECT kw infinities {dtype} fp32={fp32}", flush=True)
+    T, heads, hid = 70, 16, 192
+    rng = np.random.default_rng(5)
+    x = torch.from_numpy(rng.integers(1, 4, (T, hid)).astype(np.float32)).to(dtype)
+    w = torch.from_numpy(rng.integers(1, 4, (heads, hid)).astype(np.float32) / 64)
+    x[3, 7] = float("inf")
+    x[4, 9], x[4, 150] = float("inf"), float("-inf")
+    x[5, 0] = float("nan")
+    w[2, 100] = float("-inf")
+    w[6, 20] = float("nan")
+    w[8, 7] = 0.0
+    w = w if fp32 else w.to(dtype)
+    out = torch.empty(T, heads, dtype=dtype, device="cuda")
+    ops.indexer_project_kw(x.cuda(), None, None, None, None, None, w.cuda(), None, out, ROPE, 1.0)
+    want = (x.double() @ w.double().T).to(dtype)  # (small integers over 64: exact sums, one rounding)
+    assert torch.isinf(want).any() and torch.isnan(want).any()
+    assert torch.equal(out.cpu().isnan(), want.isnan())
+    assert torch.equal(torch.nan_to_num(out.cpu(), nan=1.0), torch.nan_to_num(want, nan=1.0))
