@@ -183,6 +183,8 @@ class DsaLayerGraph:
             self.inputs[name][real:].fill_(pad)
         for name in _TABLES:
             src, dst = runtime[name], self.inputs[name]
+            if src.data_ptr() == dst.data_ptr() and src.stride() != dst.stride():
+                src = src.clone()  # the buffer's own memory in other rows
             dst[:real, :src.shape[1]].copy_(src)
             dst[:real, src.shape[1]:].zero_()
             dst[real:].zero_()
@@ -221,7 +223,10 @@ class DsaLayerGraph:
                 raise ValueError(f"{name} must be rank 2 with {real} rows, got {tuple(shape)}")
             if shape[1] > width:
                 raise ValueError(f"{name} is wider than its graph buffer: runtime={shape[1]}, graph={width}.")
-            plain = plain and self._stageable(name, src) and src.stride(1) == 1
+            # (Rows of the buffer's own memory at another stride would be read
+            # where other rows are written.)
+            plain = (plain and self._stageable(name, src) and src.stride(1) == 1
+                     and (src.data_ptr() != self._address[name] or src.stride(0) == width or real <= 1))
             if plain:
                 staged += (self._address[name], src.data_ptr(), self.batch_size, real, 4 * width, 4 * shape[1],
                            4 * src.stride(0), 0)

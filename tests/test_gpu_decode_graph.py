@@ -155,11 +155,13 @@ def test_many_captured_graphs_keep_their_workspaces():
 
 @pytest.mark.parametrize("mtp", [False, True])
 @pytest.mark.parametrize("batch,real,form", [(1, 1, "plain"), (5, 3, "plain"), (5, 5, "odd"), (4, 2, "strided"),
-                                             (3, 0, "plain"), (6, 4, "host"), (5, 4, "own"), (4, 4, "crossed")])
+                                             (3, 0, "plain"), (6, 4, "host"), (5, 4, "own"), (4, 4, "crossed"),
+                                             (5, 4, "own_rows"), (3, 1, "own_rows")])
 def test_staged_inputs_match_copies(mtp, batch, real, form):
     """The one-launch staging against what torch copies leave: odd batches and
     addresses (2- and 4-byte units), tables that are columns of wider ones,
-    an empty batch, host tensors, a buffer's own memory, another buffer's."""
+    an empty batch, host tensors, a buffer's own memory (a table's also as
+    rows of another width), another buffer's."""
     from nanovllm_amd import decode_graph as G
 
     print(f"STAGE mtp={mtp} batch={batch} real={real} {form}", flush=True)
@@ -189,6 +191,11 @@ def test_staged_inputs_match_copies(mtp, batch, real, form):
     elif form == "own":
         g.inputs["query"].copy_(half(batch * q, heads, 512))
         runtime["query"] = g.inputs["query"][:real * q]
+    elif form == "own_rows":
+        for n, cols in zip(G._TABLES, (9, 4, 5)):
+            whole = g.inputs[n]
+            whole.copy_(ints_(*whole.shape))
+            runtime[n] = whole.view(-1)[:real * cols].view(real, cols)
     elif form == "crossed":
         g.inputs["num_cache_tokens"].copy_(ints_(batch))
         runtime["num_candidate_tokens"] = g.inputs["num_cache_tokens"]
@@ -203,7 +210,7 @@ def test_staged_inputs_match_copies(mtp, batch, real, form):
         expect[n] = torch.zeros_like(g.inputs[n])
         expect[n][:real * q] = runtime[n]
     for n, t in g.inputs.items():  # whatever the last step left
-        if form not in ("own", "crossed"):
+        if form not in ("own", "crossed", "own_rows"):
             t.fill_(77)
     assert g.copy_runtime_inputs(**runtime) == real
     torch.cuda.synchronize()
