@@ -116,6 +116,7 @@ class DsaLayerGraph:
         self._address = {k: self._span[0] + o for k, o in offsets.items()}
         self.inputs = {k: self._block[offsets[k]:offsets[k] + self._nbytes[k]].view(dt).view(shape)
                        for k, (shape, dt) in shapes.items()}
+        self._buffers = dict(self.inputs)  # (a caller may put tensors of its own into `inputs` before the capture)
         for name, pad in _ROW_INPUTS.items():
             self.inputs[name].fill_(pad)
         self.outputs = {
@@ -166,10 +167,14 @@ class DsaLayerGraph:
 
     # -- per-step inputs --------------------------------------------------------
     def _stageable(self, name: str, src: torch.Tensor) -> bool:
-        """Whether the staging kernel may read ``src`` for buffer ``name``: a
-        plain tensor of the buffer's dtype on its device, outside the static
-        inputs' memory or the buffer itself."""
-        if type(src) is not torch.Tensor or src.dtype != self.inputs[name].dtype or src.device != self._device:
+        """Whether the staging kernel may read ``src`` for input ``name``: the
+        input is still this object's buffer, and ``src`` a plain tensor of its
+        dtype on its device, outside the static inputs' memory or the buffer
+        itself."""
+        dst = self.inputs[name]
+        if dst is not self._buffers[name] or dst.data_ptr() != self._address[name]:
+            return False
+        if type(src) is not torch.Tensor or src.dtype != dst.dtype or src.device != self._device:
             return False
         at = src.data_ptr()
         lo, hi = self._span

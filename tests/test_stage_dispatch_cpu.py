@@ -65,3 +65,22 @@ def test_own_table_memory(monkeypatch, name, cols, real, compact):
         assert not _reads_what_it_writes(launches[0])
     else:
         assert torch.equal(whole, expect)
+
+
+@pytest.mark.parametrize("name", ["num_cache_tokens", "dram_block_table", "query"])
+@pytest.mark.parametrize("how", ["entry", "memory"])
+def test_replaced_inputs_get_the_step(monkeypatch, name, how):
+    """An input whose buffer a caller replaced (a tensor of its own in
+    ``inputs``, or other memory under the same tensor) receives the step's
+    data, which the captured step reads there."""
+    g, launches = _graph(monkeypatch)
+    if how == "entry":
+        g.inputs[name] = torch.full_like(g.inputs[name], 7)
+    else:
+        g.inputs[name].data = torch.full_like(g.inputs[name], 7)
+    runtime = _runtime(g, 3)
+    g.copy_runtime_inputs(**runtime)
+    assert not launches
+    part = tuple(slice(0, d) for d in runtime[name].shape)
+    assert torch.equal(g.inputs[name][part], runtime[name])
+    assert not (g.inputs[name] == 7).any() or (runtime[name] == 7).any()
