@@ -217,7 +217,8 @@ __global__ __launch_bounds__(kProjThreads) void indexer_project_kernel(IndexerAr
 // TOK/WT x OUT/WO of 32x32x16 MFMAs, the weight rows as the A operand, so a
 // lane holds runs of four consecutive outputs of one token (the rotation's
 // pairs).  The rotated 16-bit tile is turned through LDS and stored in whole
-// 16-byte chunks of a token's row.
+// 16-byte chunks of a token's row (words where the output is not 16-byte
+// aligned).
 constexpr int kGemmK = 64;
 constexpr int kGemmChunks = kGemmK / 8;
 
@@ -371,6 +372,7 @@ __global__ __launch_bounds__(64 * WT * WO) void indexer_project_gemm_kernel(Inde
   constexpr int kIters = TOK * kRowChunks / S::kThreads;
   constexpr int kBatch = kIters < 4 ? kIters : 4;
   static_assert(TOK * kRowChunks % S::kThreads == 0 && kIters % kBatch == 0, "epilogue tiling");
+  const bool out16 = (reinterpret_cast<uintptr_t>(a.q_out) & 15) == 0;  // (outputs come 4-byte aligned)
   const bool vec = (a.cos_stride & 7) == 0 && ((reinterpret_cast<uintptr_t>(a.cos) | reinterpret_cast<uintptr_t>(a.sin)) & 15) == 0;
 #pragma unroll 1
   for (int c0 = 0; c0 < kIters; c0 += kBatch) {
@@ -412,8 +414,15 @@ __global__ __launch_bounds__(64 * WT * WO) void indexer_project_gemm_kernel(Inde
           v[i][h] = T::pack2(y0, y1);
         }
       }
-      if (t[i] < ntok)
-        *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(a.q_out) + t[i] * row_elems + out0 + ch * 8) = v[i];
+      if (t[i] < ntok) {
+        uint16_t* out = static_cast<uint16_t*>(a.q_out) + t[i] * row_elems + out0 + ch * 8;
+        if (out16) {
+          *reinterpret_cast<u32x4_t*>(out) = v[i];
+        } else {
+#pragma unroll
+          for (int h = 0; h < 4; ++h) reinterpret_cast<uint32_t*>(out)[h] = v[i][h];
+        }
+      }
     }
   }
 }

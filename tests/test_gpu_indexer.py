@@ -268,6 +268,30 @@ def test_project_many_tokens_close(dtype, T, heads, head_dim, rank, rope):
     _close(got[1:T + 1][..., :rope], eq[..., :rope], dtype, min_exact=0.95, pairs=True)
 
 
+@pytest.mark.parametrize("shift", [2, 4, 6])
+@pytest.mark.parametrize("T,rank", [(64, 256), (65, 256), (130, 512)])
+def test_project_outputs_at_4_byte_addresses(T, rank, shift):
+    """An output 4, 8 or 12 bytes past a 16-byte address holds what an aligned
+    one does, and the elements around it stay untouched."""
+    from nanovllm_amd import ops
+
+    dtype, heads, head_dim, rope = torch.bfloat16, 16, 32, 18
+    print(f"PROJECT unaligned output T={T} rank={rank} shift={shift}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)  # noqa: E731
+    args = (rand(T, 64), rand(T, rank), rand(T, rope), rand(T, rope), rand(heads * head_dim, rank), None)
+    size = T * heads * head_dim
+    aligned = torch.empty(T, heads, head_dim, dtype=dtype, device="cuda")
+    buf = torch.full((size + 16,), 7.0, dtype=dtype, device="cuda")
+    out = buf[shift:shift + size].view(T, heads, head_dim)
+    assert buf.data_ptr() % 16 == 0 and aligned.data_ptr() % 16 == 0
+    for q in (aligned, out):
+        ops.indexer_project_query_only(*args, q, None, heads, head_dim, rope, 1.0)
+    torch.cuda.synchronize()
+    assert torch.equal(out, aligned)
+    assert (buf[:shift] == 7).all() and (buf[shift + size:] == 7).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,heads,hid,fp32,bias", [(1, 16, 64, True, True), (127, 32, 6144, True, False),
                                                    (128, 64, 192, False, True), (129, 32, 6144, True, True),
