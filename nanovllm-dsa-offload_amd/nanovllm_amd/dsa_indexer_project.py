@@ -13,7 +13,7 @@ buffers and ``ValueError`` conditions):
   fp32 weights, and any weights of more than 64 tokens, take a launch of
   their own (``nvdsa_dsa_indexer_project_kw``: exact products, fp32 sums, one
   cast, as the reference computes them, :82-86) where the tensors are plain
-  (contiguous, aligned, no gradient asked for), and an fp32 library GEMM
+  (contiguous, aligned, no derivative asked for), and an fp32 library GEMM
   otherwise.  ``wq_b_bmm_t`` / ``enable_q_bmm`` are accepted for signature
   parity; the kernels read ``wq_b_weight`` in its natural [H*D, R] layout, so
   the transposed BMM copy (an Ascend layout, :102-130) is not used.
@@ -32,6 +32,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import ops
 
@@ -76,6 +77,16 @@ def _plain(t, shape, dtypes, device, align=16) -> bool:
             and t.data_ptr() % align == 0)
 
 
+def _derivatives_asked(*tensors) -> bool:
+    """Whether autograd follows any of the tensors, in either mode: only the
+    library path hands derivatives on."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return True
+    # (The level is below 0 outside every forward_ad.dual_level().)
+    return (getattr(forward_ad, "_current_level", 0) >= 0
+            and any(forward_ad.unpack_dual(t).tangent is not None for t in tensors))
+
+
 def _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, n_head) -> bool:
     """Whether the head weights can come from the fp32-product kernel
     (nvdsa_dsa_indexer_project_kw): plain tensors of the indexer's shapes;
@@ -88,8 +99,7 @@ def _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out,
             and _plain(hidden_states, hidden_states.shape, (dtype,), device)
             and _plain(weights_proj_weight, (n_head, hidden), (dtype, torch.float32), device)
             and _plain(index_weights_out, (hidden_states.shape[0], n_head), (dtype,), device, 2)
-            and not (torch.is_grad_enabled() and (hidden_states.requires_grad or weights_proj_weight.requires_grad
-                                                  or index_weights_out.requires_grad)))
+            and not _derivatives_asked(hidden_states, weights_proj_weight, index_weights_out))
 
 
 # Tokens of one group of the fused decode launch; past it q comes from the
@@ -148,7 +158,7 @@ def dsa_indexer_project(hidden_states, q_c, cos, sin, wq_b_weight, wk_weight, k_
             and _plain(wk_weight, (128, hidden_states.shape[1]), (dtype,), device)
             and all(_plain(t, (128,), (dtype,), device, 4) for t in norm)
             and (cos.numel() // tokens) % 2 == 0 and index_k_out.data_ptr() % 4 == 0
-            and not (torch.is_grad_enabled() and any(t.requires_grad for t in (wk_weight, index_k_out, *norm)))):
+            and not _derivatives_asked(wk_weight, index_k_out, *norm)):
         ops.indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias, weights_proj_weight,
                                index_k_out, index_weights_out, int(rope_dim), score_scale)
         return q_index_out, index_k_out, index_weights_out

@@ -34,3 +34,37 @@ def test_outputs_with_gradients_keep_the_library_path():
     assert not P._weights_kernel_takes(hidden, weights, out.requires_grad_(), 16)
     with torch.no_grad():
         assert P._weights_kernel_takes(hidden, weights, out, 16)
+
+
+@pytest.mark.parametrize("dual", ["hidden", "weights", "wk", "norm"])
+def test_forward_mode_derivatives_are_handed_on(monkeypatch, dual):
+    """A tangent of an input reaches the outputs that depend on it."""
+    from torch.autograd import forward_ad
+
+    monkeypatch.setattr(P.ops, "indexer_project_query_only", lambda *a: None)
+    monkeypatch.setattr(P.ops, "indexer_project_kw", lambda *a: None)
+    monkeypatch.setattr(P.ops, "dsa_indexer_query_rope_inplace", lambda *a: None)
+    z = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16)  # noqa: E731
+    gen = torch.Generator().manual_seed(1)
+    half = lambda *shape: torch.randn(*shape, generator=gen).to(torch.bfloat16)  # noqa: E731
+    T = 3
+    ins = {"hidden": half(T, 64), "weights": torch.randn(16, 64, generator=gen), "wk": half(128, 64), "norm": half(128)}
+    plain = dict(ins)
+    with forward_ad.dual_level():
+        tangent = torch.ones_like(ins[dual])
+        ins[dual] = forward_ad.make_dual(ins[dual], tangent)
+        q, k, w = z(T, 16, 128), z(T, 128), z(T, 16)
+        P.dsa_indexer_project(ins["hidden"], z(T, 256), z(T, 8), z(T, 8), z(2048, 256), ins["wk"], ins["norm"], None,
+                              ins["weights"], q, k, w, n_head=16, head_dim=128, rope_dim=8, score_scale=0.5)
+        dk, dw = (forward_ad.unpack_dual(t).tangent for t in (k, w))
+        w2 = z(T, 16)
+        P.dsa_indexer_project_query_only(ins["hidden"], z(T, 256), z(T, 8), z(T, 8), z(2048, 256), ins["weights"], q, w2,
+                                         n_head=16, head_dim=128, rope_dim=8, score_scale=0.5)
+        dw2 = forward_ad.unpack_dual(w2).tangent
+    if dual in ("hidden", "weights"):
+        a, b = (tangent, plain["weights"]) if dual == "hidden" else (plain["hidden"], tangent)
+        expect = (a.float() @ b.float().T * 0.5).to(torch.bfloat16)
+        for d in (dw, dw2):
+            torch.testing.assert_close(d, expect, rtol=2.0 ** -7, atol=2.0 ** -7)
+    if dual != "weights":
+        assert dk is not None
