@@ -71,10 +71,14 @@ def _weights_fp32(hidden_states, weights_proj_weight, score_scale: float) -> tor
     return weights.to(hidden_states.dtype)
 
 
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
 def _plain(t, shape, dtypes, device, align=16) -> bool:
-    """A contiguous tensor of this shape that the HIP kernels read as it is."""
-    return (t.shape == shape and t.dtype in dtypes and t.device == device and t.is_contiguous()
-            and t.data_ptr() % align == 0)
+    """A contiguous tensor of this shape whose memory holds its values as the
+    HIP kernels read them (no subclass, lazy negation or sparse layout)."""
+    return (type(t) in _PLAIN_TYPES and t.shape == shape and t.dtype in dtypes and t.device == device
+            and t.layout is torch.strided and not t.is_neg() and t.is_contiguous() and t.data_ptr() % align == 0)
 
 
 def _derivatives_asked(*tensors) -> bool:

@@ -68,3 +68,22 @@ def test_forward_mode_derivatives_are_handed_on(monkeypatch, dual):
             torch.testing.assert_close(d, expect, rtol=2.0 ** -7, atol=2.0 ** -7)
     if dual != "weights":
         assert dk is not None
+
+
+class _Scaled(torch.Tensor):
+    """A tensor whose values are not its memory's (as of quantised weights)."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+@pytest.mark.parametrize("which", ["hidden", "weights"])
+@pytest.mark.parametrize("form", ["plain", "parameter", "negated", "subclass", "sparse"])
+def test_only_plain_memory_goes_to_the_kernel(which, form):
+    make = {"plain": lambda t: t, "parameter": lambda t: torch.nn.Parameter(t, requires_grad=False),
+            "negated": torch._neg_view, "subclass": lambda t: t.as_subclass(_Scaled), "sparse": lambda t: t.to_sparse()}[form]
+    ins = {"hidden": torch.ones(3, 64, dtype=torch.bfloat16), "weights": torch.ones(16, 64)}
+    ins[which] = make(ins[which])
+    out = torch.zeros(3, 16, dtype=torch.bfloat16)
+    assert P._weights_kernel_takes(ins["hidden"], ins["weights"], out, 16) == (form in ("plain", "parameter"))
