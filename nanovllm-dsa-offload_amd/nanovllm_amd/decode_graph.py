@@ -32,6 +32,7 @@ import math
 from typing import Iterable
 
 import torch
+from torch.autograd.graph import increment_version
 
 from . import dsa_offload_ops as ops
 from . import ops as _op_impl
@@ -246,6 +247,7 @@ class DsaLayerGraph:
                 staged += (self._address[name], src.data_ptr(), 1, 1, nbytes, nbytes // self.batch_size * real, 0, 0)
         if plain:
             _op_impl.stage_inputs(staged, self._block)
+            increment_version(self._block)  # written, for autograd (its views, the inputs, share the counter)
         else:
             self._copy_inputs(runtime, real)
         self.real_batch = real

@@ -33,6 +33,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad
+from torch.autograd.graph import increment_version  # what the library path's copies do to their outputs
 
 from . import ops
 
@@ -132,6 +133,7 @@ def dsa_indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, we
                                        head_dim, rope_dim, score_scale)
         ops.indexer_project_kw(hidden_states, None, None, None, None, None, weights_proj_weight, None,
                                index_weights_out, rope_dim, score_scale)
+        increment_version(index_weights_out)
         return q_index_out, index_weights_out
     ops.indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, weights_proj_weight if same else None,
                                    q_index_out, index_weights_out if same else None, n_head, head_dim, rope_dim,
@@ -165,6 +167,7 @@ def dsa_indexer_project(hidden_states, q_c, cos, sin, wq_b_weight, wk_weight, k_
             and not _derivatives_asked(wk_weight, index_k_out, *norm)):
         ops.indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias, weights_proj_weight,
                                index_k_out, index_weights_out, int(rope_dim), score_scale)
+        increment_version((index_k_out, index_weights_out))
         return q_index_out, index_k_out, index_weights_out
     # k: library projection and layer norm, then the RoPE kernel on [T, 1, D].
     k = F.linear(hidden_states, wk_weight)

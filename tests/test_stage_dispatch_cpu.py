@@ -84,3 +84,11 @@ def test_replaced_inputs_get_the_step(monkeypatch, name, how):
     part = tuple(slice(0, d) for d in runtime[name].shape)
     assert torch.equal(g.inputs[name][part], runtime[name])
     assert not (g.inputs[name] == 7).any() or (runtime[name] == 7).any()
+
+
+def test_staged_inputs_count_as_written(monkeypatch):
+    g, launches = _graph(monkeypatch)
+    before = {n: t._version for n, t in g.inputs.items()}
+    g.copy_runtime_inputs(**_runtime(g, 2))
+    assert launches
+    assert all(t._version > before[n] for n, t in g.inputs.items())
