@@ -10,11 +10,12 @@ buffers and ``ValueError`` conditions):
   ``weights_proj_weight`` shares the activations' dtype (the decode graph's
   cached low-precision copy, nanovllm/models/glm_mla.py:262-271) both come
   from one fused gfx950 launch (``nvdsa_dsa_indexer_project_query_only``).
-  fp32 weights, and any weights of more than 64 tokens, take a launch of
-  their own (``nvdsa_dsa_indexer_project_kw``: exact products, fp32 sums, one
-  cast, as the reference computes them, :82-86) where the tensors are plain
-  (contiguous, aligned, no derivative asked for), and an fp32 library GEMM
-  otherwise.  ``wq_b_bmm_t`` / ``enable_q_bmm`` are accepted for signature
+  fp32 weights, and any weights of many tokens (from 65 to 385 on, by the
+  sizes: :func:`_one_launch`), take launches of their own
+  (``nvdsa_dsa_indexer_project_kw``: exact products, fp32 sums, one cast, as
+  the reference computes them, :82-86) where the tensors are plain
+  (contiguous, aligned, no derivative asked for), and fp32 ones an fp32 library
+  GEMM otherwise.  ``wq_b_bmm_t`` / ``enable_q_bmm`` are accepted for signature
   parity; the kernels read ``wq_b_weight`` in its natural [H*D, R] layout, so
   the transposed BMM copy (an Ascend layout, :102-130) is not used.
 * :func:`dsa_indexer_project` (reference :245-293), the prefill path: q as
@@ -107,9 +108,30 @@ def _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out,
             and not _derivatives_asked(hidden_states, weights_proj_weight, index_weights_out))
 
 
-# Tokens of one group of the fused decode launch; past it q comes from the
-# tiled GEMM and the head weights from their own kernel.
-_GROUP_TOKENS = 64
+def _one_launch(tokens: int, n_head: int, head_dim: int, rank: int) -> bool:
+    """Whether q and 16-bit head weights come from the fused decode launch:
+    for one 64-token group, and for more while reading wq_b again for each
+    group costs less than the three launches of many tokens (the tiled GEMM,
+    the head weights and their sum), whose time hardly grows with the tokens.
+    bf16, us of one launch / of three:
+
+         heads  rank  hidden   65     96    128    160    192    256    320
+        32x128  2048    6144  20/33  24/34  30/35  38/34  43/34  57/37  70/38
+        32x128  1536    5120  16/30  19/30  23/32  30/31  34/31  44/33  55/35
+        32x128   512    2048  11/22  12/22  14/22  18/22  20/22  26/22  32/22
+        64x128  2048    6144  39/44  47/44  58/45  74/45  84/46 111/46 137/49
+        64x128   512    2048  19/23  23/22  26/24  35/23  38/24  50/25  63/27
+        16x128  2048    6144  15/33  15/33  15/33  22/33  28/33  28/35  41/34
+         64x64  1536    6144  19/33  22/33  28/33  35/34  40/34  53/34  65/37
+
+    fp16 the same within 3 us.  Called from Python the three take 40 us of host
+    time whatever the tokens, so the line lies at the upper end of where they
+    cross.  Heads narrower than 64 keep the one group (a call of 65 to 512
+    tokens, 16x16 heads: 33 to 34 us either way)."""
+    if tokens <= 64 or head_dim < 64:
+        return tokens <= 64
+    most, outputs = (256, 5 * 2 ** 17) if rank > 1024 else (384, 6 * 2 ** 17)
+    return tokens <= most and tokens * n_head * head_dim <= outputs
 
 
 def dsa_indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, weights_proj_weight, q_index_out,
@@ -123,11 +145,11 @@ def dsa_indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, we
     if index_weights_out.shape != (tokens, n_head):
         raise ValueError(f"index_weights_out shape must be {(tokens, n_head)}, got {tuple(index_weights_out.shape)}")
     same = weights_proj_weight.dtype == hidden_states.dtype
-    # One launch for both up to a group of tokens; more tokens (or fp32 head
-    # weights) take the head weights' own kernel where it reads their form.
-    # (16-bit weights only in the sizes that the one launch takes too).
-    if ((not same or (tokens > _GROUP_TOKENS and hidden_states.shape[-1] % 512 == 0
-                      and index_weights_out.data_ptr() % 4 == 0))
+    # One launch for both while that is the shorter way; more tokens (or fp32
+    # head weights) take the head weights' own kernel where it reads their
+    # form.  (16-bit weights only in the sizes that the one launch takes too).
+    if ((not same or (not _one_launch(tokens, n_head, head_dim, q_c.shape[-1])
+                      and hidden_states.shape[-1] % 512 == 0 and index_weights_out.data_ptr() % 4 == 0))
             and _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, n_head)):
         ops.indexer_project_query_only(hidden_states, q_c, cos, sin, wq_b_weight, None, q_index_out, None, n_head,
                                        head_dim, rope_dim, score_scale)

@@ -27,6 +27,24 @@ def test_16_bit_head_weights_keep_their_limits(monkeypatch, tokens, hidden, shif
     assert calls == ([False, "kw"] if split else [True])
 
 
+@pytest.mark.parametrize("tokens,heads,rank,one", [
+    (65, 32, 2048, True), (160, 32, 2048, True), (161, 32, 2048, False), (192, 32, 512, True), (193, 32, 512, False),
+    (80, 64, 1536, True), (81, 64, 1536, False), (256, 16, 2048, True), (257, 16, 2048, False), (384, 16, 512, True),
+    (385, 16, 512, False),
+])
+def test_16_bit_head_weights_by_size(monkeypatch, tokens, heads, rank, one):
+    """q and the head weights in one launch up to the size where the three
+    launches of many tokens are the shorter way."""
+    calls = []
+    monkeypatch.setattr(P.ops, "indexer_project_query_only", lambda *a: calls.append(a[5] is not None))
+    monkeypatch.setattr(P.ops, "indexer_project_kw", lambda *a: calls.append("kw"))
+    z = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16)  # noqa: E731
+    P.dsa_indexer_project_query_only(z(tokens, 512), z(tokens, rank), z(tokens, 64), z(tokens, 64), z(heads * 128, rank),
+                                     z(heads, 512), z(tokens, heads, 128), z(tokens, heads), n_head=heads, head_dim=128,
+                                     rope_dim=64, score_scale=1.0)
+    assert calls == ([True] if one else [False, "kw"])
+
+
 def test_outputs_with_gradients_keep_the_library_path():
     hidden = torch.zeros(65, 512, dtype=torch.bfloat16)
     weights, out = torch.zeros(16, 512), torch.zeros(65, 16, dtype=torch.bfloat16)
