@@ -263,7 +263,7 @@ def test_torch_library_schemas_match_reference():
         registered[name] = text[len("nanovllm_dsa::"):]
         assert hashlib.sha256(registered[name].encode()).hexdigest() == golden[name], name
     ref = Path("/root/reference")
-    if ref.exists():
+    if ref.is_dir() and any(ref.iterdir()):
         import importlib.util
 
         spec = importlib.util.spec_from_file_location("make_schema_digests",
