@@ -1126,62 +1126,17 @@ __device__ inline void load_keys8(const float* s, int n, int t0, uint32_t* u, bo
   }
 }
 
-// The float whose key `score_key` gives.
-__device__ inline float key_score(uint32_t key) {
-  return __uint_as_float((key & 0x80000000u) ? key & 0x7fffffffu : ~key);
-}
-
-// First digits of a row of linear scores: the scores of both signs that the
-// first decode ranks spread their key range over every exponent down to zero,
-// and the top bits of a key would put hundreds of tokens around the C-th
-// largest into one bin.  The digit is the score's place in [lo, hi] instead,
-// in kHistBins steps: each operation is monotone, so digits order as scores
-// do.  A range that is not finite (or empty) puts every token into bin 0,
-// where the select works on the exact keys.
-struct LinearDigits {
-  float lo, steps;
-  __device__ LinearDigits(uint32_t lo_key, uint32_t hi_key) : lo(key_score(lo_key)) {
-    const float range = key_score(hi_key) - lo;
-    steps = range > 0.f && range <= FLT_MAX ? static_cast<float>(kHistBins) / range : 0.f;
-    if (!(steps <= FLT_MAX)) steps = 0.f;  // (a range of denormals)
-  }
-  __device__ uint32_t operator()(uint32_t key) const {
-    if (steps == 0.f) return 0u;  // (uniform)
-    return min(static_cast<uint32_t>((key_score(key) - lo) * steps), static_cast<uint32_t>(kHistBins - 1));
-  }
-};
-
-// One chunk's share of a row's first-digit histogram `gh`: the row's key range
-// from its blocks' ranges `rg` (part 0 leaves the smallest key and the shift,
-// or the largest key for linear digits, in rowsel), the chunk's digits counted
-// in LDS, then added.
-template <bool LINEAR>
-__device__ __forceinline__ void chunk_first_digits(const float* s, int n, int part, const uint2* rg, uint32_t* gh,
-                                                   uint32_t* rowsel, uint32_t* hist, uint32_t* red) {
-  const int tid = threadIdx.x;
-  uint32_t u[kItems];
-  bool in[kItems];
-  load_keys8(s, n, part * kChunk + tid * kItems, u, in);
-  const int nblocks = static_cast<int>(ceil_div(n, kBlock));
-  uint32_t lo = 0xffffffffu, hi = 0u;
-  for (int i = tid; i < nblocks; i += kManageThreads) {
-    const uint2 v = rg[i];
-    lo = min(lo, v.x);
-    hi = max(hi, v.y);
-  }
-  for (int i = tid; i < kHistBins; i += kManageThreads) hist[i] = 0u;
-  block_minmax<true>(lo, hi, red);  // its barriers also order the clearing before the counts (the key loads stay in flight)
-  const int shift = hist_shift(lo, hi);
-  if (part == 0 && tid == 0) {
-    rowsel[0] = lo;
-    rowsel[1] = LINEAR ? hi : static_cast<uint32_t>(shift);
-  }
-  const LinearDigits digit(lo, hi);
+// Adds a chunk's first digits, digit(key) of its keys u (those in(e)), to the
+// row's histogram `gh`: counted in LDS (`hist`, cleared; the caller's barriers
+// order the clearing before this), then added.
+template <typename In, typename Digit>
+__device__ __forceinline__ void add_first_digits(const uint32_t (&u)[kItems], const In& in, const Digit& digit,
+                                                 uint32_t* gh, uint32_t* hist) {
 #pragma unroll
   for (int e = 0; e < kItems; ++e)
-    if (in[e]) atomicAdd(&hist[LINEAR ? digit(u[e]) : (u[e] - lo) >> shift], 1u);
+    if (in(e)) atomicAdd(&hist[digit(u[e])], 1u);
   __syncthreads();
-  for (int i = tid; i < kHistBins; i += kManageThreads) {
+  for (int i = threadIdx.x; i < kHistBins; i += kManageThreads) {
     const uint32_t v = hist[i];
     if (v != 0u) atomicAdd(&gh[i], v);
   }
@@ -1204,9 +1159,26 @@ __global__ __launch_bounds__(kManageThreads) void lim_hist_kernel(LimArgs a, Lim
   for (int i = part * kManageThreads + tid; i < c; i += parts * kManageThreads) stab[i] = kStateFree;
   if (part * kChunk >= n) return;
   const int64_t cap = a.source_capacity;
-  chunk_first_digits<false>(w.scores + static_cast<int64_t>(b) * cap, n, part,
-                            w.ranges + static_cast<int64_t>(b) * (cap / kBlock),
-                            w.hist + static_cast<int64_t>(b) * kHistBins, w.rowsel + 4 * b, hist, red);
+  uint32_t u[kItems];
+  bool in[kItems];
+  load_keys8(w.scores + static_cast<int64_t>(b) * cap, n, part * kChunk + tid * kItems, u, in);
+  const uint2* rg = w.ranges + static_cast<int64_t>(b) * (cap / kBlock);
+  const int nblocks = static_cast<int>(ceil_div(n, kBlock));
+  uint32_t lo = 0xffffffffu, hi = 0u;
+  for (int i = tid; i < nblocks; i += kManageThreads) {
+    const uint2 v = rg[i];
+    lo = min(lo, v.x);
+    hi = max(hi, v.y);
+  }
+  for (int i = tid; i < kHistBins; i += kManageThreads) hist[i] = 0u;
+  block_minmax<true>(lo, hi, red);  // its barriers also order the clearing before the counts (the key loads stay in flight)
+  const int shift = hist_shift(lo, hi);
+  if (part == 0 && tid == 0) {
+    w.rowsel[4 * b] = lo;
+    w.rowsel[4 * b + 1] = static_cast<uint32_t>(shift);
+  }
+  add_first_digits(u, [&](int e) { return in[e]; }, [=](uint32_t key) { return (key - lo) >> shift; },
+                   w.hist + static_cast<int64_t>(b) * kHistBins, hist);
 }
 
 // The hit half of an MTP0 output row: positions m, m+1, ... get the hits by
@@ -1768,12 +1740,12 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
   if (tid == 0) a.miss_counts[b] = m;
 }
 
-// The first-digit bin holding the k-th largest key of a row, and the count of
-// keys above it: thread tid owns bins [P tb, P tb + P), P = kHistPerThread, tb
+// The first-digit bin holding the k-th largest key of a row, the count of keys
+// above it and the count in it: thread tid owns bins [P tb, P tb + P), P = kHistPerThread, tb
 // = 511 - tid, so ascending threads scan descending bins.  (Barriers order LDS
 // only: the caller's loads stay in flight.)
 __device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int* scratch, int* bcast, int& bin,
-                                                int& above) {
+                                                int& above, int& count) {
   const int tid = threadIdx.x;
   constexpr int P = kHistPerThread;
   const int tb = kManageThreads - 1 - tid;
@@ -1796,7 +1768,7 @@ __device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int
   int sum = 0;
 #pragma unroll
   for (int j = 0; j < P; ++j) sum += cnt[j];
-  if (tid == 0) bcast[0] = bcast[1] = 0;  // ordered before the writes below by the scan's barriers
+  if (tid == 0) bcast[0] = bcast[1] = bcast[2] = 0;  // ordered before the writes below by the scan's barriers
   int total;
   int acc = block_exclusive_scan<true>(sum, scratch, &total);  // the token loads stay in flight
   if (acc < k && k <= acc + sum) {
@@ -1805,6 +1777,7 @@ __device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int
       if (acc < k && k <= acc + cnt[j]) {
         bcast[0] = P * tb + j;
         bcast[1] = acc;
+        bcast[2] = cnt[j];
       }
       acc += cnt[j];
     }
@@ -1812,6 +1785,7 @@ __device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int
   lds_barrier();
   bin = __builtin_amdgcn_readfirstlane(bcast[0]);
   above = __builtin_amdgcn_readfirstlane(bcast[1]);
+  count = __builtin_amdgcn_readfirstlane(bcast[2]);
 }
 
 // One 4096-token chunk of an MTP0 request (every launch shape): the row's
@@ -1835,8 +1809,8 @@ __device__ __forceinline__ ChunkSel classify_chunk(const LimArgs& a, const LimWs
   int32_t slot[kItems];
   bool in[kItems];
   load_tokens8(w.scores + static_cast<int64_t>(b) * cap, a.pool + static_cast<int64_t>(r) * cap, n, t0, u, slot, in);
-  int bin, above;
-  first_digit_bin(w.hist + static_cast<int64_t>(b) * kHistBins, kTopK, scratch, bcast, bin, above);
+  int bin, above, count;
+  first_digit_bin(w.hist + static_cast<int64_t>(b) * kHistBins, kTopK, scratch, bcast, bin, above, count);
   uint32_t* stab = w.slot_table + static_cast<int64_t>(b) * kTableStride;
   uint32_t* skey = w.slot_key + static_cast<int64_t>(b) * kTableStride;
   unsigned missm = 0u, inbin = 0u;
@@ -2245,9 +2219,10 @@ struct InitWs {
   int32_t* count;    // list length
   uint2* ranges;     // [S_cap/128] smallest and largest score key of each 128-token block
   uint32_t* hist;    // [kHistBins] first-digit histogram
-  uint32_t* rowsel;  // [4] smallest key, first-digit shift, bin of the C-th largest key, keys above it
+  uint32_t* rowsel;  // [4] range of the digits, bin of the C-th largest key, keys above it
   int32_t* counts;   // [parts, 2] keys above the bin, in-bin tokens of each chunk
   uint2* gather;     // [parts, kGatherPart] in-bin (token, key) of each chunk
+  uint2* spans;      // [parts] smallest and largest in-bin key of each chunk (written for more than kGatherPart in all)
   int32_t* done;     // (cleared by the score kernel)
 };
 
@@ -2271,6 +2246,7 @@ InitWs init_layout(void* base, int64_t cap, size_t* bytes) {
   w.rowsel = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * 4));
   w.counts = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * 2 * mtp_parts(cap)));
   w.gather = reinterpret_cast<uint2*>(take(sizeof(uint2) * kGatherPart * mtp_parts(cap)));
+  w.spans = reinterpret_cast<uint2*>(take(sizeof(uint2) * mtp_parts(cap)));
   w.done = reinterpret_cast<int32_t*>(take(sizeof(int32_t)));
   if (bytes != nullptr) *bytes = p - p0;
   return w;
@@ -2283,7 +2259,8 @@ InitWs carve_init(void* base, int64_t cap) { return init_layout(base, cap, nullp
 // rewritten over its whole length (-1 outside the selection), and the (token,
 // slot) copy list: three kernels of one 512-thread workgroup per 4096-token
 // chunk, on the key ranges that the score kernel leaves.
-//   lidu_hist    the row's first-digit histogram, as lim_hist.
+//   lidu_hist    the range of the digits from the blocks' key ranges, and the
+//                row's first-digit histogram.
 //   lidu_chunks  the bin holding the C-th largest key; each chunk's count of
 //                keys above it, and its tokens in it (count and list).
 //   lidu_init    every chunk ranks the in-bin tokens of all chunks (a few
@@ -2294,35 +2271,147 @@ InitWs carve_init(void* base, int64_t cap) { return init_layout(base, cap, nullp
 // kernels take 16 us at 32768 tokens (initialize_lidu_row: 78.5 -> 68 us with the
 // copy).
 
+// The float whose key `score_key` gives.
+__device__ inline float key_score(uint32_t key) {
+  return __uint_as_float((key & 0x80000000u) ? key & 0x7fffffffu : ~key);
+}
+
+// Score keys of tokens [t0, t0 + 8) of a row of whole blocks (n a multiple of
+// kBlock, t0 of 8: all of them exist or none); whether they exist.
+__device__ __forceinline__ bool load_keys8_whole(const float* s, int n, int t0, uint32_t (&u)[kItems]) {
+  const bool in = t0 < n;
+  if (in) {
+    const float4 x = *reinterpret_cast<const float4*>(s + t0);
+    const float4 y = *reinterpret_cast<const float4*>(s + t0 + 4);
+    u[0] = score_key(x.x); u[1] = score_key(x.y); u[2] = score_key(x.z); u[3] = score_key(x.w);
+    u[4] = score_key(y.x); u[5] = score_key(y.y); u[6] = score_key(y.z); u[7] = score_key(y.w);
+  }
+  return in;
+}
+
+// First digits of a row of linear scores: the scores of both signs that the
+// first decode ranks spread their key range over every exponent down to zero,
+// and the top bits of a key would put hundreds of tokens around the C-th
+// largest into one bin.  The digit is the score's place in [lo, hi] instead,
+// in kHistBins - 2 steps between a bin for the keys below and one for those
+// above: each operation is monotone, so digits order as keys do.  A range that
+// is not finite (or empty) puts every token into one bin.
+struct LinearDigits {
+  uint32_t lo, hi;
+  float base, steps;
+  __device__ LinearDigits(uint32_t lo_key, uint32_t hi_key) : lo(lo_key), hi(hi_key), base(key_score(lo_key)) {
+    const float range = key_score(hi_key) - base;
+    steps = range > 0.f && range <= FLT_MAX ? static_cast<float>(kHistBins - 2) / range : 0.f;
+    if (!(steps <= FLT_MAX)) steps = 0.f;  // (a range of denormals)
+  }
+  __device__ uint32_t operator()(uint32_t key) const {
+    // (Selects: with branches for the rare keys outside, lidu_hist and lidu_chunks take 1 us more.)
+    const uint32_t inside =
+        1u + min(static_cast<uint32_t>((key_score(key) - base) * steps), static_cast<uint32_t>(kHistBins - 3));
+    const uint32_t digit = key < lo ? 0u : key > hi ? static_cast<uint32_t>(kHistBins - 1) : inside;
+    return steps == 0.f ? 0u : digit;
+  }
+};
+
+// Range [lo, hi] of keys for the digits of a row of whole blocks whose key
+// ranges are rg, so that outlying keys of a few blocks do not stretch it.  The
+// blocks are dealt in turn to up to 16 pairs of groups; a pair reaches as far
+// as both of its groups do, and the range as far as one of the pairs, without
+// unmapped blocks (-FLT_MAX throughout).  The C-th largest key may lie outside,
+// if the selection ends among the outlying keys: that costs time only.
+// (Between the smallest and largest key of all, one outlying score or an
+// unmapped block put the other tokens into one bin: 118 us for the call at
+// 32768 tokens instead of 67.)
+constexpr int kWindowPairs = kManageThreads / 32;
+
+__device__ __forceinline__ void row_window(const uint2* rg, int nblocks, uint2* red, uint32_t& lo, uint32_t& hi) {
+  const int pairs = min(kWindowPairs, max(1, nblocks / 16));
+  const int pair = threadIdx.x >> 5, row = (threadIdx.x >> 4) & 1, pos = threadIdx.x & 15;
+  lo = 0xffffffffu;
+  hi = 0u;
+  if (pair < pairs)
+    for (int i = (2 * pos + row) * pairs + pair; i < nblocks; i += 32 * pairs) {
+      const uint2 v = rg[i];
+      if (v.y != score_key(-FLT_MAX)) {
+        lo = min(lo, v.x);
+        hi = max(hi, v.y);
+      }
+    }
+  // Over the 16 lanes of a row, in every lane of it.
+  auto row_minmax = [&]() {
+    auto step = [&](auto ctrl) {
+      auto dpp = [](uint32_t v) {
+        return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v),
+                                                                 decltype(ctrl)::value, 0xf, 0xf, false));
+      };
+      lo = min(lo, dpp(lo));
+      hi = max(hi, dpp(hi));
+    };
+    step(std::integral_constant<int, 0xb1>{});   // quad_perm [1,0,3,2]
+    step(std::integral_constant<int, 0x4e>{});   // quad_perm [2,3,0,1]
+    step(std::integral_constant<int, 0x141>{});  // row_half_mirror
+    step(std::integral_constant<int, 0x140>{});  // row_mirror
+  };
+  row_minmax();
+  const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);  // the values of the pair's two rows
+  const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  if ((threadIdx.x & 31) == 0)
+    red[pair] = pair < pairs ? make_uint2(max(l[0], l[1]), min(h[0], h[1])) : make_uint2(0xffffffffu, 0u);
+  lds_barrier();
+  const uint2 v = red[threadIdx.x & (kWindowPairs - 1)];
+  lo = v.x;
+  hi = v.y;
+  static_assert(kWindowPairs == 16, "one row of lanes");
+  row_minmax();
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  hi = __builtin_amdgcn_readfirstlane(hi);
+}
+
 // Chunk p's keys above the bin and in-bin tokens: counts[2 p], counts[2 p + 1];
 // the first kGatherPart in-bin (token, key) pairs, in token order, at
 // gather[p * kGatherPart].
 __global__ __launch_bounds__(kManageThreads) void lidu_hist_kernel(const float* s, int n, InitWs w) {
   __shared__ uint32_t hist[kHistBins];
-  __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
-  chunk_first_digits<true>(s, n, blockIdx.x, w.ranges, w.hist, w.rowsel, hist, red);
+  __shared__ uint2 red[kWindowPairs];
+  const int part = blockIdx.x, tid = threadIdx.x;
+  uint32_t u[kItems];
+  const bool in = load_keys8_whole(s, n, part * kChunk + tid * kItems, u);
+  for (int i = tid; i < kHistBins; i += kManageThreads) hist[i] = 0u;
+  uint32_t lo, hi;
+  row_window(w.ranges, n / kBlock, red, lo, hi);  // its barrier also orders the clearing before the counts
+  if (part == 0 && tid == 0) {
+    w.rowsel[0] = lo;
+    w.rowsel[1] = hi;
+  }
+  const LinearDigits digit(lo, hi);
+  if (digit.steps == 0.f) {  // (uniform) one bin: the chunk's tokens at once
+    if (tid == 0) atomicAdd(&w.hist[0], static_cast<uint32_t>(min(kChunk, n - part * kChunk)));
+    return;
+  }
+  add_first_digits(u, [=](int) { return in; }, digit, w.hist, hist);
 }
 
 __global__ __launch_bounds__(kManageThreads) void lidu_chunks_kernel(const float* s, int n, int c, InitWs w) {
+  __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
   __shared__ int scratch[kManageThreads / 64 + 1];
   __shared__ uint64_t scratch64[kManageThreads / 64 + 1];
   __shared__ int bcast[4];
   const int part = blockIdx.x, tid = threadIdx.x;
   const int t0 = part * kChunk + tid * kItems;
   uint32_t u[kItems];
-  bool in[kItems];
-  load_keys8(s, n, t0, u, in);
+  const bool in = load_keys8_whole(s, n, t0, u);
   const LinearDigits digit(w.rowsel[0], w.rowsel[1]);
-  int bin, above;
-  first_digit_bin(w.hist, c, scratch, bcast, bin, above);
+  int bin, above, count;
+  first_digit_bin(w.hist, c, scratch, bcast, bin, above, count);
   unsigned inbin = 0u;
   int over = 0;
+  if (in) {
 #pragma unroll
-  for (int e = 0; e < kItems; ++e) {
-    if (!in[e]) continue;
-    const uint32_t d = digit(u[e]);
-    if (d == static_cast<uint32_t>(bin)) inbin |= 1u << e;
-    if (d > static_cast<uint32_t>(bin)) ++over;
+    for (int e = 0; e < kItems; ++e) {
+      const uint32_t d = digit(u[e]);
+      if (d == static_cast<uint32_t>(bin)) inbin |= 1u << e;
+      if (d > static_cast<uint32_t>(bin)) ++over;
+    }
   }
   uint64_t tot;
   const uint64_t pos =
@@ -2343,12 +2432,115 @@ __global__ __launch_bounds__(kManageThreads) void lidu_chunks_kernel(const float
       w.rowsel[3] = static_cast<uint32_t>(above);
     }
   }
+  if (count > kGatherPart) {  // (uniform) the lists may overflow: the range of the keys in the bin
+    uint32_t lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+    for (int e = 0; e < kItems; ++e)
+      if ((inbin >> e) & 1u) {
+        lo = min(lo, u[e]);
+        hi = max(hi, u[e]);
+      }
+    block_minmax<true>(lo, hi, red);
+    if (tid == 0) w.spans[part] = make_uint2(lo, hi);
+  }
+}
+
+// The last selected of g (token, key) pairs in LDS, keys descending and equal
+// ones by ascending token, k of them selected: its key and token to bcast[0]
+// and bcast[1].
+__device__ __forceinline__ void rank_pairs(const uint32_t* lkey, const int* ltok, int g, int k, int* bcast, int* cim) {
+  const int tid = threadIdx.x;
+  if (tid >= g) return;
+  const int my_t = ltok[tid];
+  const uint32_t my_k = lkey[tid];
+  int rank = 0;
+  for (int j = 0; j < g; ++j) rank += (lkey[j] > my_k || (lkey[j] == my_k && ltok[j] < my_t)) ? 1 : 0;
+  if (rank < k) atomicAdd(&cim[my_t / kChunk], 1);  // selected tokens of each chunk
+  if (rank == k - 1) {
+    bcast[0] = static_cast<int>(my_k);
+    bcast[1] = my_t;
+  }
+}
+
+// The threshold and the tie cutoff of the row, and the selected tokens before
+// token `end`, by one workgroup from the whole row: the k-th largest of its
+// keys in [lo, hi] (the first-digit bin's; lo < hi), exactly.  For bins that
+// hold more than the lists, but not one key alone: outlying scores in as many
+// blocks as the selection fills, scores over many exponents, ties among others.
+__device__ __forceinline__ void init_select_row(const float* s, int n, int k, uint32_t lo, uint32_t hi, int end,
+                                                uint32_t* hist, int* scratch, int* bcast, uint32_t& thr, int& cutoff,
+                                                int& before) {
+  const int tid = threadIdx.x;
+  // f(key, token) for tokens < upto (a multiple of kItems), kBatch chunks of
+  // loads in flight.  (A rolled loop: with the keys of 32768 tokens in
+  // registers the kernel is 12000 instructions long and spills scalar
+  // registers, which cost the rows that never come here 0.9 of 7.3 us.)
+  constexpr int kBatch = 4;
+  auto each = [&](int upto, auto f) {
+#pragma unroll 1
+    for (int t0 = tid * kItems; t0 < upto; t0 += kBatch * kChunk) {
+      float4 x[kBatch][2];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        const float4* p = reinterpret_cast<const float4*>(s + min(t0 + j * kChunk, upto - kItems));
+        x[j][0] = p[0];
+        x[j][1] = p[1];
+      }
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        const int t = t0 + j * kChunk;
+        if (t < upto) {
+          f(score_key(x[j][0].x), t);
+          f(score_key(x[j][0].y), t + 1);
+          f(score_key(x[j][0].z), t + 2);
+          f(score_key(x[j][0].w), t + 3);
+          f(score_key(x[j][1].x), t + 4);
+          f(score_key(x[j][1].y), t + 5);
+          f(score_key(x[j][1].z), t + 6);
+          f(score_key(x[j][1].w), t + 7);
+        }
+      }
+    }
+  };
+  for (int i = 4 * tid; i < kBins; i += 4 * kManageThreads) *reinterpret_cast<uint4*>(hist + i) = make_uint4(0u, 0u, 0u, 0u);
+  lds_barrier();
+  const SelectOut sel = radix_select_visit(
+      k, lo, hi,
+      [&](auto&& fn) {
+        each(n, [&](uint32_t u, int) {
+          if (u - lo <= hi - lo) fn(u);
+        });
+      },
+      hist, scratch, bcast);
+  thr = sel.thresh;
+  cutoff = INT_MAX;
+  if (sel.cnt_eq != sel.need_eq) {  // the need_eq lowest tokens of the ties: the last of them is the cutoff
+    int ties = 0;
+#pragma unroll 1
+    for (int c0 = 0; c0 < n; c0 += kChunk) {
+      const int t0 = c0 + tid * kItems;
+      uint32_t u[kItems];
+      unsigned eqm = 0u;
+      if (load_keys8_whole(s, n, t0, u)) {
+#pragma unroll
+        for (int e = 0; e < kItems; ++e)
+          if (u[e] == thr) eqm |= 1u << e;
+      }
+      ties = tie_cutoff_step(eqm, t0, sel.need_eq - 1, ties, scratch, bcast);
+    }
+    __syncthreads();
+    cutoff = bcast[3];
+  }
+  int mine = 0;
+  each(end, [&](uint32_t u, int t) { mine += mtp0_selected(u, t, thr, cutoff) ? 1 : 0; });
+  before = block_sum<true>(mine, scratch);
 }
 
 __global__ __launch_bounds__(kManageThreads) void lidu_init_kernel(const float* s, int n, int c, int32_t* pool_row,
                                                                    int64_t row_len, InitWs w) {
-  __shared__ __align__(16) uint32_t hist[kBins];  // the ranking lists, or the streamed select's histogram
+  __shared__ __align__(16) uint32_t hist[kBins];  // the ranking lists, or the whole-row select's histogram
   __shared__ int scratch[kManageThreads / 64 + 1];
+  __shared__ uint32_t red[2 * (kManageThreads / 64) + 2];
   __shared__ int bcast[4];
   __shared__ int goff[kManageThreads], cim[kManageThreads];
   const int tid = threadIdx.x;
@@ -2371,12 +2563,10 @@ __global__ __launch_bounds__(kManageThreads) void lidu_init_kernel(const float* 
     return;
   }
   uint32_t u[kItems];
-  bool in[kItems];
-  load_keys8(s, n, static_cast<int>(t0), u, in);
+  const bool in = load_keys8_whole(s, n, static_cast<int>(t0), u);
   const int active = static_cast<int>(ceil_div(n, kChunk));  // <= kManageThreads (n < 2^21)
   const int above = tid < active ? w.counts[2 * tid] : 0;
   const int ni = tid < active ? w.counts[2 * tid + 1] : 0;
-  const uint32_t lo = w.rowsel[0], hi = w.rowsel[1], bin = w.rowsel[2];
   const int k = c - static_cast<int>(w.rowsel[3]);  // in-bin tokens to select
   cim[tid] = 0;
   int g;
@@ -2396,68 +2586,44 @@ __global__ __launch_bounds__(kManageThreads) void lidu_init_kernel(const float* 
       lkey[tid] = x.y;
     }
     lds_barrier();
-    if (tid < g) {  // key descending, then token ascending
-      const int my_t = ltok[tid];
-      const uint32_t my_k = lkey[tid];
-      int rank = 0;
-      for (int j = 0; j < g; ++j) rank += (lkey[j] > my_k || (lkey[j] == my_k && ltok[j] < my_t)) ? 1 : 0;
-      if (rank < k) atomicAdd(&cim[my_t / kChunk], 1);
-      if (rank == k - 1) {  // the last selected token: the threshold and the tie cutoff
-        bcast[0] = static_cast<int>(my_k);
-        bcast[1] = my_t;
-      }
-    }
+    rank_pairs(lkey, ltok, g, k, bcast, cim);
     lds_barrier();
     thr = static_cast<uint32_t>(bcast[0]);
     cutoff = bcast[1];
     before = block_sum<true>(tid < part ? above + cim[tid] : 0, scratch);
   } else {
-    // More in-bin tokens than the lists hold (heavy ties): every chunk selects
-    // from the whole row by itself.
-    for (int i = tid; i < kBins; i += kManageThreads) hist[i] = 0u;
-    __syncthreads();
-    const LinearDigits digit(lo, hi);
-    const int ngroups = static_cast<int>(ceil_div(n, 4));
-    auto load_bin = [&](int gi, uint32_t* key, bool* inc) {
-      load_score_keys(s, n, 4 * gi, key, inc);
+    // More in-bin tokens than the lists hold.
+    uint32_t blo = 0xffffffffu, bhi = 0u;
+    if (tid < active && ni > 0) {
+      const uint2 r = w.spans[tid];
+      blo = r.x;
+      bhi = r.y;
+    }
+    block_minmax<true>(blo, bhi, red);
+    if (blo == bhi) {
+      // Ties alone: the lowest k tokens of the bin, by the chunks' counts.
+      thr = blo;
+      const int first = goff[part];
+      if (k - first < (part + 1 < active ? goff[part + 1] : g) - first) {  // (uniform) not all of this chunk's
+        unsigned eqm = 0u;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) inc[e] = inc[e] && digit(key[e]) == bin;
-    };
-    const SelectOut sel = radix_select(ngroups, k, lo, hi, load_bin, hist, scratch, bcast);
-    thr = sel.thresh;
-    // Ties in token order up to the last one selected (its token is the
-    // cutoff), and the selected tokens before this chunk on the way.
-    int ties = 0, mine = 0;
-    for (int g0 = 0; g0 < ngroups; g0 += kManageThreads) {
-      const int gi = g0 + tid;
-      unsigned eqm = 0u;
-      if (gi < ngroups) {
-        uint32_t key[4];
-        bool inc[4];
-        load_score_keys(s, n, 4 * gi, key, inc);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (inc[e] && key[e] == thr) eqm |= 1u << e;
-          if (inc[e] && key[e] > thr && 4 * gi + e < part * kChunk) ++mine;
-        }
+        for (int e = 0; e < kItems; ++e)
+          if (in && u[e] == thr) eqm |= 1u << e;
+        if (tid == 0) bcast[3] = -1;  // (none of them)
+        lds_barrier();
+        tie_cutoff_step(eqm, static_cast<int>(t0), k - first - 1, 0, scratch, bcast);
+        __syncthreads();
+        cutoff = bcast[3];
       }
-      ties = tie_cutoff_step(eqm, 4 * gi, sel.need_eq - 1, ties, scratch, bcast);
+      before = block_sum<true>(tid < part ? above : 0, scratch) + min(first, k);
+    } else {
+      init_select_row(s, n, k, blo, bhi, part * kChunk, hist, scratch, bcast, thr, cutoff, before);
     }
-    __syncthreads();
-    cutoff = bcast[3];
-    for (int gi = tid; 4 * gi < part * kChunk; gi += kManageThreads) {
-      uint32_t key[4];
-      bool inc[4];
-      load_score_keys(s, n, 4 * gi, key, inc);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) mine += inc[e] && key[e] == thr && 4 * gi + e <= cutoff ? 1 : 0;
-    }
-    before = block_sum(mine, scratch);
   }
   unsigned selm = 0u;
 #pragma unroll
   for (int e = 0; e < kItems; ++e)
-    if (in[e] && mtp0_selected(u[e], static_cast<int>(t0) + e, thr, cutoff)) selm |= 1u << e;
+    if (in && mtp0_selected(u[e], static_cast<int>(t0) + e, thr, cutoff)) selm |= 1u << e;
   int tot;
   int pos = before + block_exclusive_scan<true>(__popc(selm), scratch, &tot);
   int pv[kItems];

@@ -279,6 +279,55 @@ def test_gpu_initialize_lidu_row_chunk_edges(n_blocks, c, extra, ties):
     assert np.array_equal(bits(g["hbm_kpe"]), hkpe)
 
 
+def _spread(case, form):
+    """Scores (closed form: a token's score is its key row's dims 0 to 3 in
+    base 64) of ranges that leave most tokens in one first digit."""
+    n, c = case["n"], case["c"]
+    rng = np.random.default_rng(n + c)
+    keys, table = case["keys"].reshape(-1, 128).copy(), case["table"].copy()
+    rows = table[np.arange(n) // 128].astype(np.int64) * 128 + np.arange(n) % 128
+    score = lambda t, v: keys.__setitem__(rows[t], O.f32_to_bits(  # noqa: E731  -- token(s) t: dim 0 alone
+        np.eye(1, 128, dtype=np.float32) * np.reshape(v, (-1, 1)).astype(np.float32), case["dtype"]))
+    if form == "unmapped":
+        table[[0, 3, table.size // 2]] = -1
+    elif form == "high":
+        score([n // 3], 1e30)
+    elif form == "low":
+        score([n - 1], -1e30)
+    elif form == "infinite":  # 65 x 3e38 in fp32
+        keys[rows[n // 2], :2] = O.f32_to_bits(np.full(2, 3e38, np.float32), case["dtype"])
+    if form in ("scales", "scales_ties"):
+        score([7, n // 2, n // 3, n - 2], [1e30, 1e15, 1e8, -1e20])
+    if form in ("ties", "scales_ties"):
+        score(rng.choice(np.arange(n - c - 900, n - c + 900), 1500, replace=False), np.full(1500, (n - c) // 256 * 256))
+    elif form == "log":
+        score(np.arange(n), rng.choice([-1, 1], n) * 2.0 ** rng.integers(-60, 60, n) * (1 + rng.integers(0, 128, n) / 128))
+    elif form == "equal":
+        score(np.arange(n), np.full(n, -3.0))
+    elif form == "two":
+        score(np.arange(n), np.where(rng.random(n) < 0.5 * c / n, 7.0, 5.0))
+    return dict(case, keys=keys.reshape(case["keys"].shape), table=table)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["unmapped", "high", "low", "infinite", "scales", "ties", "scales_ties", "log", "equal", "two"])
+@pytest.mark.parametrize("n_blocks,c", [(24, 2048), (160, 3000), (265, 8192)])
+def test_gpu_initialize_lidu_row_stretched_ranges(n_blocks, c, form):
+    """Outlying, infinite, unmapped, tied and widely spread scores, in one
+    chunk, several, and past the sources whose keys stay in registers."""
+    from nanovllm_amd import dsa_offload_ops as ops
+
+    case = _spread(_init_case(n_blocks, n_blocks, c, 32, "bf16", True), form)
+    print(f"LIDU-INIT spread n={case['n']} c={c} {form}", flush=True)
+    slots, hkpe, hckv = _oracle_init(case)
+    g = _to_gpu(case)
+    ops.initialize_lidu_row(candidate_len=case["n"], cache_tokens=c, block_size=128, **g)
+    torch.cuda.synchronize()
+    assert np.array_equal(ints(g["cache_slots_row"]), slots)
+    assert np.array_equal(bits(g["hbm_ckv"]), hckv)
+    assert np.array_equal(bits(g["hbm_kpe"]), hkpe)
+
+
 def _unaligned(t: torch.Tensor) -> torch.Tensor:
     """A copy of 1-D ``t`` whose data starts 4 bytes into an allocation (not
     16-byte aligned), so the kernels take their element-wise path."""
