@@ -38,6 +38,12 @@ int nvdsa_dsa_indexer_project_kw(const nvdsa_tensor* hidden_states,
                                  size_t workspace_bytes,
                                  void* stream);
 
+/* The tile (64, 128 or 256 tokens by as many outputs) in which
+ * nvdsa_dsa_indexer_project_query_only multiplies more than 64 tokens into
+ * `outputs` = n_head * head_dim values; 0 for up to 64 tokens, which take no
+ * tiled product. */
+int nvdsa_dsa_indexer_project_tile(int64_t tokens, int64_t outputs);
+
 /* One row-wise copy of nvdsa_stage_inputs: rows [0, real) of dst (dst_bytes
  * apart) take src_bytes of src's row (src_stride bytes apart) and the 32-bit
  * pattern `fill` after them, rows [real, rows) the pattern alone.  All sizes

@@ -769,24 +769,12 @@ hipError_t launch_project(const IndexerArgs& a, hipStream_t stream) {
   const int q_tiles = static_cast<int>(a.heads * a.head_dim / kRowTile);
   if (a.w_proj == nullptr && a.tokens > kTokPerGroup) {
     // More than one 64-token group: the tiled GEMM (n_head and head_dim are
-    // multiples of 16, so its output tiles divide the rows of wq_b).  Its
-    // tile by the time each would take, measured at 4096 outputs of K 2048: a
-    // launch's 64 x 64 tiles fill the chip's 256 CUs at 13 us and then cost
-    // 26.5 ns each, 128 x 128 ones 29.5 us and 75 ns, 256 x 256 ones 69 us per
-    // round of 256.  64-token groups / 64 / 128 / 256 tiles: 65 tokens 15.8 /
-    // 12.2 / 26 / 56 us, 512: 89 / 22 / 33 / 60, 1024: 174 / 34 / 29.5 / 59,
-    // 2048: 339 / 63 / 46 / 60, 4096: 675 / 120 / 85 / 69 us.
-    const int64_t outs = a.heads * a.head_dim;
-    const int64_t n64 = ceil_div(a.tokens, 64) * (outs / 64), n128 = ceil_div(a.tokens, 128) * (outs / 128);
-    const int64_t n256 = ceil_div(a.tokens, 256) * (outs / 256);
-    const double us64 = std::max(13.0, 7.0 + 0.0265 * n64), us128 = std::max(29.5, 8.0 + 0.075 * n128);
-    const double us256 = 69.0 * ceil_div(n256, 256);
-    if (us64 <= us128 && us64 <= us256)
-      launch_gemm_shape<T, 64, 64, 2, 2>(a, stream);
-    else if (us128 <= us256)
-      launch_gemm_shape<T, 128, 128, 2, 2>(a, stream);
-    else
-      launch_gemm_shape<T, 256, 256, 2, 4>(a, stream);
+    // multiples of 16, so its output tiles divide the rows of wq_b).
+    switch (indexer_gemm_tile(a.tokens, a.heads * a.head_dim)) {
+      case 64: launch_gemm_shape<T, 64, 64, 2, 2>(a, stream); break;
+      case 128: launch_gemm_shape<T, 128, 128, 2, 2>(a, stream); break;
+      default: launch_gemm_shape<T, 256, 256, 2, 4>(a, stream);
+    }
     return hipGetLastError();
   }
   const dim3 grid(static_cast<uint32_t>(q_tiles), static_cast<uint32_t>(ceil_div(a.tokens, kTokPerGroup)));
@@ -805,6 +793,25 @@ hipError_t launch_rope(const RopeArgs& a, hipStream_t stream) {
 }  // namespace
 
 int64_t indexer_k_chunk() { return kKChunk; }
+
+// The GEMM's tile (64, 128 or 256: tokens and outputs of a workgroup) by the
+// time that each would take, measured at 4096 outputs of K 2048: a launch's
+// 64 x 64 tiles fill the chip's 256 CUs at 13 us and then cost 26.5 ns each,
+// 128 x 128 ones 29.5 us and 75 ns, 256 x 256 ones 69 us per round of 256.
+// 64-token groups / 64 / 128 / 256 tiles: 65 tokens 15.8 / 12.2 / 26 / 56 us,
+// 512: 89 / 22 / 33 / 60, 1024: 174 / 34 / 29.5 / 59, 2048: 339 / 63 / 46 / 60,
+// 4096: 675 / 120 / 85 / 69 us.  (Runs back to back; a trace says 74 to 78 us
+// at 4096.)  K is not in the rule, which is fitted at that one: at K 256 to
+// 7168, 256 to 16384 outputs and 65 to 16384 tokens the tile it takes runs in
+// 0.08 to 0.94 of the groups' time.
+int indexer_gemm_tile(int64_t tokens, int64_t outs) {
+  const int64_t n64 = ceil_div(tokens, 64) * (outs / 64), n128 = ceil_div(tokens, 128) * (outs / 128);
+  const int64_t n256 = ceil_div(tokens, 256) * (outs / 256);
+  const double us64 = std::max(13.0, 7.0 + 0.0265 * n64), us128 = std::max(29.5, 8.0 + 0.075 * n128);
+  const double us256 = 69.0 * ceil_div(n256, 256);
+  if (us64 <= us128 && us64 <= us256) return 64;
+  return us128 <= us256 ? 128 : 256;
+}
 
 hipError_t launch_indexer_project(const IndexerArgs& a, hipStream_t stream) {
   if (a.tokens == 0) return hipSuccess;

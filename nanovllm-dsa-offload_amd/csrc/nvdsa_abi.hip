@@ -1107,6 +1107,10 @@ int nvdsa_dsa_indexer_project_query_only(const nvdsa_tensor* hidden_states, cons
 }
 
 // ------------------------------------------------------------------------
+int nvdsa_dsa_indexer_project_tile(int64_t tokens, int64_t outputs) {
+  return tokens > 64 && outputs > 0 ? nvdsa::indexer_gemm_tile(tokens, outputs) : 0;
+}
+
 size_t nvdsa_dsa_indexer_project_kw_workspace_size(int64_t tokens, int64_t n_head, int64_t hidden_size, int32_t with_k) {
   if (tokens < 0 || n_head <= 0 || hidden_size <= 0) return 0;
   return nvdsa::indexer_kw_workspace_bytes(tokens, n_head, hidden_size, with_k != 0);

@@ -204,6 +204,7 @@ struct IndexerArgs {
 };
 // K extents (rank, hid) must be multiples of this.
 int64_t indexer_k_chunk();
+int indexer_gemm_tile(int64_t tokens, int64_t outs);
 hipError_t launch_indexer_project(const IndexerArgs& a, hipStream_t stream);
 
 // Products of hidden_states for many tokens: the index key (wk != null) and

@@ -86,6 +86,7 @@ SIGNATURES = {
 
 # include/nvdsa_ext.h
 EXT_SIGNATURES = {
+    "nvdsa_dsa_indexer_project_tile": ([_I64, _I64], ctypes.c_int),
     "nvdsa_dsa_indexer_project_kw_workspace_size": ([_I64, _I64, _I64, ctypes.c_int32], _SZ),
     "nvdsa_stage_inputs": ([_VP, _I64, _VP], ctypes.c_int),
     "nvdsa_dsa_indexer_project_kw": ([_P] * 9 + [_I64, _DBL, _VP, _SZ, _VP], ctypes.c_int),

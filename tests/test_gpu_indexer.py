@@ -235,13 +235,22 @@ def test_project_errors():
                                        rope_dim=ROPE, score_scale=1.0)
 
 
+def _tile(tokens, outputs):
+    """The tile that the dispatch takes (0: the launch of up to 64 tokens)."""
+    from nanovllm_amd import _lib
+
+    return _lib.lib.nvdsa_dsa_indexer_project_tile(tokens, outputs)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,heads,head_dim,rank,rope", [
     (65, 16, 16, 256, 6),        # 64 x 64 tiles, one token in the last
     (1000, 16, 48, 256, 18),     # heads that end inside a 32-wide tile
     (15999, 16, 16, 512, 16),    # 128 x 128 tiles, all dims rotated
-    (49001, 16, 16, 256, 10),    # 256 x 256 tiles
+    (49001, 16, 16, 256, 10),    # the same, ragged in another place
     (300, 32, 128, 2048, 64),    # the GLM indexer's shape
+    (55001, 16, 16, 256, 10),    # 256 x 256 tiles, one round and more
+    (4001, 32, 128, 256, 62),    # 256 x 256 tiles, heads of 128, a rotation that ends inside a chunk
 ])
 def test_project_many_tokens_close(dtype, T, heads, head_dim, rank, rope):
     """The tiled GEMM path (more than 64 tokens), every tile shape, ragged
@@ -249,6 +258,7 @@ def test_project_many_tokens_close(dtype, T, heads, head_dim, rank, rope):
     from nanovllm_amd import ops
 
     print(f"PROJECT GEMM {dtype} T={T} heads={heads}x{head_dim} rank={rank} rope={rope}", flush=True)
+    assert _tile(T, heads * head_dim) == {65: 64, 1000: 64, 300: 64, 15999: 128, 49001: 128}.get(T, 256)
     rng = np.random.default_rng(T)
     qc = _to_bits(rng.standard_normal((T, rank)), dtype)
     wq = _to_bits(rng.standard_normal((heads * head_dim, rank)) / np.sqrt(rank), dtype)
@@ -269,13 +279,14 @@ def test_project_many_tokens_close(dtype, T, heads, head_dim, rank, rope):
 
 
 @pytest.mark.parametrize("shift", [2, 4, 6])
-@pytest.mark.parametrize("T,rank", [(64, 256), (65, 256), (130, 512)])
-def test_project_outputs_at_4_byte_addresses(T, rank, shift):
+@pytest.mark.parametrize("T,rank,tile", [(64, 256, 0), (65, 256, 64), (130, 512, 64), (8001, 256, 128), (27001, 256, 256)])
+def test_project_outputs_at_4_byte_addresses(T, rank, tile, shift):
     """An output 4, 8 or 12 bytes past a 16-byte address holds what an aligned
     one does, and the elements around it stay untouched."""
     from nanovllm_amd import ops
 
     dtype, heads, head_dim, rope = torch.bfloat16, 16, 32, 18
+    assert _tile(T, heads * head_dim) == tile
     print(f"PROJECT unaligned output T={T} rank={rank} shift={shift}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(T)
     rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)  # noqa: E731
