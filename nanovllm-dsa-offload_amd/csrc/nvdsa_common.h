@@ -56,12 +56,6 @@ struct Bf16 {
     u += 0x7fffu + ((u >> 16) & 1u);
     return static_cast<uint16_t>(u >> 16);
   }
-  // Round-to-nearest-even for finite values (no NaN check).
-  __device__ static inline uint16_t from_finite(float f) {
-    uint32_t u = __float_as_uint(f);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
-  }
   // Two values rounded to nearest even into one 32-bit word (v_cvt_pk_bf16_f32:
   // one instruction for what from_float does in six per value).
   __device__ static inline uint32_t pack2(float a, float b) {
@@ -89,7 +83,6 @@ struct F16 {
     _Float16 h = static_cast<_Float16>(f);
     return __builtin_bit_cast(uint16_t, h);
   }
-  __device__ static inline uint16_t from_finite(float f) { return from_float(f); }
   __device__ static inline uint32_t pack2(float a, float b) {
     return static_cast<uint32_t>(from_float(a)) | (static_cast<uint32_t>(from_float(b)) << 16);
   }
