@@ -181,7 +181,9 @@ def dsa_indexer_project(hidden_states, q_c, cos, sin, wq_b_weight, wk_weight, k_
     # or in 16 bits, which only the library path widens before the product).
     dtype, device = hidden_states.dtype, hidden_states.device
     norm = [t for t in (k_norm_weight, k_norm_bias) if t is not None]
+    # (A rope_dim that the key's RoPE operator refuses goes there too.)
     if (weights_proj_weight.dtype == torch.float32 and int(head_dim) == 128 and k_norm_weight is not None
+            and int(rope_dim) % 16 == 0
             and _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, int(n_head))
             and _plain(wk_weight, (128, hidden_states.shape[1]), (dtype,), device)
             and all(_plain(t, (128,), (dtype,), device, 4) for t in norm)

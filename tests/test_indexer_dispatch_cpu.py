@@ -123,3 +123,18 @@ def test_outputs_count_as_written(monkeypatch):
     P.dsa_indexer_project(z(3, 64), z(3, 256), z(3, 8), z(3, 8), z(2048, 256), z(128, 64), z(128), None,
                           torch.zeros(16, 64), q, k, w, n_head=16, head_dim=128, rope_dim=8, score_scale=0.5)
     assert k._version > before[0] and w._version > before[1]
+
+
+@pytest.mark.parametrize("rope_dim,kernel", [(64, True), (16, True), (6, False), (40, False)])
+def test_key_rotation_keeps_its_limits(monkeypatch, rope_dim, kernel):
+    """A rope_dim that is no multiple of 16 goes to the key's RoPE operator,
+    which refuses it."""
+    calls = []
+    monkeypatch.setattr(P.ops, "indexer_project_query_only", lambda *a: None)
+    monkeypatch.setattr(P.ops, "indexer_project_kw", lambda *a: calls.append("kw"))
+    monkeypatch.setattr(P.ops, "dsa_indexer_query_rope_inplace", lambda *a: calls.append(a[3]))
+    z = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16)  # noqa: E731
+    P.dsa_indexer_project(z(3, 64), z(3, 256), z(3, 64), z(3, 64), z(2048, 256), z(128, 64), z(128), None,
+                          torch.zeros(16, 64), z(3, 16, 128), z(3, 128), z(3, 16), n_head=16, head_dim=128,
+                          rope_dim=rope_dim, score_scale=0.5)
+    assert calls == (["kw"] if kernel else [rope_dim])
