@@ -115,13 +115,13 @@ def test_outputs_count_as_written(monkeypatch):
     z = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16)  # noqa: E731
     q, k, w, scale = z(3, 16, 128), z(3, 128), z(3, 16), torch.ones(3, 16, requires_grad=True)
     loss = (w * scale).sum()
-    P.dsa_indexer_project_query_only(z(3, 64), z(3, 256), z(3, 8), z(3, 8), z(2048, 256), torch.zeros(16, 64), q, w,
-                                     n_head=16, head_dim=128, rope_dim=8, score_scale=0.5)
+    P.dsa_indexer_project_query_only(z(3, 64), z(3, 256), z(3, 16), z(3, 16), z(2048, 256), torch.zeros(16, 64), q, w,
+                                     n_head=16, head_dim=128, rope_dim=16, score_scale=0.5)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         loss.backward()
     before = k._version, w._version
-    P.dsa_indexer_project(z(3, 64), z(3, 256), z(3, 8), z(3, 8), z(2048, 256), z(128, 64), z(128), None,
-                          torch.zeros(16, 64), q, k, w, n_head=16, head_dim=128, rope_dim=8, score_scale=0.5)
+    P.dsa_indexer_project(z(3, 64), z(3, 256), z(3, 16), z(3, 16), z(2048, 256), z(128, 64), z(128), None,
+                          torch.zeros(16, 64), q, k, w, n_head=16, head_dim=128, rope_dim=16, score_scale=0.5)
     assert k._version > before[0] and w._version > before[1]
 
 
