@@ -167,6 +167,10 @@ class DsaLayerGraph:
         torch.cuda.current_stream().wait_stream(stream)
 
     # -- per-step inputs --------------------------------------------------------
+    def _launches_here(self) -> bool:
+        """Whether the buffers are on the current GPU."""
+        return self._device.type == "cuda" and torch.cuda.current_device() == self._device.index
+
     def _stageable(self, name: str, src: torch.Tensor) -> bool:
         """Whether the staging kernel may read ``src`` for input ``name``: the
         input is still this object's buffer, and ``src`` a plain tensor of its
@@ -214,7 +218,7 @@ class DsaLayerGraph:
         # as it is (same device and dtype, contiguous rows).  Anything else
         # sends the whole step through torch copies, one after another.
         staged: list[int] = []
-        plain = torch.cuda.current_device() == self._device.index
+        plain = self._launches_here()
         for name, pad in _ROW_INPUTS.items():
             src = runtime[name]
             if src.shape != (real,):

@@ -12,15 +12,17 @@ from nanovllm_amd import decode_graph as G
 BATCH, HEADS = 4, 4
 
 
-def _graph(monkeypatch):
-    """A graph of CPU buffers, and the staging launches it makes."""
+def _graph(monkeypatch, on_gpu=True):
+    """A graph of CPU buffers, and the staging launches it makes (as if the
+    buffers were on the current GPU)."""
     z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)  # noqa: E731
     g = G.DsaLayerGraph(BATCH, index_key_cache=z(1, 128, 1, 128), cache_slots_pool=torch.zeros(1, 1280),
                         hbm_k_rope=z(1, 128, 1, 64), hbm_kv_cache=z(1, 128, 1, 512), dram_k_rope=z(1, 128, 64),
                         dram_kv_cache=z(1, 128, 512), hbm_block_columns=7, dram_block_columns=9, heads=HEADS,
                         index_heads=32, scale=1.0)
     launches = []
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: g._device.index)
+    if on_gpu:
+        monkeypatch.setattr(g, "_launches_here", lambda: True)
     monkeypatch.setattr(G._op_impl, "stage_inputs",
                         lambda fields, like: launches.append([fields[i:i + 8] for i in range(0, len(fields), 8)]))
     return g, launches
@@ -92,3 +94,14 @@ def test_staged_inputs_count_as_written(monkeypatch):
     g.copy_runtime_inputs(**_runtime(g, 2))
     assert launches
     assert all(t._version > before[n] for n, t in g.inputs.items())
+
+
+def test_host_buffers_take_the_copies(monkeypatch):
+    """A graph object over host memory copies its inputs there, also where
+    there is no GPU."""
+    g, launches = _graph(monkeypatch, on_gpu=False)
+    runtime = _runtime(g, 3)
+    assert g.copy_runtime_inputs(**runtime) == 3 and not launches
+    for name, t in runtime.items():
+        assert torch.equal(g.inputs[name][tuple(slice(0, d) for d in t.shape)], t)
+    assert (g.inputs["req_pool_entries"][3:] == -1).all() and not g.inputs["query"][3:].any()
