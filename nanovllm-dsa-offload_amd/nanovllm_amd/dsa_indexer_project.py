@@ -73,13 +73,17 @@ def _weights_fp32(hidden_states, weights_proj_weight, score_scale: float) -> tor
     return weights.to(hidden_states.dtype)
 
 
-_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+def _plain_type(cls) -> bool:
+    """Tensors, parameters, and parameter classes that leave torch's functions
+    as they are."""
+    return cls is torch.Tensor or (cls.__torch_function__ is torch.nn.Parameter.__torch_function__
+                                   and cls.__torch_dispatch__ is torch.Tensor.__torch_dispatch__)
 
 
 def _plain(t, shape, dtypes, device, align=16) -> bool:
     """A contiguous tensor of this shape whose memory holds its values as the
     HIP kernels read them (no subclass, lazy negation or sparse layout)."""
-    return (type(t) in _PLAIN_TYPES and t.shape == shape and t.dtype in dtypes and t.device == device
+    return (_plain_type(type(t)) and t.shape == shape and t.dtype in dtypes and t.device == device
             and t.layout is torch.strided and not t.is_neg() and t.is_contiguous() and t.data_ptr() % align == 0)
 
 

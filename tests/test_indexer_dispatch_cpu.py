@@ -96,15 +96,20 @@ class _Scaled(torch.Tensor):
         return super().__torch_function__(func, types, args, kwargs or {})
 
 
+class _Loaded(torch.nn.Parameter):
+    """A parameter class that only adds attributes (weight loaders)."""
+
+
 @pytest.mark.parametrize("which", ["hidden", "weights"])
-@pytest.mark.parametrize("form", ["plain", "parameter", "negated", "subclass", "sparse"])
+@pytest.mark.parametrize("form", ["plain", "parameter", "loaded", "negated", "subclass", "sparse"])
 def test_only_plain_memory_goes_to_the_kernel(which, form):
     make = {"plain": lambda t: t, "parameter": lambda t: torch.nn.Parameter(t, requires_grad=False),
-            "negated": torch._neg_view, "subclass": lambda t: t.as_subclass(_Scaled), "sparse": lambda t: t.to_sparse()}[form]
+            "loaded": lambda t: _Loaded(t, requires_grad=False), "negated": torch._neg_view,
+            "subclass": lambda t: t.as_subclass(_Scaled), "sparse": lambda t: t.to_sparse()}[form]
     ins = {"hidden": torch.ones(3, 64, dtype=torch.bfloat16), "weights": torch.ones(16, 64)}
     ins[which] = make(ins[which])
     out = torch.zeros(3, 16, dtype=torch.bfloat16)
-    assert P._weights_kernel_takes(ins["hidden"], ins["weights"], out, 16) == (form in ("plain", "parameter"))
+    assert P._weights_kernel_takes(ins["hidden"], ins["weights"], out, 16) == (form in ("plain", "parameter", "loaded"))
 
 
 def test_outputs_count_as_written(monkeypatch):
