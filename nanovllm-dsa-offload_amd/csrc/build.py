@@ -29,8 +29,8 @@ COMMON_FLAGS = [
     "-fPIC",
     "-std=c++17",
     "-mcode-object-version=5",
-    # Packed fp32 ops have produced silent wrong results on this pool; keep
-    # the compiler from forming them.
+    # Some forms of the packed fp32 instructions have given wrong results now
+    # and then, without an error; keep the compiler from forming them.
     "-Xclang",
     "-target-feature",
     "-Xclang",

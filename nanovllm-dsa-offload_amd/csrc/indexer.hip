@@ -446,8 +446,11 @@ void launch_gemm_shape(const IndexerArgs& a, hipStream_t stream) {
 // product is exact and only the fp32 sums round, as in an fp32 GEMM; sums that
 // an infinity makes NaN are taken again by the finish kernel.  (On the
 // fp32 MFMA, at 1/16 of the rate, the kernel takes 33 us at 4096 tokens, this
-// form 28.6 us, both 2.0e-3 off fp64 in the rounded outputs; what bounds it
-// now is each CU's pull of 40 KB per K step.)  It replaces two library GEMMs (27 +
+// form 28.6 us, both 2.0e-3 off fp64 in the rounded outputs.  Counters: its
+// waves wait for loads or barriers 61% of their cycles and the MFMA pipes are
+// busy 16% of the time; its operands arrive at 7 bytes per clock and CU, where
+// the GEMM above pulls 16, so that pull is not what holds it, and which of
+// the two waits does is not known.)  It replaces two library GEMMs (27 +
 // 24 us), the fp32 copy of hidden_states (22 us), a layer norm, the rotation
 // and six small copies and casts.  Slices leave fp32 partial sums; the finish
 // kernel adds them in slice order, rounds, and does the layer norm, the
