@@ -29,6 +29,7 @@ memset.
 from __future__ import annotations
 
 import math
+import operator
 from typing import Iterable
 
 import torch
@@ -117,7 +118,8 @@ class DsaLayerGraph:
         self._address = {k: self._span[0] + o for k, o in offsets.items()}
         self.inputs = {k: self._block[offsets[k]:offsets[k] + self._nbytes[k]].view(dt).view(shape)
                        for k, (shape, dt) in shapes.items()}
-        self._buffers = dict(self.inputs)  # (a caller may put tensors of its own into `inputs` before the capture)
+        self._buffers = list(self.inputs.values())
+        self._pointers = [t.data_ptr() for t in self._buffers]
         for name, pad in _ROW_INPUTS.items():
             self.inputs[name].fill_(pad)
         self.outputs = {
@@ -171,19 +173,22 @@ class DsaLayerGraph:
         """Whether the buffers are on the current GPU."""
         return self._device.type == "cuda" and torch.cuda.current_device() == self._device.index
 
-    def _stageable(self, name: str, src: torch.Tensor) -> bool:
-        """Whether the staging kernel may read ``src`` for input ``name``: the
-        input is still this object's buffer, and ``src`` a plain tensor of its
-        dtype on its device, outside the static inputs' memory or the buffer
-        itself."""
-        dst = self.inputs[name]
-        if dst is not self._buffers[name] or dst.data_ptr() != self._address[name]:
-            return False
-        if type(src) is not torch.Tensor or src.dtype != dst.dtype or src.device != self._device:
-            return False
+    def _own_buffers(self) -> bool:
+        """Whether the inputs are still the buffers that this object made: a
+        caller may put tensors of its own into ``inputs`` before the capture."""
+        inputs = self.inputs.values()
+        return (len(inputs) == len(self._buffers) and all(map(operator.is_, inputs, self._buffers))
+                and list(map(torch.Tensor.data_ptr, inputs)) == self._pointers)
+
+    def _source(self, name: str, src: torch.Tensor) -> int | None:
+        """The address from which the staging kernel may read ``src`` for buffer
+        ``name``, if it is a plain tensor of the buffer's dtype on its device,
+        outside the static inputs' memory or the buffer itself."""
+        if type(src) is not torch.Tensor or src.dtype != self.inputs[name].dtype or src.device != self._device:
+            return None
         at = src.data_ptr()
         lo, hi = self._span
-        return (at == self._address[name] or not lo <= at < hi) and not (src.requires_grad or src.is_neg())
+        return None if (lo <= at < hi and at != self._address[name]) or src.requires_grad or src.is_neg() else at
 
     def _copy_inputs(self, runtime: dict[str, torch.Tensor], real: int) -> None:
         """The same with torch copies (any device, dtype and layout)."""
@@ -218,14 +223,15 @@ class DsaLayerGraph:
         # as it is (same device and dtype, contiguous rows).  Anything else
         # sends the whole step through torch copies, one after another.
         staged: list[int] = []
-        plain = self._launches_here()
+        plain = self._launches_here() and self._own_buffers()
         for name, pad in _ROW_INPUTS.items():
             src = runtime[name]
             if src.shape != (real,):
                 raise ValueError(f"{name} must be [{real}], got {tuple(src.shape)}")
-            plain = plain and self._stageable(name, src) and src.is_contiguous()
+            at = self._source(name, src) if plain else None
+            plain = at is not None and src.is_contiguous()
             if plain:
-                staged += (self._address[name], src.data_ptr(), 1, 1, 4 * self.batch_size, 4 * real, 0, pad)
+                staged += (self._address[name], at, 1, 1, 4 * self.batch_size, 4 * real, 0, pad)
         for name in _TABLES:
             src, width = runtime[name], self.inputs[name].shape[1]
             shape = src.shape
@@ -235,20 +241,22 @@ class DsaLayerGraph:
                 raise ValueError(f"{name} is wider than its graph buffer: runtime={shape[1]}, graph={width}.")
             # (Rows of the buffer's own memory at another stride would be read
             # where other rows are written.)
-            plain = (plain and self._stageable(name, src) and src.stride(1) == 1
-                     and (src.data_ptr() != self._address[name] or src.stride(0) == width or real <= 1))
+            at = self._source(name, src) if plain else None
+            plain = (at is not None and src.stride(1) == 1
+                     and (at != self._address[name] or src.stride(0) == width or real <= 1))
             if plain:
-                staged += (self._address[name], src.data_ptr(), self.batch_size, real, 4 * width, 4 * shape[1],
+                staged += (self._address[name], at, self.batch_size, real, 4 * width, 4 * shape[1],
                            4 * src.stride(0), 0)
         for name in _QUERY_INPUTS:
             src, dst = runtime[name], self.inputs[name]
             if src.shape[0] != real * q or src.shape[1:] != dst.shape[1:]:
                 raise ValueError(f"{name} must be [{real * q}, {', '.join(map(str, dst.shape[1:]))}], "
                                  f"got {tuple(src.shape)}")
-            plain = plain and self._stageable(name, src) and src.is_contiguous()
+            at = self._source(name, src) if plain else None
+            plain = at is not None and src.is_contiguous()
             if plain:
                 nbytes = self._nbytes[name]
-                staged += (self._address[name], src.data_ptr(), 1, 1, nbytes, nbytes // self.batch_size * real, 0, 0)
+                staged += (self._address[name], at, 1, 1, nbytes, nbytes // self.batch_size * real, 0, 0)
         if plain:
             _op_impl.stage_inputs(staged, self._block)
             increment_version(self._block)  # written, for autograd (its views, the inputs, share the counter)

@@ -73,28 +73,35 @@ def _weights_fp32(hidden_states, weights_proj_weight, score_scale: float) -> tor
     return weights.to(hidden_states.dtype)
 
 
+_TYPES, _STRIDED = frozenset((torch.Tensor, torch.nn.Parameter)), torch.strided
+
+
 def _plain_type(cls) -> bool:
     """Tensors, parameters, and parameter classes that leave torch's functions
     as they are."""
-    return cls is torch.Tensor or (cls.__torch_function__ is torch.nn.Parameter.__torch_function__
-                                   and cls.__torch_dispatch__ is torch.Tensor.__torch_dispatch__)
+    return cls in _TYPES or (cls.__torch_function__ is torch.nn.Parameter.__torch_function__
+                             and cls.__torch_dispatch__ is torch.Tensor.__torch_dispatch__)
 
 
 def _plain(t, shape, dtypes, device, align=16) -> bool:
     """A contiguous tensor of this shape whose memory holds its values as the
     HIP kernels read them (no subclass, lazy negation or sparse layout)."""
-    return (_plain_type(type(t)) and t.shape == shape and t.dtype in dtypes and t.device == device
-            and t.layout is torch.strided and not t.is_neg() and t.is_contiguous() and t.data_ptr() % align == 0)
+    return ((type(t) in _TYPES or _plain_type(type(t))) and t.layout is _STRIDED and t.shape == shape
+            and t.dtype in dtypes and t.device == device and not t.is_neg() and t.is_contiguous()
+            and t.data_ptr() % align == 0)
 
 
 def _derivatives_asked(*tensors) -> bool:
     """Whether autograd follows any of the tensors, in either mode: only the
     library path hands derivatives on."""
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-        return True
     # (The level is below 0 outside every forward_ad.dual_level().)
-    return (getattr(forward_ad, "_current_level", 0) >= 0
-            and any(forward_ad.unpack_dual(t).tangent is not None for t in tensors))
+    dual = getattr(forward_ad, "_current_level", 0) >= 0
+    grad = torch.is_grad_enabled()
+    if grad or dual:
+        for t in tensors:
+            if (grad and t.requires_grad) or (dual and forward_ad.unpack_dual(t).tangent is not None):
+                return True
+    return False
 
 
 def _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, n_head) -> bool:
@@ -184,13 +191,14 @@ def dsa_indexer_project(hidden_states, q_c, cos, sin, wq_b_weight, wk_weight, k_
     # has the plain form that the kernels read (weights_proj_weight in fp32,
     # or in 16 bits, which only the library path widens before the product).
     dtype, device = hidden_states.dtype, hidden_states.device
-    norm = [t for t in (k_norm_weight, k_norm_bias) if t is not None]
+    norm = (k_norm_weight,) if k_norm_bias is None else (k_norm_weight, k_norm_bias)
     # (A rope_dim that the key's RoPE operator refuses goes there too.)
     if (weights_proj_weight.dtype == torch.float32 and int(head_dim) == 128 and k_norm_weight is not None
             and int(rope_dim) % 16 == 0
             and _weights_kernel_takes(hidden_states, weights_proj_weight, index_weights_out, int(n_head))
             and _plain(wk_weight, (128, hidden_states.shape[1]), (dtype,), device)
-            and all(_plain(t, (128,), (dtype,), device, 4) for t in norm)
+            and _plain(k_norm_weight, (128,), (dtype,), device, 4)
+            and (k_norm_bias is None or _plain(k_norm_bias, (128,), (dtype,), device, 4))
             and (cos.numel() // tokens) % 2 == 0 and index_k_out.data_ptr() % 4 == 0
             and not _derivatives_asked(wk_weight, index_k_out, *norm)):
         ops.indexer_project_kw(hidden_states, cos, sin, wk_weight, k_norm_weight, k_norm_bias, weights_proj_weight,
