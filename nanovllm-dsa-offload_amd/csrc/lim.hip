@@ -2314,17 +2314,20 @@ struct LinearDigits {
 };
 
 // Range [lo, hi] of keys for the digits of a row of whole blocks whose key
-// ranges are rg, so that outlying keys of a few blocks do not stretch it.  The
-// blocks are dealt in turn to up to 16 pairs of groups; a pair reaches as far
-// as both of its groups do, and the range as far as one of the pairs, without
-// unmapped blocks (-FLT_MAX throughout).  The C-th largest key may lie outside,
-// if the selection ends among the outlying keys: that costs time only.
-// (Between the smallest and largest key of all, one outlying score or an
+// ranges are rg: from the smallest to the largest key, without unmapped blocks
+// (-FLT_MAX throughout), unless that is kWindowStretch times what the row has
+// without the outlying keys of a few blocks.  For that range the blocks are
+// dealt in turn to up to 16 pairs of groups; a pair reaches as far as both of
+// its groups do, and the range as far as one of the pairs.  The C-th largest
+// key may lie outside, if the selection ends among the outlying keys: that
+// costs time only, as a stretched range does.  (One outlying score or an
 // unmapped block put the other tokens into one bin: 118 us for the call at
-// 32768 tokens instead of 67.)
+// 32768 tokens instead of 67.  With the narrow range throughout, 16 blocks that
+// hold the whole selection took 81 us, and 2048-token stripes 89.)
 constexpr int kWindowPairs = kManageThreads / 32;
+constexpr float kWindowStretch = 6.f;  // (bins that much wider still hold a few dozen tokens)
 
-__device__ __forceinline__ void row_window(const uint2* rg, int nblocks, uint2* red, uint32_t& lo, uint32_t& hi) {
+__device__ __forceinline__ void row_window(const uint2* rg, int nblocks, uint4* red, uint32_t& lo, uint32_t& hi) {
   const int pairs = min(kWindowPairs, max(1, nblocks / 16));
   const int pair = threadIdx.x >> 5, row = (threadIdx.x >> 4) & 1, pos = threadIdx.x & 15;
   lo = 0xffffffffu;
@@ -2338,33 +2341,36 @@ __device__ __forceinline__ void row_window(const uint2* rg, int nblocks, uint2* 
       }
     }
   // Over the 16 lanes of a row, in every lane of it.
-  auto row_minmax = [&]() {
+  auto over_row = [&](uint32_t v, auto op) {
     auto step = [&](auto ctrl) {
-      auto dpp = [](uint32_t v) {
-        return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v),
-                                                                 decltype(ctrl)::value, 0xf, 0xf, false));
-      };
-      lo = min(lo, dpp(lo));
-      hi = max(hi, dpp(hi));
+      v = op(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v),
+                                                                  decltype(ctrl)::value, 0xf, 0xf, false)));
     };
     step(std::integral_constant<int, 0xb1>{});   // quad_perm [1,0,3,2]
     step(std::integral_constant<int, 0x4e>{});   // quad_perm [2,3,0,1]
     step(std::integral_constant<int, 0x141>{});  // row_half_mirror
     step(std::integral_constant<int, 0x140>{});  // row_mirror
+    return v;
   };
-  row_minmax();
+  lo = over_row(lo, MinU32Op{});
+  hi = over_row(hi, MaxU32Op{});
   const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);  // the values of the pair's two rows
   const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
   if ((threadIdx.x & 31) == 0)
-    red[pair] = pair < pairs ? make_uint2(max(l[0], l[1]), min(h[0], h[1])) : make_uint2(0xffffffffu, 0u);
+    red[pair] = pair < pairs ? make_uint4(max(l[0], l[1]), min(h[0], h[1]), min(l[0], l[1]), max(h[0], h[1]))
+                             : make_uint4(0xffffffffu, 0u, 0xffffffffu, 0u);
   lds_barrier();
-  const uint2 v = red[threadIdx.x & (kWindowPairs - 1)];
-  lo = v.x;
-  hi = v.y;
   static_assert(kWindowPairs == 16, "one row of lanes");
-  row_minmax();
-  lo = __builtin_amdgcn_readfirstlane(lo);
-  hi = __builtin_amdgcn_readfirstlane(hi);
+  const uint4 v = red[threadIdx.x & (kWindowPairs - 1)];
+  lo = __builtin_amdgcn_readfirstlane(over_row(v.x, MinU32Op{}));
+  hi = __builtin_amdgcn_readfirstlane(over_row(v.y, MaxU32Op{}));
+  const uint32_t all_lo = __builtin_amdgcn_readfirstlane(over_row(v.z, MinU32Op{}));
+  const uint32_t all_hi = __builtin_amdgcn_readfirstlane(over_row(v.w, MaxU32Op{}));
+  const float near = key_score(hi) - key_score(lo), all = key_score(all_hi) - key_score(all_lo);
+  if (!(near > 0.f) || all <= kWindowStretch * near) {
+    lo = all_lo;
+    hi = all_hi;
+  }
 }
 
 // Chunk p's keys above the bin and in-bin tokens: counts[2 p], counts[2 p + 1];
@@ -2372,7 +2378,7 @@ __device__ __forceinline__ void row_window(const uint2* rg, int nblocks, uint2* 
 // gather[p * kGatherPart].
 __global__ __launch_bounds__(kManageThreads) void lidu_hist_kernel(const float* s, int n, InitWs w) {
   __shared__ uint32_t hist[kHistBins];
-  __shared__ uint2 red[kWindowPairs];
+  __shared__ uint4 red[kWindowPairs];
   const int part = blockIdx.x, tid = threadIdx.x;
   uint32_t u[kItems];
   const bool in = load_keys8_whole(s, n, part * kChunk + tid * kItems, u);

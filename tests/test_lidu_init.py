@@ -296,6 +296,9 @@ def _spread(case, form):
         score([n - 1], -1e30)
     elif form == "infinite":  # 65 x 3e38 in fp32
         keys[rows[n // 2], :2] = O.f32_to_bits(np.full(2, 3e38, np.float32), case["dtype"])
+    elif form in ("cluster", "stripes"):  # 262144 more for 16 blocks in a row, or for every other 2048 tokens
+        hot = (np.arange(n) - 128) // 2048 == 0 if form == "cluster" else np.arange(n) // 2048 % 2 == 0
+        keys[rows[hot], 3] = O.f32_to_bits(np.ones(1, np.float32), case["dtype"])[0]
     if form in ("scales", "scales_ties"):
         score([7, n // 2, n // 3, n - 2], [1e30, 1e15, 1e8, -1e20])
     if form in ("ties", "scales_ties"):
@@ -310,7 +313,8 @@ def _spread(case, form):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("form", ["unmapped", "high", "low", "infinite", "scales", "ties", "scales_ties", "log", "equal", "two"])
+@pytest.mark.parametrize("form", ["unmapped", "high", "low", "infinite", "scales", "ties", "scales_ties", "log", "equal", "two",
+                                  "cluster", "stripes"])
 @pytest.mark.parametrize("n_blocks,c", [(24, 2048), (160, 3000), (265, 8192)])
 def test_gpu_initialize_lidu_row_stretched_ranges(n_blocks, c, form):
     """Outlying, infinite, unmapped, tied and widely spread scores, in one
