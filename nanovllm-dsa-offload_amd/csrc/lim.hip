@@ -1126,15 +1126,8 @@ __device__ inline void load_keys8(const float* s, int n, int t0, uint32_t* u, bo
   }
 }
 
-// Adds a chunk's first digits, digit(key) of its keys u (those in(e)), to the
-// row's histogram `gh`: counted in LDS (`hist`, cleared; the caller's barriers
-// order the clearing before this), then added.
-template <typename In, typename Digit>
-__device__ __forceinline__ void add_first_digits(const uint32_t (&u)[kItems], const In& in, const Digit& digit,
-                                                 uint32_t* gh, uint32_t* hist) {
-#pragma unroll
-  for (int e = 0; e < kItems; ++e)
-    if (in(e)) atomicAdd(&hist[digit(u[e])], 1u);
+// Adds a chunk's first digits, counted in LDS, to the row's histogram.
+__device__ __forceinline__ void add_digit_counts(const uint32_t* hist, uint32_t* gh) {
   __syncthreads();
   for (int i = threadIdx.x; i < kHistBins; i += kManageThreads) {
     const uint32_t v = hist[i];
@@ -1177,8 +1170,10 @@ __global__ __launch_bounds__(kManageThreads) void lim_hist_kernel(LimArgs a, Lim
     w.rowsel[4 * b] = lo;
     w.rowsel[4 * b + 1] = static_cast<uint32_t>(shift);
   }
-  add_first_digits(u, [&](int e) { return in[e]; }, [=](uint32_t key) { return (key - lo) >> shift; },
-                   w.hist + static_cast<int64_t>(b) * kHistBins, hist);
+#pragma unroll
+  for (int e = 0; e < kItems; ++e)
+    if (in[e]) atomicAdd(&hist[(u[e] - lo) >> shift], 1u);
+  add_digit_counts(hist, w.hist + static_cast<int64_t>(b) * kHistBins);
 }
 
 // The hit half of an MTP0 output row: positions m, m+1, ... get the hits by
@@ -1741,11 +1736,12 @@ __device__ __forceinline__ void mtp0_resolve(const LimArgs& a, const LimWs& w, i
 }
 
 // The first-digit bin holding the k-th largest key of a row, the count of keys
-// above it and the count in it: thread tid owns bins [P tb, P tb + P), P = kHistPerThread, tb
-// = 511 - tid, so ascending threads scan descending bins.  (Barriers order LDS
-// only: the caller's loads stay in flight.)
+// above it and, if asked for, the count in it: thread tid owns bins
+// [P tb, P tb + P), P = kHistPerThread, tb = 511 - tid, so ascending threads
+// scan descending bins.  (Barriers order LDS only: the caller's loads stay in
+// flight.)
 __device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int* scratch, int* bcast, int& bin,
-                                                int& above, int& count) {
+                                                int& above, int* count = nullptr) {
   const int tid = threadIdx.x;
   constexpr int P = kHistPerThread;
   const int tb = kManageThreads - 1 - tid;
@@ -1768,7 +1764,7 @@ __device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int
   int sum = 0;
 #pragma unroll
   for (int j = 0; j < P; ++j) sum += cnt[j];
-  if (tid == 0) bcast[0] = bcast[1] = bcast[2] = 0;  // ordered before the writes below by the scan's barriers
+  if (tid == 0) bcast[0] = bcast[1] = 0;  // ordered before the writes below by the scan's barriers
   int total;
   int acc = block_exclusive_scan<true>(sum, scratch, &total);  // the token loads stay in flight
   if (acc < k && k <= acc + sum) {
@@ -1777,7 +1773,7 @@ __device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int
       if (acc < k && k <= acc + cnt[j]) {
         bcast[0] = P * tb + j;
         bcast[1] = acc;
-        bcast[2] = cnt[j];
+        if (count != nullptr) bcast[2] = cnt[j];
       }
       acc += cnt[j];
     }
@@ -1785,7 +1781,7 @@ __device__ __forceinline__ void first_digit_bin(const uint32_t* hist, int k, int
   lds_barrier();
   bin = __builtin_amdgcn_readfirstlane(bcast[0]);
   above = __builtin_amdgcn_readfirstlane(bcast[1]);
-  count = __builtin_amdgcn_readfirstlane(bcast[2]);
+  if (count != nullptr) *count = __builtin_amdgcn_readfirstlane(bcast[2]);
 }
 
 // One 4096-token chunk of an MTP0 request (every launch shape): the row's
@@ -1809,8 +1805,8 @@ __device__ __forceinline__ ChunkSel classify_chunk(const LimArgs& a, const LimWs
   int32_t slot[kItems];
   bool in[kItems];
   load_tokens8(w.scores + static_cast<int64_t>(b) * cap, a.pool + static_cast<int64_t>(r) * cap, n, t0, u, slot, in);
-  int bin, above, count;
-  first_digit_bin(w.hist + static_cast<int64_t>(b) * kHistBins, kTopK, scratch, bcast, bin, above, count);
+  int bin, above;
+  first_digit_bin(w.hist + static_cast<int64_t>(b) * kHistBins, kTopK, scratch, bcast, bin, above);
   uint32_t* stab = w.slot_table + static_cast<int64_t>(b) * kTableStride;
   uint32_t* skey = w.slot_key + static_cast<int64_t>(b) * kTableStride;
   unsigned missm = 0u, inbin = 0u;
@@ -2394,7 +2390,11 @@ __global__ __launch_bounds__(kManageThreads) void lidu_hist_kernel(const float* 
     if (tid == 0) atomicAdd(&w.hist[0], static_cast<uint32_t>(min(kChunk, n - part * kChunk)));
     return;
   }
-  add_first_digits(u, [=](int) { return in; }, digit, w.hist, hist);
+  if (in) {
+#pragma unroll
+    for (int e = 0; e < kItems; ++e) atomicAdd(&hist[digit(u[e])], 1u);
+  }
+  add_digit_counts(hist, w.hist);
 }
 
 __global__ __launch_bounds__(kManageThreads) void lidu_chunks_kernel(const float* s, int n, int c, InitWs w) {
@@ -2408,7 +2408,7 @@ __global__ __launch_bounds__(kManageThreads) void lidu_chunks_kernel(const float
   const bool in = load_keys8_whole(s, n, t0, u);
   const LinearDigits digit(w.rowsel[0], w.rowsel[1]);
   int bin, above, count;
-  first_digit_bin(w.hist, c, scratch, bcast, bin, above, count);
+  first_digit_bin(w.hist, c, scratch, bcast, bin, above, &count);
   unsigned inbin = 0u;
   int over = 0;
   if (in) {
